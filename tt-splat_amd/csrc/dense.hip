@@ -1,4 +1,4 @@
-// Dense (unbinned) poly-splat + WSR: every gaussian against every pixel, O(P*G).
+// Dense (unbinned) poly-splat + WSR: every gaussian against every pixel it may weigh on.
 //
 // Two forms of the reference's dense entry points:
 //   quad  : spike/render.py:14-49 arm "A" -- Q = a dx^2 + 2b dx dy + c dy^2 with dx = px - mu_x
@@ -10,8 +10,9 @@
 //           basis Phi[P,6], w = o*keep*max(u,0)^2; backward gives g_theta[G,6], g_o[G],
 //           g_color[G,3], g_w_b.
 //
-// Forward: one thread per pixel, gaussians staged through LDS 256 at a time.
-// Backward: one thread per gaussian; the pixels are cut into bands, each (gaussian chunk, band)
+// Quad forward: a block per tile of pixels, the gaussians whose support reaches it listed in LDS
+// (DenseWalk below).  theta forward: one thread per pixel, gaussians staged through LDS 256 at a
+// time.  Backward: one thread per gaussian; the pixels are cut into bands, each (gaussian chunk, band)
 // block stages its band's per-pixel WSR gradients (gnum = gC/den, gden = -(gC.C)/den) in LDS and
 // accumulates the gaussian's sums over the band.  Band partials go to a workspace and are summed
 // in band order by a second kernel, so the result is deterministic and there are no atomics.
@@ -59,81 +60,258 @@ inline size_t dense_ws_bytes(int G, int P, int ncomp) {
          nb * (size_t)G * ncomp * 4;
 }
 
+// ---------------------------------------------------------------- support culling
+//
+// A gaussian weighs nothing where Q >= k, so a tile of pixels only needs the gaussians whose
+// support may reach it.  support_half returns half-extents of a box around the mean that holds
+// every point where the *computed* u = 1 - Q/k can be positive, or infinity when it cannot say.
+// The computed Q is off by at most 12 eps (a dx^2 + c dy^2) (three rounded products and sums;
+// |2b dx dy| <= a dx^2 + c dy^2), so the points lie in the ellipse of the form with a and c
+// reduced by 1e-6; 3e-5 is taken from a*c below, which also covers the rounding of a*c - b^2, and
+// 0.1 % is added to k.  No bound is given, and the gaussian is taken everywhere, when the form is
+// not positive definite by that margin, or when a value is so large (or not a number) that its
+// product with a zero weight would not be zero.
+__device__ __forceinline__ float2 support_half(float4 r0, float4 r1, float4 r2, float kk) {
+  const float a = r0.z, b = r0.w, c = r1.x;
+  const float det = a * c * (1.0f - 3e-5f) - b * b;
+  const bool ok = fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && a > 0.0f && a < 1e9f &&
+                  c > 0.0f && c < 1e9f && det > 1e-30f &&
+                  fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e18f;
+  const float s = kk / det;
+  return ok ? make_float2(sqrtf(s * c), sqrtf(s * a)) : make_float2(INFINITY, INFINITY);
+}
+// u = 1 - Q/k with its roundings spelled out: the same value wherever it is inlined.
+__device__ __forceinline__ float quad_u(float dx, float dy, float a, float b2, float c,
+                                        float inv_k) {
+  const float Q = __builtin_fmaf(__builtin_fmaf(a, dx, b2 * dy), dx, (c * dy) * dy);
+  return __builtin_fmaf(-Q, inv_k, 1.0f);
+}
+// k with the margin above
+__device__ __forceinline__ float support_k(float inv_k) { return 1.001f / inv_k; }
+
+// Largest magnitude that still gives zero when a zero weight multiplies it and its products.
+__device__ __forceinline__ bool tame(float v) { return fabsf(v) < 1e18f; }
+
+// Does the box reach the pixel centres within `half` of `centre`?  (false only when it cannot:
+// an infinite extent gives true, a NaN difference too; 0.01 covers the rounding of both sides)
+__device__ __forceinline__ bool reaches(float centre, float half, float mu, float ext) {
+  return !(fabsf(centre - mu) > ext + half + 0.01f);
+}
+
+// A block's walk over the gaussians that reach its TS x TS pixels.  All threads test NT
+// gaussians at a time against the tile and append the hits, in order, to a list in LDS (one
+// barrier a round: the waves' hit counts are exchanged through a double buffer); when the list
+// could overflow in the next round, and at the end, it is evaluated.  For that the tile is cut
+// into 8 x 8 patches, one pixel per lane, and each patch's gaussians are dealt to SPL waves:
+// a wave tests 64 list entries at once against its patch and visits every SPL-th hit, two at a
+// time.  The order of a pixel's additions depends on nothing but the inputs.
+template <int TS, int NT>
+struct DenseWalk {
+  static constexpr int NW = NT / 64;
+  static constexpr int PATCH = (TS / 8) * (TS / 8);
+  static constexpr int SPL = NW / PATCH;
+  static constexpr int CAP = NT + NT / 4;
+  static_assert(SPL * PATCH == NW, "whole waves per patch");
+  float4 a[CAP];  // mu_x, mu_y, a, 2b
+  float4 b[CAP];  // c, col_o r, g, b
+  float2 o[CAP];  // o_col, depth
+  float2 h[TS > 8 ? CAP : 1];  // half-extents
+  int cnt[2][NW];
+
+  // pixel of this lane: its tile starts at (X0, Y0)
+  __device__ __forceinline__ static int lane_x() {
+    return ((threadIdx.x >> 6) / SPL) % (TS / 8) * 8 + (threadIdx.x & 7);
+  }
+  __device__ __forceinline__ static int lane_y() {
+    return ((threadIdx.x >> 6) / SPL) / (TS / 8) * 8 + ((threadIdx.x & 63) >> 3);
+  }
+  __device__ __forceinline__ static int split() { return (threadIdx.x >> 6) % SPL; }
+
+  template <class F>
+  __device__ __forceinline__ void evaluate(int n, int X0, int Y0, const F& f) {
+    const int lane = threadIdx.x & 63, sp = split();
+    if (TS == 8) {
+      for (int j = sp; j < n; j += 2 * SPL) {
+        const bool two = j + SPL < n;
+        const int j1 = two ? j + SPL : j;
+        const float4 A0 = a[j], B0 = b[j], A1 = a[j1], B1 = b[j1];
+        const float2 O0 = o[j], O1 = o[j1];
+        f(A0, B0, O0);
+        if (two) f(A1, B1, O1);
+      }
+      return;
+    }
+    const float cx = (float)(X0 + (lane_x() & ~7)) + 4.0f, cy = (float)(Y0 + (lane_y() & ~7)) + 4.0f;
+    int seen = 0;
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int j = min(j0 + lane, n - 1);
+      const float4 A = a[j];
+      const float2 e = h[j];
+      const bool hit = j0 + lane < n && reaches(cx, 3.5f, A.x, e.x) && reaches(cy, 3.5f, A.y, e.y);
+      uint64_t m = __ballot(hit);
+      if (SPL > 1) {
+        const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        const int hits = __popcll(m);
+        m = __ballot(hit && (seen + rank) % SPL == sp);
+        seen += hits;
+      }
+      while (m) {
+        const int i0 = j0 + __builtin_ctzll(m);
+        m &= m - 1;
+        const bool two = m != 0;
+        const int i1 = two ? j0 + __builtin_ctzll(m) : i0;
+        m &= m - 1;
+        const float4 A0 = a[i0], B0 = b[i0], A1 = a[i1], B1 = b[i1];
+        const float2 O0 = o[i0], O1 = o[i1];
+        f(A0, B0, O0);
+        if (two) f(A1, B1, O1);
+      }
+    }
+  }
+
+  // f(A, B, O) for every gaussian that may weigh on this lane's pixel (and some that do not).
+  // cull = 0 takes every gaussian.  Ends with a barrier.
+  template <class F>
+  __device__ __forceinline__ void walk(const float* __restrict__ proj, int G, float inv_k, int cull,
+                                       int X0, int Y0, const F& f) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float kk = support_k(inv_k);
+    const float half = 0.5f * (TS - 1);
+    const float cx = (float)X0 + 0.5f * TS, cy = (float)Y0 + 0.5f * TS;
+    const float4* rec = reinterpret_cast<const float4*>(proj);
+    int n = 0, buf = 0;
+    float4 n0, n1, n2;
+    if (G > 0) {
+      const int64_t g = min((int)threadIdx.x, G - 1);
+      n0 = rec[g * 3]; n1 = rec[g * 3 + 1]; n2 = rec[g * 3 + 2];
+    }
+    for (int g0 = 0; g0 < G; g0 += NT) {
+      const float4 r0 = n0, r1 = n1, r2 = n2;
+      if (G - g0 > NT) {   // the next round's records, in flight during this one
+        const int64_t g = min(g0 + NT + (int)threadIdx.x, G - 1);
+        n0 = rec[g * 3]; n1 = rec[g * 3 + 1]; n2 = rec[g * 3 + 2];
+      }
+      const float2 e = cull ? support_half(r0, r1, r2, kk) : make_float2(INFINITY, INFINITY);
+      const bool hit = (int)threadIdx.x < G - g0 && reaches(cx, half, r0.x, e.x) &&
+                       reaches(cy, half, r0.y, e.y);
+      const uint64_t m = __ballot(hit);
+      if (lane == 0) cnt[buf][wave] = __popcll(m);
+      __syncthreads();
+      const int v = lane < NW ? cnt[buf][lane] : 0;
+      const int incl = wave_incl_scan(v);
+      const int base = __builtin_amdgcn_readlane(incl, wave) - __builtin_amdgcn_readlane(v, wave);
+      const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+      if (hit) {
+        const int at = n + base + rank;
+        a[at] = make_float4(r0.x, r0.y, r0.z, 2.0f * r0.w);
+        b[at] = make_float4(r1.x, r1.z, r1.w, r2.x);
+        o[at] = make_float2(r2.y, r1.y);
+        if (TS > 8) h[at] = e;
+      }
+      n += __builtin_amdgcn_readlane(incl, 63);
+      buf ^= 1;
+      if (n > CAP - NT || G - g0 <= NT) {
+        __syncthreads();
+        evaluate(n, X0, Y0, f);
+        n = 0;
+        __syncthreads();
+      }
+    }
+  }
+
+  // Sums v over the SPL waves of each patch, in wave order, through the list's storage; call it
+  // after walk().  Ends with a barrier.
+  template <int N>
+  __device__ __forceinline__ void join(float (&v)[N]) {
+    if (SPL == 1) return;
+    static_assert(SPL == 1 || N * NT <= 8 * CAP, "fits the list");
+    float* s = reinterpret_cast<float*>(this);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < N; ++i) s[(i * NW + wave) * 64 + lane] = v[i];
+    __syncthreads();
+    const int w0 = wave / SPL * SPL;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float t = 0.0f;
+#pragma unroll
+      for (int j = 0; j < SPL; ++j) t += s[(i * NW + w0 + j) * 64 + lane];
+      v[i] = t;
+    }
+    __syncthreads();
+  }
+};
+
 // ---------------------------------------------------------------- forward
 
-template <int ARM>
-__global__ __launch_bounds__(256) void k_render_dense(const float* __restrict__ proj, int G,
-                                                      int W, int P, float inv_k,
-                                                      const float* __restrict__ bg,
-                                                      const float* __restrict__ szb,
-                                                      float* __restrict__ image,
-                                                      float* __restrict__ den_out,
-                                                      float4* __restrict__ aux) {
-  __shared__ float4 s_a[kDenseChunk];  // mu_x, mu_y, a, 2b
-  __shared__ float4 s_b[kDenseChunk];  // c, col_o r, g, b
-  __shared__ float2 s_o[kDenseChunk];  // o_col, depth
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  const float px = (float)(p % W) + 0.5f, py = (float)(p / W) + 0.5f;
+// Bound by the tile tests (48 bytes of L2 per gaussian and tile) and by the pairs inside the
+// support.  Visiting every pair instead, one thread per pixel, took 91 us at G 2000, 128x128 (64
+// blocks, a serial chain of 2000), 1840-2040 us at G 10000, 800x800, and 441 us for SZ at G 3001,
+// 173x131; this walk takes under 13, 41 and 20 us.
+template <int ARM, int TS, int NT>
+__global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ proj, int G, int W,
+                                                     int H, float inv_k, int cull,
+                                                     const float* __restrict__ bg,
+                                                     const float* __restrict__ szb,
+                                                     float* __restrict__ image,
+                                                     float* __restrict__ den_out,
+                                                     float4* __restrict__ aux) {
+  using Walk = DenseWalk<TS, NT>;
+  __shared__ Walk s;
+  const int tx = (W + TS - 1) / TS;
+  const int X0 = (int)(blockIdx.x % tx) * TS, Y0 = (int)(blockIdx.x / tx) * TS;
+  const int x = X0 + Walk::lane_x(), y = Y0 + Walk::lane_y();
+  const float px = (float)x + 0.5f, py = (float)y + 0.5f;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
   float zstar = 0.0f, den0 = 0.0f;
-  // SZ runs the gaussian loop twice: pass 0 finds z*, pass 1 blends
-  for (int pass = (ARM == kArmSZ ? 0 : 1); pass < 2; ++pass) {
-    float nr = 0.f, ng = 0.f, nb = 0.f, nd = 0.f, lr = 0.f;
-    for (int g0 = 0; g0 < G; g0 += kDenseChunk) {
-      const int n = min(kDenseChunk, G - g0);
-      __syncthreads();
-      if ((int)threadIdx.x < n) {
-        const float4* r = reinterpret_cast<const float4*>(proj + (int64_t)(g0 + threadIdx.x) * 12);
-        const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-        s_a[threadIdx.x] = make_float4(r0.x, r0.y, r0.z, 2.0f * r0.w);
-        s_b[threadIdx.x] = make_float4(r1.x, r1.z, r1.w, r2.x);
-        s_o[threadIdx.x] = make_float2(r2.y, r1.y);
-      }
-      __syncthreads();
-      for (int j = 0; j < n; ++j) {
-        const float4 A = s_a[j], B = s_b[j];
-        const float2 O = s_o[j];
-        const float dx = px - A.x, dy = py - A.y;
-        const float Q = (A.z * dx + A.w * dy) * dx + (B.x * dy) * dy;
-        const float r = relu_nan(1.0f - Q * inv_k);
-        float w = r * r;
-        if (ARM == kArmSZ && pass == 0) {
-          nd += w * O.x;
-          nr += w * O.x * O.y;
-          continue;
-        }
-        if (ARM == kArmSZ) w *= sigmoidf_(-beta * (O.y - zstar));
-        if (ARM == kArmRV) lr += log1pf(-fminf(w * O.x, 1.0f - 1e-4f));
-        nr += w * B.y;
-        ng += w * B.z;
-        nb += w * B.w;
-        nd += w * O.x;
-      }
-    }
-    if (ARM == kArmSZ && pass == 0) {
-      den0 = nd + 1e-6f;
-      zstar = nr / den0;
-      continue;
-    }
-    if (p < P) {
-      if (ARM == kArmRV) {
-        const float d = nd + 1e-6f, R = expf(lr);
-        const float a0 = nr / d, a1 = ng / d, a2 = nb / d;
-        image[(int64_t)p * 3 + 0] = a0 * (1.0f - R) + bg[1] * R;
-        image[(int64_t)p * 3 + 1] = a1 * (1.0f - R) + bg[2] * R;
-        image[(int64_t)p * 3 + 2] = a2 * (1.0f - R) + bg[3] * R;
-        if (den_out) den_out[p] = d;
-        aux[p] = make_float4(R, a0, a1, a2);
-      } else {
-        const float wb = bg[0];
-        const float d = nd + wb;
-        image[(int64_t)p * 3 + 0] = (nr + wb * bg[1]) / d;
-        image[(int64_t)p * 3 + 1] = (ng + wb * bg[2]) / d;
-        image[(int64_t)p * 3 + 2] = (nb + wb * bg[3]) / d;
-        if (den_out) den_out[p] = d;
-        if (ARM == kArmSZ) aux[p] = make_float4(zstar, den0, 0.0f, 0.0f);
-      }
-    }
+  auto weight = [&](const float4& A, const float4& B) {
+    const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
+    return r * r;
+  };
+  if (ARM == kArmSZ) {   // z* first
+    if (!tame(beta)) cull = 0;
+    float v[2] = {0.f, 0.f};
+    s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
+      const float w = weight(A, B);
+      v[0] += w * O.x;
+      v[1] += w * O.x * O.y;
+    });
+    s.join(v);
+    den0 = v[0] + 1e-6f;
+    zstar = v[1] / den0;
+    if (__syncthreads_or(!tame(zstar))) cull = 0;
+  }
+  float v[ARM == kArmRV ? 5 : 4] = {};
+  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
+    float w = weight(A, B);
+    if (ARM == kArmSZ) w *= sigmoidf_(-beta * (O.y - zstar));
+    if (ARM == kArmRV) v[4] += log1pf(-fminf(w * O.x, 1.0f - 1e-4f));
+    v[0] += w * B.y;
+    v[1] += w * B.z;
+    v[2] += w * B.w;
+    v[3] += w * O.x;
+  });
+  s.join(v);
+  if (Walk::split() != 0 || x >= W || y >= H) return;
+  const int64_t p = (int64_t)y * W + x;
+  if (ARM == kArmRV) {
+    const float d = v[3] + 1e-6f, R = expf(v[ARM == kArmRV ? 4 : 0]);
+    const float a0 = v[0] / d, a1 = v[1] / d, a2 = v[2] / d;
+    image[p * 3 + 0] = a0 * (1.0f - R) + bg[1] * R;
+    image[p * 3 + 1] = a1 * (1.0f - R) + bg[2] * R;
+    image[p * 3 + 2] = a2 * (1.0f - R) + bg[3] * R;
+    if (den_out) den_out[p] = d;
+    aux[p] = make_float4(R, a0, a1, a2);
+  } else {
+    const float wb = bg[0];
+    const float d = v[3] + wb;
+    image[p * 3 + 0] = (v[0] + wb * bg[1]) / d;
+    image[p * 3 + 1] = (v[1] + wb * bg[2]) / d;
+    image[p * 3 + 2] = (v[2] + wb * bg[3]) / d;
+    if (den_out) den_out[p] = d;
+    if (ARM == kArmSZ) aux[p] = make_float4(zstar, den0, 0.0f, 0.0f);
   }
 }
 
@@ -500,6 +678,40 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
   }
 }
 
+inline int dense_tiles(int H, int W, int ts) { return ((H + ts - 1) / ts) * ((W + ts - 1) / ts); }
+
+// Pixel coordinates must be exact floats for the support boxes to hold.
+inline int dense_cull(int H, int W) { return H <= (1 << 22) && W <= (1 << 22); }
+
+// Tile side of the forward: every block tests all gaussians against its tile, so large tiles
+// test less, and small ones make more blocks.  Measured, arm A, sides 8 / 16 / 32 (us; SZ and RV
+// order the same way):
+//   G 10000, 800x800 (625 tiles of 32): 262 / 91 / 41;  G 500, 500x600 (304): 16 / 13 / 13
+//   G 2000, 400x400 (169 of 32, 625 of 16): 20 / 13 / 13 (RV 29 / 22 / 32)
+//   G 10000, 300x300 (361 of 16): 53 / 25 / 38;  100x60 (28 of 16): 28 / 43 / 113
+//   G 3001, 131x173 (99 of 16): 12 / 12 / 18 (SZ 20 / 22 / 47)
+inline int dense_tile_side(int H, int W) {
+  if (dense_tiles(H, W, 32) >= 300) return 32;
+  return dense_tiles(H, W, 16) >= 256 ? 16 : 8;
+}
+
+template <int ARM>
+void launch_render_dense(const float* proj, int G, int H, int W, float ik, const float* bg,
+                         const float* szb, float* image, float* den, float4* aux,
+                         hipStream_t stream) {
+  const int ts = dense_tile_side(H, W), cull = dense_cull(H, W);
+  const int nb = dense_tiles(H, W, ts);
+  if (ts == 32)
+    k_render_dense<ARM, 32, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
+                                                           den, aux);
+  else if (ts == 16)
+    k_render_dense<ARM, 16, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
+                                                           den, aux);
+  else
+    k_render_dense<ARM, 8, 512><<<nb, 512, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
+                                                        den, aux);
+}
+
 // Unpacks the workspace into (partials, gwb partials, per-pixel scratch); returns the band
 // count or an error.
 inline int dense_ws(void* ws, size_t ws_bytes, int G, int P, int ncomp, float** part,
@@ -534,9 +746,8 @@ int tts_render_dense(const float* proj, int G, int H, int W, float k, const floa
     return TTS_EINVAL;
   if (G > (1 << 30)) return TTS_EG;
   if ((int64_t)H * W > (int64_t(1) << 30)) return TTS_EINVAL;
-  const int P = H * W;
-  k_render_dense<kArmA><<<grid1d(P, 256), 256, 0, stream>>>(
-      proj, G, W, P, (float)(1.0 / (double)k), bg, nullptr, image, den, nullptr);
+  launch_render_dense<kArmA>(proj, G, H, W, (float)(1.0 / (double)k), bg, nullptr, image, den,
+                             nullptr, stream);
   return launch_status();
 }
 
@@ -550,19 +761,14 @@ int tts_render_dense_arm(const float* proj, int G, int H, int W, float k, const 
   if (arm == kArmSZ && !softz_beta) return TTS_EINVAL;
   if (G > (1 << 30)) return TTS_EG;
   if ((int64_t)H * W > (int64_t(1) << 30)) return TTS_EINVAL;
-  const int P = H * W;
   const float ik = (float)(1.0 / (double)k);
   float4* ax = reinterpret_cast<float4*>(aux);
-  const dim3 grid = grid1d(P, 256);
   if (arm == kArmSZ)
-    k_render_dense<kArmSZ><<<grid, 256, 0, stream>>>(proj, G, W, P, ik, bg, softz_beta, image,
-                                                     den, ax);
+    launch_render_dense<kArmSZ>(proj, G, H, W, ik, bg, softz_beta, image, den, ax, stream);
   else if (arm == kArmRV)
-    k_render_dense<kArmRV><<<grid, 256, 0, stream>>>(proj, G, W, P, ik, bg, nullptr, image, den,
-                                                     ax);
+    launch_render_dense<kArmRV>(proj, G, H, W, ik, bg, nullptr, image, den, ax, stream);
   else
-    k_render_dense<kArmA><<<grid, 256, 0, stream>>>(proj, G, W, P, ik, bg, nullptr, image, den,
-                                                    nullptr);
+    launch_render_dense<kArmA>(proj, G, H, W, ik, bg, nullptr, image, den, nullptr, stream);
   return launch_status();
 }
 
