@@ -494,7 +494,7 @@ int tts_relocate(float* params, float* m, float* v, float* sh_rest, float* sh_m,
 /* Fill n fp32 values with zero (a kernel, so graph captures hold no memset node). */
 int tts_zero(float* buf, int64_t n, hipStream_t stream);
 
-/* ---- dense (unbinned) forms, O(H*W*G): every gaussian against every pixel ---- */
+/* ---- dense (unbinned) forms: every gaussian against every pixel it may weigh on ---- */
 
 /* Dense blend arms of tts_render_dense_arm (spike/arms.py). */
 #define TTS_ARM_A 0   /* depth-free WSR (:22-31); arm B = A with the depth weight of tts_geom_fwd_ex */
@@ -512,8 +512,8 @@ int tts_render_dense(const float* proj, int G, int H, int W, float k, const floa
                      float* image, float* den, hipStream_t stream);
 
 /* Backward of tts_render_dense: grad9 [G,9] = dL/d(a, b, c, mu_x, mu_y, col_o rgb, o_col) (the
- * geometry backward's input), gwb[0] = dL/dw_b (gwb may be NULL).  Deterministic (band partials
- * summed in a fixed order).  Replaces autograd through spike/render.py:14-49. */
+ * geometry backward's input), gwb[0] = dL/dw_b (gwb may be NULL).  Deterministic (sums in
+ * a fixed order).  Replaces autograd through spike/render.py:14-49. */
 int tts_render_dense_bwd(const float* proj, int G, int H, int W, float k, const float* bg,
                          const float* image, const float* den, const float* gimage, float* grad9,
                          float* gwb, void* workspace, size_t workspace_bytes, hipStream_t stream);

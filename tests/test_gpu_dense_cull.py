@@ -109,3 +109,72 @@ def test_forward_non_finite_record_reaches_every_pixel(col, value):
     p[11, 0:2] = -500.0
     p[11, col] = value
     assert bool(torch.isnan(render(p.cuda(), H, W)).any(-1).all())
+
+
+def grads(proj, H, W, arm, gi):
+    """Backward of `render`: (grad [G,9 or 10], gwb)."""
+    bg = torch.tensor(BG, device="cuda")
+    if arm == "A":
+        img, den = kernels.render_dense(proj, H, W, 4.0, bg)
+        return kernels.render_dense_bwd(proj, H, W, 4.0, bg, img, den, gi)
+    sz = torch.tensor([3.0], device="cuda") if arm == "SZ" else None
+    img, den, aux = kernels.render_dense_arm(proj, H, W, 4.0, bg, arm, sz)
+    return kernels.render_dense_arm_bwd(proj, H, W, 4.0, bg, arm, img, den, aux, gi, sz)
+
+
+# row shares 16, 4 and 1; one wave per gaussian (G > 4096, small image) and four (large image);
+# a box of one pixel row, boxes larger than the image
+@pytest.mark.parametrize("G,H,W,size", [(1, 5, 70, 3.0), (63, 40, 23, 3.0), (65, 33, 31, 50.0),
+                                        (255, 1, 90, 3.0), (300, 64, 48, 6.0),
+                                        (4101, 41, 27, 2.0), (4097, 400, 340, 0.7)])
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+def test_backward_follows_autograd(G, H, W, size, arm):
+    print(f"[cull-bwd] {G} {H}x{W} {arm}", flush=True)
+    proj = records(G, H, W, seed=G, cond=10.0, size=size)
+    if H * W * G > 2e7:       # the 64-bit reference visits every pair: a corner of the image
+        proj[:, 0:2] = proj[:, 0:2] % 40
+    h, w = (H, W) if H * W * G <= 2e7 else (56, 56)
+    g = torch.Generator().manual_seed(3)
+    gi = torch.zeros(H, W, 3)
+    gi[:h, :w] = torch.randn(h, w, 3, generator=g)
+    got, gwb = grads(proj.cuda(), H, W, arm, gi.cuda())
+    P = proj.double().requires_grad_(True)
+    beta = torch.tensor(3.0, dtype=torch.float64, requires_grad=True)
+    img = oracle_detached_z(P, h, w, arm, beta)
+    (img * gi[:h, :w].double()).sum().backward()
+    ref = torch.cat([P.grad[:, 2:5], P.grad[:, 0:2], P.grad[:, 6:10]], 1)
+    # the contract of the dense gradients: 1e-3 relative L2 (u carries 12 eps cond, cond 10)
+    for sl in (slice(0, 3), slice(3, 5), slice(5, 8), slice(8, 9)):
+        e = float((got[:, sl].cpu().double() - ref[:, sl]).norm() / ref[:, sl].norm())
+        assert e <= 1e-3, (sl, e)
+    if arm == "SZ":
+        assert abs(float(got[:, 9].double().sum()) - float(beta.grad)) <= 1e-3 * abs(float(beta.grad)) + 1e-5
+
+
+def oracle_detached_z(P, H, W, arm, beta):
+    Pz = torch.cat([P[:, :5], P[:, 5:6].detach(), P[:, 6:]], 1)
+    return oracle(Pz, H, W, arm, beta)
+
+
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+def test_backward_non_finite_image_gradient_reaches_every_gaussian(arm):
+    H, W = 40, 40
+    proj = records(300, H, W, seed=5).cuda()
+    gi = torch.ones(H, W, 3, device="cuda")
+    gi[3, 4, 1] = float("nan")
+    got, _ = grads(proj, H, W, arm, gi)
+    assert bool(torch.isnan(got[:, 8]).all()) and bool(torch.isnan(got[:, 0:5]).all())
+
+
+@pytest.mark.parametrize("G,H,W,size", [(300, 50, 41, 4.0), (4200, 30, 50, 2.0)])
+def test_backward_matches_the_general_path(G, H, W, size):
+    """Boxes against the whole image (depth 1e19), thin gaussians included: the pairs outside the
+    box add exact zeros, so only the order of the sums differs."""
+    p = records(G, H, W, seed=9, cond=1e5, size=size).cuda()
+    gi = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+    bg = torch.tensor(BG, device="cuda")
+    img, den = kernels.render_dense(p, H, W, 4.0, bg)
+    a, _ = kernels.render_dense_bwd(p, H, W, 4.0, bg, img, den, gi)
+    b, _ = kernels.render_dense_bwd(everywhere(p), H, W, 4.0, bg, img, den, gi)
+    # H W terms in another order; they cancel in part, so against each column's largest gradient
+    assert float(((a - b).abs() / b.abs().amax(0)).max()) <= H * W * 2.0 ** -24

@@ -11,11 +11,13 @@
 //           g_color[G,3], g_w_b.
 //
 // Quad forward: a block per tile of pixels, the gaussians whose support reaches it listed in LDS
-// (DenseWalk below).  theta forward: one thread per pixel, gaussians staged through LDS 256 at a
-// time.  Backward: one thread per gaussian; the pixels are cut into bands, each (gaussian chunk, band)
-// block stages its band's per-pixel WSR gradients (gnum = gC/den, gden = -(gC.C)/den) in LDS and
-// accumulates the gaussian's sums over the band.  Band partials go to a workspace and are summed
-// in band order by a second kernel, so the result is deterministic and there are no atomics.
+// (DenseWalk below).  Quad backward: a pass over the pixels for their WSR gradients (gnum = gC/den,
+// gden = -(gC.C)/den), then waves per gaussian over the pixels of its support box.
+// theta forward: one thread per pixel, gaussians staged through LDS 256 at a time.
+// theta backward: one thread per gaussian; the pixels are cut into bands, each (gaussian chunk,
+// band) block stages its band's per-pixel WSR gradients in LDS and accumulates the gaussian's sums
+// over the band.  Band partials go to a workspace and are summed in band order by a second kernel.
+// All results are deterministic and there are no floating-point atomics.
 //
 // The quad form also renders the two per-pixel occlusion arms of spike/arms.py (ARM template):
 //   SZ (soft-Z, :50-68):  W0 = o w_geo, z* = sum W0 z / (sum W0 + 1e-6) per pixel (pass 1),
@@ -50,14 +52,31 @@ inline int dense_band_pixels(int G, int P) {
   return pb;
 }
 
-// Workspace layout: [align to 256][gwb partials, nb floats, padded to 256]
-// [per-pixel scratch, P floats, padded to 256][partials nb*G*ncomp].
-inline size_t dense_ws_bytes(int G, int P, int ncomp) {
+// Workspace of the theta form: [align to 256][gwb partials, nb floats, padded to 256]
+// [partials nb*G*kThetaComp].
+inline size_t pad256(size_t n) { return (n + 255) & ~size_t(255); }
+inline size_t theta_ws_bytes(int G, int P) {
   if (G <= 0 || P <= 0) return 0;
   const int pb = dense_band_pixels(G, P);
   const size_t nb = (size_t)((P + pb - 1) / pb);
-  return 256 + ((nb * 4 + 255) & ~size_t(255)) + (((size_t)P * 4 + 255) & ~size_t(255)) +
-         nb * (size_t)G * ncomp * 4;
+  return 256 + pad256(nb * 4) + nb * (size_t)G * kThetaComp * 4;
+}
+
+// Workspace of the quad form: [align to 256][gwb partials, kPreBlocks floats][wild flags,
+// kPreBlocks + 1 ints, padded to 256][per-pixel gradients, P float4][arm extras, P float2, padded]
+// [row-share partials, shares*G*(kQuadComp + 1), when there is more than one share].
+constexpr int kPreBlocks = 256;
+
+// Row shares of a gaussian's box in the backward: few gaussians over a large image would leave
+// most of the GPU idle (four waves per gaussian and share).  G 1, 20, 100 over 800x800, every pixel
+// in the box: 68, 71 and 217 us.
+inline int quad_shares(int G) { return G >= 256 ? 1 : (G >= 64 ? 4 : 16); }
+
+inline size_t quad_ws_bytes(int G, int P) {
+  if (G <= 0 || P <= 0) return 0;
+  const size_t sh = (size_t)quad_shares(G);
+  return 256 + kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4) + pad256((size_t)P * 16) +
+         pad256((size_t)P * 8) + (sh > 1 ? sh * (size_t)G * (kQuadComp + 1) * 4 : 0);
 }
 
 // ---------------------------------------------------------------- support culling
@@ -389,161 +408,198 @@ __device__ __forceinline__ float stage_pixel_grads(const float* __restrict__ ima
   return q.x * bg[1] + q.y * bg[2] + q.z * bg[3] + q.w;
 }
 
-// Per-pixel WSR gradients of the quad form, staged in LDS: (gnum r,g,b, gden) and the arm's
-// pair-independent extras (SZ: z*, Z/den0; RV: dL/dlogR).  Returns this thread's share of
-// dL/dw_b (zero for RV, which has no w_b).
+// Quad backward, pass 1: each pixel's WSR gradients q = (gnum r,g,b, gden) and RV's dL/dlogR
+// (ex.x), this block's share of dL/dw_b (RV has no w_b) and whether any of its values is wild:
+// such a value times a zero weight need not be zero, so pass 2 then visits every pair.  Block 0
+// clears the flag the soft-Z pass may raise.
 template <int ARM>
-__device__ __forceinline__ float stage_arm_grads(const float* __restrict__ image,
-                                                 const float* __restrict__ den,
-                                                 const float4* __restrict__ aux,
-                                                 const float* __restrict__ zk,
-                                                 const float* __restrict__ gimage, int p, bool in,
-                                                 const float* __restrict__ bg, float4* s_px,
-                                                 float2* s_ex) {
-  if (ARM != kArmRV) {
-    const float wpart = stage_pixel_grads(image, den, gimage, p, in, bg, s_px);
-    if (ARM == kArmSZ) s_ex[threadIdx.x] = in ? make_float2(aux[p].x, zk[p]) : make_float2(0.f, 0.f);
-    return wpart;
-  }
-  float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
-  float gs = 0.0f;
-  if (in) {
-    const float4 x = aux[p];  // R, C_avg
-    const float R = x.x, inv = 1.0f / den[p];
-    const float g0 = gimage[(int64_t)p * 3 + 0], g1 = gimage[(int64_t)p * 3 + 1],
-                g2 = gimage[(int64_t)p * 3 + 2];
-    const float k = (1.0f - R) * inv;  // dC/dC_avg / den
-    q = make_float4(g0 * k, g1 * k, g2 * k, -(g0 * x.y + g1 * x.z + g2 * x.w) * k);
-    // dL/dR * R = dL/dlogR
-    gs = (g0 * (bg[1] - x.y) + g1 * (bg[2] - x.z) + g2 * (bg[3] - x.w)) * R;
-  }
-  s_px[threadIdx.x] = q;
-  s_ex[threadIdx.x] = make_float2(gs, 0.0f);
-  return 0.0f;
-}
-
-// Soft-Z backward pre-pass, one thread per pixel: Z/den0 with Z = dL/dz* =
-// beta sum_g w_geo (gnum . col_o + gden o_col) h (1 - h).
-__global__ __launch_bounds__(256) void k_softz_pre(const float* __restrict__ proj, int G, int W,
-                                                   int P, float inv_k,
-                                                   const float* __restrict__ szb,
-                                                   const float* __restrict__ image,
+__global__ __launch_bounds__(256) void k_dense_pre(const float* __restrict__ image,
                                                    const float* __restrict__ den,
                                                    const float4* __restrict__ aux,
-                                                   const float* __restrict__ gimage,
-                                                   float* __restrict__ zk) {
-  __shared__ float4 s_a[kDenseChunk];
-  __shared__ float4 s_b[kDenseChunk];
-  __shared__ float2 s_o[kDenseChunk];
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  const bool in = p < P;
-  const float px = (float)(p % W) + 0.5f, py = (float)(p / W) + 0.5f;
-  const float beta = szb[0];
-  float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f, zs = 0.f, d0 = 1.f;
-  if (in) {
+                                                   const float* __restrict__ gimage, int P,
+                                                   const float* __restrict__ bg,
+                                                   float4* __restrict__ q_out,
+                                                   float2* __restrict__ ex,
+                                                   float* __restrict__ gwb_part,
+                                                   int* __restrict__ wild) {
+  __shared__ float s_ftmp[4];
+  float wpart = 0.0f;
+  bool bad = false;
+  for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < P; p += (int64_t)gridDim.x * 256) {
     const float inv = 1.0f / den[p];
-    const float g0 = gimage[(int64_t)p * 3 + 0], g1 = gimage[(int64_t)p * 3 + 1],
-                g2 = gimage[(int64_t)p * 3 + 2];
-    q0 = g0 * inv; q1 = g1 * inv; q2 = g2 * inv;
-    q3 = -(g0 * image[(int64_t)p * 3 + 0] + g1 * image[(int64_t)p * 3 + 1] +
-           g2 * image[(int64_t)p * 3 + 2]) * inv;
-    zs = aux[p].x;
-    d0 = aux[p].y;
-  }
-  float Z = 0.0f;
-  for (int g0 = 0; g0 < G; g0 += kDenseChunk) {
-    const int n = min(kDenseChunk, G - g0);
-    __syncthreads();
-    if ((int)threadIdx.x < n) {
-      const float4* r = reinterpret_cast<const float4*>(proj + (int64_t)(g0 + threadIdx.x) * 12);
-      const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-      s_a[threadIdx.x] = make_float4(r0.x, r0.y, r0.z, 2.0f * r0.w);
-      s_b[threadIdx.x] = make_float4(r1.x, r1.z, r1.w, r2.x);
-      s_o[threadIdx.x] = make_float2(r2.y, r1.y);
+    const float g0 = gimage[p * 3 + 0], g1 = gimage[p * 3 + 1], g2 = gimage[p * 3 + 2];
+    float4 q;
+    if (ARM == kArmRV) {
+      const float4 x = aux[p];  // R, C_avg
+      const float R = x.x, k = (1.0f - R) * inv;  // dC/dC_avg / den
+      q = make_float4(g0 * k, g1 * k, g2 * k, -(g0 * x.y + g1 * x.z + g2 * x.w) * k);
+      // dL/dR * R = dL/dlogR
+      const float gs = (g0 * (bg[1] - x.y) + g1 * (bg[2] - x.z) + g2 * (bg[3] - x.w)) * R;
+      ex[p] = make_float2(gs, 0.0f);
+      bad |= !tame(gs);
+    } else {
+      const float c0 = image[p * 3 + 0], c1 = image[p * 3 + 1], c2 = image[p * 3 + 2];
+      q = make_float4(g0 * inv, g1 * inv, g2 * inv, -(g0 * c0 + g1 * c1 + g2 * c2) * inv);
+      wpart += q.x * bg[1] + q.y * bg[2] + q.z * bg[3] + q.w;
     }
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-      const float4 A = s_a[j], B = s_b[j];
-      const float2 O = s_o[j];
-      const float dx = px - A.x, dy = py - A.y;
-      const float Q = (A.z * dx + A.w * dy) * dx + (B.x * dy) * dy;
-      const float r = relu_nan(1.0f - Q * inv_k);
-      const float h = sigmoidf_(-beta * (O.y - zs));
-      Z += r * r * (q0 * B.y + q1 * B.z + q2 * B.w + q3 * O.x) * h * (1.0f - h);
-    }
+    q_out[p] = q;
+    bad |= !tame(fabsf(q.x) + fabsf(q.y) + fabsf(q.z) + fabsf(q.w));
   }
-  if (in) zk[p] = beta * Z / d0;
+  const float tot = block_sum256(wpart, s_ftmp);
+  const int any = __syncthreads_or(bad);
+  if (threadIdx.x == 0) {
+    gwb_part[blockIdx.x] = tot;
+    wild[blockIdx.x] = any;
+    if (blockIdx.x == 0) wild[gridDim.x] = 0;
+  }
 }
 
-// ncomp = 9 (a, b, c, mu_x, mu_y, col_o rgb, o_col), 10 for SZ (+ this gaussian's dL/dbeta).
-template <int ARM>
-__global__ __launch_bounds__(256) void k_render_dense_bwd(
-    const float* __restrict__ proj, int G, int W, int P, int PB, float inv_k,
-    const float* __restrict__ bg, const float* __restrict__ szb, const float* __restrict__ image,
-    const float* __restrict__ den, const float4* __restrict__ aux, const float* __restrict__ zk,
-    const float* __restrict__ gimage, float* __restrict__ part, float* __restrict__ gwb_part) {
-  constexpr int NC = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
-  __shared__ float4 s_px[256];
-  __shared__ float2 s_xy[256];
-  __shared__ float2 s_ex[256];
-  __shared__ float s_ftmp[4];
-  const int band = blockIdx.y;
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  const bool act = g < G;
-  float mx = 0.f, my = 0.f, a = 0.f, b = 0.f, c = 0.f, cr = 0.f, cg = 0.f, cb = 0.f, oc = 0.f;
-  float zg = 0.f;
-  if (act) {
-    const float4* r = reinterpret_cast<const float4*>(proj + (int64_t)g * 12);
-    const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-    mx = r0.x; my = r0.y; a = r0.z; b = r0.w; c = r1.x;
-    cr = r1.z; cg = r1.w; cb = r2.x; oc = r2.y;
-    zg = r1.y;
+// Soft-Z backward, between the passes: Z/den0 of every pixel, Z = dL/dz* =
+// beta sum_g w_geo (gnum . col_o + gden o_col) h (1 - h); ex = (z*, Z/den0).  The forward's walk.
+template <int TS, int NT>
+__global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj, int G, int W,
+                                                  int H, float inv_k, int cull,
+                                                  const float* __restrict__ szb,
+                                                  const float4* __restrict__ aux,
+                                                  const float4* __restrict__ qbuf,
+                                                  float2* __restrict__ ex, int* __restrict__ wild) {
+  using Walk = DenseWalk<TS, NT>;
+  __shared__ Walk s;
+  const int tx = (W + TS - 1) / TS;
+  const int X0 = (int)(blockIdx.x % tx) * TS, Y0 = (int)(blockIdx.x / tx) * TS;
+  const int x = X0 + Walk::lane_x(), y = Y0 + Walk::lane_y();
+  const bool in = x < W && y < H;
+  const int64_t p = (int64_t)y * W + x;
+  const float px = (float)x + 0.5f, py = (float)y + 0.5f;
+  const float beta = szb[0];
+  float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+  float zs = 0.f, d0 = 1.f;
+  if (in) {
+    q = qbuf[p];
+    const float4 ax = aux[p];
+    zs = ax.x;
+    d0 = ax.y;
   }
+  const bool bad = !tame(fabsf(q.x) + fabsf(q.y) + fabsf(q.z) + fabsf(q.w)) || !tame(zs) ||
+                   !tame(beta);
+  if (__syncthreads_or(bad)) cull = 0;
+  float Z[1] = {0.0f};
+  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
+    const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
+    const float h = sigmoidf_(-beta * (O.y - zs));
+    Z[0] += r * r * (q.x * B.y + q.y * B.z + q.z * B.w + q.w * O.x) * h * (1.0f - h);
+  });
+  s.join(Z);
+  const float zk = beta * Z[0] / d0;
+  if (in && Walk::split() == 0) {
+    ex[p] = make_float2(zs, zk);
+    if (!tame(zs) || !tame(zk) || !tame(beta)) atomicOr(wild, 1);
+  }
+}
+
+// Quad backward, pass 2: WPG waves per gaussian (and row share) walk the pixels of its support
+// box, one pixel per lane, and sum its gradients over lanes and waves in a fixed order.
+// ncomp = 9 (a, b, c, mu_x, mu_y, col_o rgb, o_col), 10 for SZ (+ this gaussian's dL/dbeta).
+// Bound by the latency of a wave's few dependent steps (record, box, two to ten rounds of pixel
+// loads, lane sums); on large images by L2 reads of q (16 bytes a pair).  One thread per gaussian
+// over every pixel, bands of pixels staged in LDS, took 43 us at G 2000, 128x128, 472 at G 10000,
+// 300x300 and 3061 at 800x800 (soft-Z 296, 2994, 15818), its band sums included; this takes 19,
+// 25 and 85 (soft-Z 23, 63, 189).  That form is the faster one only where the support boxes fill
+// over half of the image on average (every box the whole image, G 2000, 400x400: 226 against 340).
+template <int ARM, int WPG>
+__global__ __launch_bounds__(256) void k_render_dense_bwd(
+    const float* __restrict__ proj, int G, int W, int H, float inv_k, int cull,
+    const float* __restrict__ szb, const float4* __restrict__ qbuf, const float2* __restrict__ ex,
+    const int* __restrict__ wild, int n_pre, int n_wild, const float* __restrict__ gwb_part,
+    float* __restrict__ out, float* __restrict__ gwb) {
+  constexpr int NC = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
+  __shared__ float s_sum[4][NC];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int sub = wave % WPG;
+  const int g = (int)blockIdx.x * (4 / WPG) + wave / WPG;
+  const bool act = g < G;
+  const float4* rec = reinterpret_cast<const float4*>(proj + (int64_t)min(g, G - 1) * 12);
+  const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+  int any = 0;
+  for (int i = lane; i < n_wild; i += 64) any |= wild[i];
+  if (__ballot(any != 0)) cull = 0;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && gwb) {
+    float t = 0.0f;
+    for (int i = lane; i < n_pre; i += 64) t += gwb_part[i];
+    t = wave_sum(t);
+    if (lane == 0) gwb[0] = t;
+  }
+  const float mx = r0.x, my = r0.y, a = r0.z, b = r0.w, c = r1.x, zg = r1.y;
+  const float cr = r1.z, cg = r1.w, cb = r2.x, oc = r2.y;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
   const float b2 = 2.0f * b;
+  // pixels [x0, x1) x [y0, y1): centres within the box; fminf / fmaxf turn an infinite box (and
+  // the NaN of an infinite mean less an infinite extent) into the whole image
+  int x0 = 0, x1 = W, y0 = 0, y1 = H;
+  if (cull) {
+    const float2 e = support_half(r0, r1, r2, support_k(inv_k));
+    x0 = (int)fminf(fmaxf(ceilf(mx - e.x - 0.51f), 0.0f), (float)W);
+    y0 = (int)fminf(fmaxf(ceilf(my - e.y - 0.51f), 0.0f), (float)H);
+    x1 = (int)fmaxf(fminf(floorf(mx + e.x - 0.49f) + 1.0f, (float)W), (float)x0);
+    y1 = (int)fmaxf(fminf(floorf(my + e.y - 0.49f) + 1.0f, (float)H), (float)y0);
+  }
+  const int rows = y1 - y0;
+  y1 = y0 + (int)((int64_t)rows * (blockIdx.y + 1) / gridDim.y);
+  y0 = y0 + (int)((int64_t)rows * blockIdx.y / gridDim.y);
+  const int bw = x1 - x0, n = act ? bw * (y1 - y0) : 0;
+  constexpr int S = 64 * WPG;
   float sxx = 0.f, sxy = 0.f, syy = 0.f, sx = 0.f, sy = 0.f;
   float gr = 0.f, gg = 0.f, gbl = 0.f, go = 0.f, gbeta = 0.f;
-  float wpart = 0.f;
-  const int pend = min(P, (band + 1) * PB);
-  for (int p0 = band * PB; p0 < pend; p0 += 256) {
-    __syncthreads();
-    const int pp = p0 + threadIdx.x;
-    wpart += stage_arm_grads<ARM>(image, den, aux, zk, gimage, pp, pp < pend, bg, s_px, s_ex);
-    s_xy[threadIdx.x] = make_float2((float)(pp % W) + 0.5f, (float)(pp / W) + 0.5f);
-    __syncthreads();
-    const int n = min(256, pend - p0);
-    for (int j = 0; j < n; ++j) {
-      const float4 q = s_px[j];
-      const float2 xy = s_xy[j];
-      const float dx = xy.x - mx, dy = xy.y - my;
-      const float Q = (a * dx + b2 * dy) * dx + (c * dy) * dy;
-      const float r = relu_nan(1.0f - Q * inv_k);
+  int i = sub * 64 + lane;
+  if (i < n) {
+    // this lane's pixel, stepped by S pixels in box order without dividing again
+    int x = i % bw, y = i / bw;
+    const int dxs = S % bw, dys = S / bw;
+    int64_t p = (int64_t)(y0 + y) * W + x0 + x;
+    float4 q = qbuf[p];
+    float2 e = ARM != kArmA ? ex[p] : make_float2(0.f, 0.f);
+    while (true) {
+      const float dx = (float)(x0 + x) + 0.5f - mx, dy = (float)(y0 + y) + 0.5f - my;
+      const float4 qc = q;
+      const float2 ec = e;
+      i += S;
+      if (i < n) {   // the next pixel's loads, in flight during this one
+        x += dxs;
+        y += dys;
+        if (x >= bw) {
+          x -= bw;
+          ++y;
+        }
+        p = (int64_t)(y0 + y) * W + x0 + x;
+        q = qbuf[p];
+        if (ARM != kArmA) e = ex[p];
+      }
+      const float r = relu_nan(quad_u(dx, dy, a, b2, c, inv_k));
       const float w = r * r;
-      const float gw = q.x * cr + q.y * cg + q.z * cb + q.w * oc;  // dL/dw_geo of arm A
-      float dw;                                                   // dL/dw_geo of this arm
-      if (ARM == kArmSZ) {
-        const float2 ex = s_ex[j];  // z*, Z/den0
-        const float h = sigmoidf_(-beta * (zg - ex.x));
-        const float e = ex.y * (zg - ex.x);  // dL/dW0 through z*
-        gr += w * h * q.x;
-        gg += w * h * q.y;
-        gbl += w * h * q.z;
-        go += w * (h * q.w + e);
-        gbeta -= w * gw * h * (1.0f - h) * (zg - ex.x);
-        dw = h * gw + oc * e;
-      } else if (ARM == kArmRV) {
+      const float gw = qc.x * cr + qc.y * cg + qc.z * cb + qc.w * oc;  // dL/dw_geo of arm A
+      float dw;                                                       // dL/dw_geo of this arm
+      if (ARM == kArmSZ) {   // ec: z*, Z/den0
+        const float h = sigmoidf_(-beta * (zg - ec.x));
+        const float t = ec.y * (zg - ec.x);  // dL/dW0 through z*
+        gr += w * h * qc.x;
+        gg += w * h * qc.y;
+        gbl += w * h * qc.z;
+        go += w * (h * qc.w + t);
+        gbeta -= w * gw * h * (1.0f - h) * (zg - ec.x);
+        dw = h * gw + oc * t;
+      } else if (ARM == kArmRV) {   // ec.x: dL/dlogR
         const float W0 = w * oc;
-        const float e = W0 <= 1.0f - 1e-4f ? -s_ex[j].x / (1.0f - W0) : 0.0f;  // clamp gate
-        gr += w * q.x;
-        gg += w * q.y;
-        gbl += w * q.z;
-        go += w * (q.w + e);
-        dw = gw + oc * e;
+        const float t = W0 <= 1.0f - 1e-4f ? -ec.x / (1.0f - W0) : 0.0f;  // clamp gate
+        gr += w * qc.x;
+        gg += w * qc.y;
+        gbl += w * qc.z;
+        go += w * (qc.w + t);
+        dw = gw + oc * t;
       } else {
-        gr += w * q.x;
-        gg += w * q.y;
-        gbl += w * q.z;
-        go += w * q.w;
+        gr += w * qc.x;
+        gg += w * qc.y;
+        gbl += w * qc.z;
+        go += w * qc.w;
         dw = gw;
       }
       const float gu = r * dw;  // half of dL/du
@@ -553,28 +609,44 @@ __global__ __launch_bounds__(256) void k_render_dense_bwd(
       syy += ty * dy;
       sx += tx;
       sy += ty;
+      if (i >= n) break;
     }
   }
-  if (blockIdx.x == 0) {
-    const float tot = block_sum256(wpart, s_ftmp);
-    if (threadIdx.x == 0) gwb_part[band] = tot;
+  float v[NC] = {sxx, sxy, syy, sx, sy, gr, gg, gbl, go};
+  if (ARM == kArmSZ) v[NC - 1] = gbeta;
+#pragma unroll
+  for (int k = 0; k < NC; ++k) v[k] = wave_sum(v[k]);
+  if (WPG > 1) {
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < NC; ++k) s_sum[wave][k] = v[k];
+    }
+    __syncthreads();
+    const int w0 = wave / WPG * WPG;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      float t = s_sum[w0][k];
+#pragma unroll
+      for (int j = 1; j < WPG; ++j) t += s_sum[w0 + j][k];
+      v[k] = t;
+    }
   }
-  if (act) {
-    // dL/dQ = dL/du * (-1/k) = -2 gu / k
-    const float s = -2.0f * inv_k;
-    const float mxx = s * sxx, mxy = s * sxy, myy = s * syy, m_x = s * sx, m_y = s * sy;
-    float* dst = part + ((int64_t)band * G + g) * NC;
-    dst[0] = mxx;                          // dQ/da = dx^2
-    dst[1] = 2.0f * mxy;                   // dQ/db = 2 dx dy
-    dst[2] = myy;                          // dQ/dc = dy^2
-    dst[3] = -2.0f * (a * m_x + b * m_y);  // dQ/dmu_x = -2 (a dx + b dy)
-    dst[4] = -2.0f * (b * m_x + c * m_y);  // dQ/dmu_y = -2 (b dx + c dy)
-    dst[5] = gr;
-    dst[6] = gg;
-    dst[7] = gbl;
-    dst[8] = go;
-    if (ARM == kArmSZ) dst[9] = gbeta;
-  }
+  if (!act || sub != 0 || lane >= NC) return;
+  // dL/dQ = dL/du * (-1/k) = -2 gu / k
+  const float s = -2.0f * inv_k;
+  const float mxx = s * v[0], mxy = s * v[1], myy = s * v[2], m_x = s * v[3], m_y = s * v[4];
+  float r[NC];
+  r[0] = mxx;                          // dQ/da = dx^2
+  r[1] = 2.0f * mxy;                   // dQ/db = 2 dx dy
+  r[2] = myy;                          // dQ/dc = dy^2
+  r[3] = -2.0f * (a * m_x + b * m_y);  // dQ/dmu_x = -2 (a dx + b dy)
+  r[4] = -2.0f * (b * m_x + c * m_y);  // dQ/dmu_y = -2 (b dx + c dy)
+#pragma unroll
+  for (int k = 5; k < NC; ++k) r[k] = v[k];
+  float o = r[0];
+#pragma unroll
+  for (int k = 1; k < NC; ++k) o = lane == k ? r[k] : o;
+  out[((int64_t)blockIdx.y * G + g) * NC + lane] = o;
 }
 
 __global__ __launch_bounds__(256) void k_wsr_dense_bwd(
@@ -678,10 +750,16 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
   }
 }
 
+// Does pass 2 of the backward take four waves per gaussian, or one?  A support box grows with the
+// image.  Measured, whole arm-A backward, four / one (us): G 10000, 800x800 85 / 151; G 4000,
+// 800x800 57 / 124; G 2000, 400x400 19 / 32; G 10000, 300x300 31 / 25; 100x60 21 / 17; below 4096
+// gaussians on small images the same within 5 %.
+inline bool dense_wide(int G, int P) { return G <= 4096 || P >= (1 << 17); }
+
 inline int dense_tiles(int H, int W, int ts) { return ((H + ts - 1) / ts) * ((W + ts - 1) / ts); }
 
-// Pixel coordinates must be exact floats for the support boxes to hold.
-inline int dense_cull(int H, int W) { return H <= (1 << 22) && W <= (1 << 22); }
+// The support boxes allow 0.01 for the rounding of pixel coordinates (2^-8 at 2^16).
+inline int dense_cull(int H, int W) { return H <= (1 << 16) && W <= (1 << 16); }
 
 // Tile side of the forward: every block tests all gaussians against its tile, so large tiles
 // test less, and small ones make more blocks.  Measured, arm A, sides 8 / 16 / 32 (us; SZ and RV
@@ -712,20 +790,61 @@ void launch_render_dense(const float* proj, int G, int H, int W, float ik, const
                                                         den, aux);
 }
 
-// Unpacks the workspace into (partials, gwb partials, per-pixel scratch); returns the band
-// count or an error.
-inline int dense_ws(void* ws, size_t ws_bytes, int G, int P, int ncomp, float** part,
-                    float** gwbp, int* PB, float** pix = nullptr) {
-  if (!ws) return TTS_EWORKSPACE;
-  if (ws_bytes < dense_ws_bytes(G, P, ncomp)) return TTS_EWORKSPACE;
+// The whole quad backward of an arm; grad has kQuadComp columns (SZ: one more).
+template <int ARM>
+int launch_dense_bwd(const float* proj, int G, int H, int W, float ik, const float* bg,
+                     const float* szb, const float* image, const float* den, const float4* aux,
+                     const float* gimage, float* grad, float* gwb, void* ws, size_t ws_bytes,
+                     hipStream_t stream) {
+  const int P = H * W;
+  if (!ws || ws_bytes < quad_ws_bytes(G, P)) return TTS_EWORKSPACE;
+  char* base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(ws) + 255) & ~uintptr_t(255));
+  float* gwbp = reinterpret_cast<float*>(base);
+  int* wild = reinterpret_cast<int*>(base + kPreBlocks * 4);
+  base += kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4);
+  float4* q = reinterpret_cast<float4*>(base);
+  base += pad256((size_t)P * 16);
+  float2* ex = reinterpret_cast<float2*>(base);
+  float* part = reinterpret_cast<float*>(base + pad256((size_t)P * 8));
+  const int cull = dense_cull(H, W);
+  const int npre = P / 256 + 1 < kPreBlocks ? P / 256 + 1 : kPreBlocks;
+  k_dense_pre<ARM><<<npre, 256, 0, stream>>>(image, den, aux, gimage, P, bg, q, ex, gwbp, wild);
+  if (ARM == kArmSZ) {
+    const int ts = dense_tile_side(H, W), nb = dense_tiles(H, W, ts);
+    if (ts == 32)
+      k_softz_pre<32, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                     wild + npre);
+    else if (ts == 16)
+      k_softz_pre<16, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                     wild + npre);
+    else
+      k_softz_pre<8, 512><<<nb, 512, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                  wild + npre);
+  }
+  const int sh = quad_shares(G), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
+  float* dst = sh > 1 ? part : grad;
+  const int nw = npre + (ARM == kArmSZ ? 1 : 0);
+  if (dense_wide(G, P))
+    k_render_dense_bwd<ARM, 4><<<dim3(G, sh), 256, 0, stream>>>(
+        proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
+  else
+    k_render_dense_bwd<ARM, 1><<<dim3((G + 3) / 4, sh), 256, 0, stream>>>(
+        proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
+  if (sh > 1)
+    k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, sh, G, nc, nullptr,
+                                                                    grad, nullptr);
+  return launch_status();
+}
+
+// Unpacks the theta form's workspace into (partials, gwb partials); returns the band count or an
+// error.
+inline int theta_ws(void* ws, size_t ws_bytes, int G, int P, float** part, float** gwbp, int* PB) {
+  if (!ws || ws_bytes < theta_ws_bytes(G, P)) return TTS_EWORKSPACE;
   *PB = dense_band_pixels(G, P);
   const int nb = (P + *PB - 1) / *PB;
   uintptr_t base = (reinterpret_cast<uintptr_t>(ws) + 255) & ~uintptr_t(255);
   *gwbp = reinterpret_cast<float*>(base);
-  base += ((size_t)nb * 4 + 255) & ~size_t(255);
-  if (pix) *pix = reinterpret_cast<float*>(base);
-  base += ((size_t)P * 4 + 255) & ~size_t(255);
-  *part = reinterpret_cast<float*>(base);
+  *part = reinterpret_cast<float*>(base + pad256((size_t)nb * 4));
   return nb;
 }
 
@@ -736,8 +855,9 @@ using namespace tts;
 extern "C" {
 
 size_t tts_dense_workspace_bytes(int G, int P) {
-  // sized for the larger (theta form) partial record; serves both forms
-  return dense_ws_bytes(G, P, kThetaComp);
+  // serves both forms
+  const size_t t = theta_ws_bytes(G, P), q = quad_ws_bytes(G, P);
+  return t > q ? t : q;
 }
 
 int tts_render_dense(const float* proj, int G, int H, int W, float k, const float* bg,
@@ -781,18 +901,8 @@ int tts_render_dense_bwd(const float* proj, int G, int H, int W, float k, const 
     return TTS_EINVAL;
   if (G > (1 << 30)) return TTS_EG;
   if ((int64_t)H * W > (int64_t(1) << 30)) return TTS_EINVAL;
-  const int P = H * W;
-  float *part, *gwbp;
-  int PB;
-  const int nb = dense_ws(workspace, workspace_bytes, G, P, kQuadComp, &part, &gwbp, &PB);
-  if (nb < 0) return nb;
-  dim3 grid(grid1d(G, 256), nb);
-  k_render_dense_bwd<kArmA><<<grid, 256, 0, stream>>>(proj, G, W, P, PB, (float)(1.0 / (double)k),
-                                                      bg, nullptr, image, den, nullptr, nullptr,
-                                                      gimage, part, gwbp);
-  k_dense_reduce<<<grid1d((int64_t)G * kQuadComp, 256), 256, 0, stream>>>(part, nb, G, kQuadComp,
-                                                                         gwbp, grad9, gwb);
-  return launch_status();
+  return launch_dense_bwd<kArmA>(proj, G, H, W, (float)(1.0 / (double)k), bg, nullptr, image, den,
+                                 nullptr, gimage, grad9, gwb, workspace, workspace_bytes, stream);
 }
 
 int tts_render_dense_arm_bwd(const float* proj, int G, int H, int W, float k, const float* bg,
@@ -808,30 +918,16 @@ int tts_render_dense_arm_bwd(const float* proj, int G, int H, int W, float k, co
   if (arm == kArmSZ && !softz_beta) return TTS_EINVAL;
   if (G > (1 << 30)) return TTS_EG;
   if ((int64_t)H * W > (int64_t(1) << 30)) return TTS_EINVAL;
-  const int P = H * W;
-  const int nc = arm == kArmSZ ? kQuadComp + 1 : kQuadComp;
-  float *part, *gwbp, *zk;
-  int PB;
-  const int nb = dense_ws(workspace, workspace_bytes, G, P, nc, &part, &gwbp, &PB, &zk);
-  if (nb < 0) return nb;
   const float ik = (float)(1.0 / (double)k);
   const float4* ax = reinterpret_cast<const float4*>(aux);
-  dim3 grid(grid1d(G, 256), nb);
-  if (arm == kArmSZ) {
-    k_softz_pre<<<grid1d(P, 256), 256, 0, stream>>>(proj, G, W, P, ik, softz_beta, image, den,
-                                                    ax, gimage, zk);
-    k_render_dense_bwd<kArmSZ><<<grid, 256, 0, stream>>>(proj, G, W, P, PB, ik, bg, softz_beta,
-                                                         image, den, ax, zk, gimage, part, gwbp);
-  } else if (arm == kArmRV) {
-    k_render_dense_bwd<kArmRV><<<grid, 256, 0, stream>>>(proj, G, W, P, PB, ik, bg, nullptr, image,
-                                                         den, ax, nullptr, gimage, part, gwbp);
-  } else {
-    k_render_dense_bwd<kArmA><<<grid, 256, 0, stream>>>(proj, G, W, P, PB, ik, bg, nullptr, image,
-                                                        den, nullptr, nullptr, gimage, part, gwbp);
-  }
-  k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, nb, G, nc, gwbp, grad10,
-                                                                  gwb);
-  return launch_status();
+  if (arm == kArmSZ)
+    return launch_dense_bwd<kArmSZ>(proj, G, H, W, ik, bg, softz_beta, image, den, ax, gimage,
+                                    grad10, gwb, workspace, workspace_bytes, stream);
+  if (arm == kArmRV)
+    return launch_dense_bwd<kArmRV>(proj, G, H, W, ik, bg, nullptr, image, den, ax, gimage, grad10,
+                                    gwb, workspace, workspace_bytes, stream);
+  return launch_dense_bwd<kArmA>(proj, G, H, W, ik, bg, nullptr, image, den, nullptr, gimage,
+                                 grad10, gwb, workspace, workspace_bytes, stream);
 }
 
 int tts_wsr_dense(const float* theta, const float* o, const float* color, const uint8_t* keep,
@@ -854,7 +950,7 @@ int tts_wsr_dense_bwd(const float* theta, const float* o, const float* color,
   if (G > (1 << 30) || P > (1 << 30)) return TTS_EINVAL;
   float *part, *gwbp;
   int PB;
-  const int nb = dense_ws(workspace, workspace_bytes, G, P, kThetaComp, &part, &gwbp, &PB);
+  const int nb = theta_ws(workspace, workspace_bytes, G, P, &part, &gwbp, &PB);
   if (nb < 0) return nb;
   dim3 grid(grid1d(G, 256), nb);
   k_wsr_dense_bwd<<<grid, 256, 0, stream>>>(theta, o, color, keep, phi, G, P, PB, bg, C, den, gC,
