@@ -100,6 +100,14 @@ int tts_assign_bins(const float* mu2d, int mu_stride, const uint8_t* keep, int k
                     int32_t* idx, uint8_t* valid, int32_t* count, int32_t* ncand, int32_t* inv,
                     int32_t* order, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* tts_assign_bins with the ids as int64 (the reference's index type):
+ * same arguments, checks and results otherwise. */
+int tts_assign_bins_i64(const float* mu2d, int mu_stride, const uint8_t* keep, int keep_stride,
+                        int G, int H, int W, int S, int R, int K, int span,
+                        int64_t* idx, uint8_t* valid, int32_t* count, int32_t* ncand,
+                        int32_t* inv, int32_t* order, void* workspace, size_t workspace_bytes,
+                        hipStream_t stream);
+
 /* Size of the fixed device scratch behind tts_assign_bins_noalloc (40 MiB per GPU: enough for
  * G = 2^20 gaussians on 1920 x 1072 at S = 16, which needs 36.4 MiB). */
 #define TTS_BIN_SCRATCH_BYTES ((size_t)40 << 20)

@@ -124,16 +124,16 @@ def geom_bwd(params, camera, grad9, near=NEAR, blur=BLUR, out=None, sh_rest=None
 
 # -------------------------------------------------------------------------------- binning --
 def bin_workspace(G, H, W, S, device):
-    """Zero-initialised workspace for assign_bins (kept zeroed by the library)."""
+    """Workspace for assign_bins (every pass writes what the next one reads: no initial values)."""
     n = _lib.load().tts_bin_workspace_bytes(G, H, W, S)
-    return torch.zeros(max(n, 1), device=device, dtype=U8)
+    return torch.empty(max(n, 1), device=device, dtype=U8)
 
 
 def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, idx=None,
-                valid=None, count=None, ncand=None, inv=None, order=None):
+                valid=None, count=None, ncand=None, inv=None, order=None, idx_dtype=I32):
     """mu2d: [G,2] fp32 (or any [G,>=2] row-contiguous view, e.g. the proj record),
-    keep: [G] uint8 or bool.  Returns idx[T,K] int32, valid[T,K] uint8, count[T], ncand[T];
-    the inverse table inv[G,9] and the heaviest-first tile order[T] are written when buffers are
+    keep: [G] uint8 or bool.  Returns idx[T,K] int32 (idx_dtype=torch.int64: int64),
+    valid[T,K] uint8, count[T], ncand[T]; the inverse table inv[G,9] and the heaviest-first tile order[T] are written when buffers are
     passed."""
     G = mu2d.shape[0]
     dev = mu2d.device
@@ -146,11 +146,13 @@ def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, i
     if S not in (16, 32) or H % S or W % S:
         raise ValueError(f"tile side {S} must be 16 or 32 and divide {H}x{W}")
     T = (H // S) * (W // S)
-    idx = torch.empty(T, K, device=dev, dtype=I32) if idx is None else idx
+    if idx_dtype not in (I32, torch.int64):
+        raise ValueError(f"idx_dtype must be torch.int32 or torch.int64, got {idx_dtype}")
+    idx = torch.empty(T, K, device=dev, dtype=idx_dtype) if idx is None else idx
     valid = torch.empty(T, K, device=dev, dtype=U8) if valid is None else valid
     count = torch.empty(T, device=dev, dtype=I32) if count is None else count
     ncand = torch.empty(T, device=dev, dtype=I32) if ncand is None else ncand
-    require(idx, "idx", I32, (T, K), dev)
+    require(idx, "idx", idx_dtype, (T, K), dev)
     require(valid, "valid", U8, (T, K), dev)
     require(count, "count", I32, (T,), dev)
     require(ncand, "ncand", I32, (T,), dev)
@@ -159,7 +161,7 @@ def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, i
     if order is not None:
         require(order, "order", I32, (T,), dev)
     workspace = bin_workspace(G, H, W, S, dev) if workspace is None else workspace
-    call("tts_assign_bins", ptr(mu2d), mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span,
+    call("tts_assign_bins" if idx_dtype == I32 else "tts_assign_bins_i64", ptr(mu2d), mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span,
          ptr(idx), ptr(valid), ptr(count), ptr(ncand), ptr(inv), ptr(order), ptr(workspace),
          workspace.numel(), stream())
     return idx, valid, count, ncand
