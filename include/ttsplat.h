@@ -258,6 +258,11 @@ size_t tts_loss_workspace_bytes(int H, int W);
  *   loss = (1-l) * sum|x-y| / (3HW) + l * (1 - sumS / (3 (H-10)(W-10))). */
 int tts_loss_partials_count(int H, int W, int* n_ssim);
 
+/* Loss value (1-lambda) sum|x-y|/N + lambda (1 - sum S/Ns) from the partial sums
+ * tts_loss_grad / tts_loss_grad_stats wrote for an H x W image; loss: a device scalar. */
+int tts_loss_value(const float* partials, int H, int W, double lambda, float* loss,
+                   hipStream_t stream);
+
 /* The target's SSIM statistics (stats: tts_loss_stats_bytes bytes, written whole), computed
  * whenever the target changes: the target maps muy/sy that tools/resident_traced.py:305-325
  * builds and recompute_gt_stats refreshes on each view switch (:677-678).  Size limits as
@@ -501,6 +506,12 @@ int tts_relocate(float* params, float* m, float* v, float* sh_rest, float* sh_m,
 
 /* Fill n fp32 values with zero (a kernel, so graph captures hold no memset node). */
 int tts_zero(float* buf, int64_t n, hipStream_t stream);
+
+/* Background block bg[4] = (softplus(w_b_raw), c_b r, g, b) (spike/render.py:28), and
+ * gw_b_raw[0] = softplus'(w_b_raw) * sum gwb[0..n) (spike's autograd through it). */
+int tts_background(const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream);
+int tts_background_grad(const float* gwb, int n, const float* w_b_raw, float* gw_b_raw,
+                        hipStream_t stream);
 
 /* ---- dense (unbinned) forms: every gaussian against every pixel it may weigh on ---- */
 

@@ -1280,6 +1280,38 @@ int launch_geom_seam(float* params, int G, const float* cam_b, const float* cam_
   return launch_status();
 }
 
+// The blend's background block [w_b, c_b], w_b = softplus(w_b_raw) (spike/render.py:28), and the
+// gradient back to w_b_raw from per-tile partial sums of dL/dw_b (summed in 64 bits, a fixed
+// order).  Latency-bound launches of one wave, in place of two (forward) and eight (backward)
+// tensor operations on four floats.
+__global__ __launch_bounds__(64) void k_background(const float* __restrict__ raw,
+                                                   const float* __restrict__ c_b,
+                                                   float* __restrict__ bg) {
+  if (threadIdx.x == 0) {
+    const float x = raw[0];
+    bg[0] = x > 20.0f ? x : log1pf(expf(x));
+  } else if (threadIdx.x < 4) {
+    bg[threadIdx.x] = c_b[threadIdx.x - 1];
+  }
+}
+
+__global__ __launch_bounds__(256) void k_background_grad(const float* __restrict__ gwb, int n,
+                                                         const float* __restrict__ raw,
+                                                         float* __restrict__ graw) {
+  __shared__ double s_sum[4];
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) v += (double)gwb[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const float g = (float)((s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3])), x = raw[0];
+    const float z = expf(x);
+    graw[0] = x > 20.0f ? g : g * z / (z + 1.0f);
+  }
+}
+
 }  // namespace tts
 
 using namespace tts;
@@ -1550,6 +1582,19 @@ int tts_zero(float* buf, int64_t n, hipStream_t stream) {
   if (n < 0 || (n > 0 && !buf)) return TTS_EINVAL;
   if (n == 0) return TTS_OK;
   k_zero<<<grid1d(n, 256), 256, 0, stream>>>(buf, n);
+  return launch_status();
+}
+
+int tts_background(const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream) {
+  if (!w_b_raw || !c_b || !bg) return TTS_EINVAL;
+  k_background<<<1, 64, 0, stream>>>(w_b_raw, c_b, bg);
+  return launch_status();
+}
+
+int tts_background_grad(const float* gwb, int n, const float* w_b_raw, float* gw_b_raw,
+                        hipStream_t stream) {
+  if (n < 0 || (n > 0 && !gwb) || !w_b_raw || !gw_b_raw) return TTS_EINVAL;
+  k_background_grad<<<1, 256, 0, stream>>>(gwb, n, w_b_raw, gw_b_raw);
   return launch_status();
 }
 

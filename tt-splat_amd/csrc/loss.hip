@@ -66,12 +66,18 @@ __device__ __forceinline__ void bst(Rsrc r, unsigned voff, float v) {
 // ------------------------------------------------------------------ target statistics ------
 // One block per (64 x 16 tile of the valid map, channel): mu_y and s_y of the clamped target ->
 // stats[2][3][Wo][Ho], each channel's planes column-major (the step kernel reads them along map
-// rows per lane).
+// rows per lane), and the target channel-planar ([3][H][W], after the statistics planes: the step
+// kernel's loads of one channel then touch contiguous floats; the interleaved image spreads a
+// wave's 64 columns over six cache lines per load).  Bound by its stores and the interleaved
+// loads: the statistics go out through LDS in runs of 16 rows of a column (64 bytes; a lane
+// storing its own 4 columns wrote 4-byte pieces, 12.4 us at 640x480), and the planar copy is made
+// from the rows the vertical filter holds anyway (its own pass over the target: 4.3 us).
 constexpr int kSW = 64, kSH = 16, kSR = 6;   // tile, vertical run (3 runs cover 16 rows)
 __global__ __launch_bounds__(256) void k_loss_target_stats(const float* __restrict__ y, int H,
                                                            int W, int tiles_x, Taps taps,
                                                            float* __restrict__ stats) {
   __shared__ float V[2][kSH][kSW + kHalo + 1];
+  __shared__ float F[2][kSW][kSH + 1];
   const int Ho = H - kHalo, Wo = W - kHalo;
   const int t = blockIdx.x / 3, ch = blockIdx.x - 3 * t;
   const int R0 = (t / tiles_x) * kSH, C0 = (t % tiles_x) * kSW;
@@ -83,7 +89,18 @@ __global__ __launch_bounds__(256) void k_loss_target_stats(const float* __restri
     const unsigned base = gc < W ? (unsigned)((((R0 + m0) * W + gc) * 3 + ch) * 4) : kOOB;
     float v[kSR + kHalo];
 #pragma unroll
-    for (int k = 0; k < kSR + kHalo; ++k) v[k] = clamp01(bld(ys, base + (unsigned)k * W * 12u));
+    for (int k = 0; k < kSR + kHalo; ++k) v[k] = bld(ys, base + (unsigned)k * W * 12u);
+    // this thread's share of the planar copy: its run's own rows, and past the last tile row and
+    // column the halo beyond them
+    const bool own_c = gc < W && (j < kSW || C0 + kSW >= Wo);
+    const bool last_r = R0 + kSH >= Ho && m0 + kSR >= kSH;
+    float* yp = stats + 6 * (size_t)Ho * Wo + (size_t)ch * H * W + gc;
+#pragma unroll
+    for (int k = 0; k < kSR + kHalo; ++k) {
+      const int r = R0 + m0 + k;
+      if (own_c && r < H && (last_r || (k < kSR && m0 + k < kSH))) yp[(size_t)r * W] = v[k];
+      v[k] = clamp01(v[k]);
+    }
     float a[2][kSR];
 #pragma unroll
     for (int o = 0; o < kSR; ++o) a[0][o] = a[1][o] = 0.f;
@@ -124,29 +141,23 @@ __global__ __launch_bounds__(256) void k_loss_target_stats(const float* __restri
       }
     }
   }
-  const int gm = R0 + m;
+#pragma unroll
+  for (int o = 0; o < 4; ++o) {
+    F[0][q0 + o][m] = f[0][o];
+    F[1][q0 + o][m] = f[1][o] - f[0][o] * f[0][o];
+  }
+  __syncthreads();
+  const int fr = tid & (kSH - 1), gm = R0 + fr;
   const size_t plane = (size_t)Ho * Wo;
 #pragma unroll
   for (int o = 0; o < 4; ++o) {
-    const int gq = C0 + q0 + o;
+    const int q = (tid >> 4) + o * 16, gq = C0 + q;
     if (gm < Ho && gq < Wo) {
       const size_t i = (size_t)gq * Ho + gm;   // column-major: a column's rows are contiguous
-      stats[(size_t)ch * plane + i] = f[0][o];
-      stats[(size_t)(3 + ch) * plane + i] = f[1][o] - f[0][o] * f[0][o];
+      stats[(size_t)ch * plane + i] = F[0][q][fr];
+      stats[(size_t)(3 + ch) * plane + i] = F[1][q][fr];
     }
   }
-}
-
-// The target channel-planar ([3][H][W], after the statistics planes): the step kernel's loads of
-// one channel then touch contiguous floats (the interleaved image spreads a wave's 64 columns
-// over six cache lines per load).
-__global__ __launch_bounds__(256) void k_loss_target_planar(const float* __restrict__ y,
-                                                            int64_t n, float* __restrict__ yp) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  yp[i] = y[i * 3];
-  yp[n + i] = y[i * 3 + 1];
-  yp[2 * n + i] = y[i * 3 + 2];
 }
 
 // Random-background compositing of a training target (the reference's --random-bg,
@@ -467,6 +478,36 @@ __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
   }
 }
 
+// The loss value from the step kernel's partial sums, in 64 bits and in a fixed order:
+// (1 - l) sum|x - y| / N + l (1 - sum S / Ns).  One block: a latency-bound launch in place of a
+// dozen (two conversions, two sums and the scalar arithmetic as tensor operations, some 60 us of
+// launches per loss value).
+__global__ __launch_bounds__(1024) void k_loss_value(const float* __restrict__ partials, int nb,
+                                                     double n, double ns, double lambda,
+                                                     float* __restrict__ out) {
+  __shared__ double s_sum[2][16];
+  double v[2] = {0.0, 0.0};
+  for (int i = threadIdx.x; i < nb; i += 1024) {
+    v[0] += (double)partials[i];
+    v[1] += (double)partials[nb + i];
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+    if ((threadIdx.x & 63) == 0) s_sum[k][threadIdx.x >> 6] = v[k];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0, l1 = 0.0;
+    for (int w = 0; w < 16; ++w) {
+      s += s_sum[0][w];
+      l1 += s_sum[1][w];
+    }
+    out[0] = (float)((1.0 - lambda) * l1 / n + lambda * (1.0 - s / ns));
+  }
+}
+
 // 40 rows: with 256 threads phase 4 takes exactly 4 runs of 10 rows, phases 2 and 3 use 250 of
 // the threads (5 runs on each of the 50 map rows), and V's 51 KB still lets three blocks share
 // a CU.  Measured at 1264x832: 34 rows 32.4 us, 38 rows 32.5, 40 rows 30.4, 41 rows 30.4 (42
@@ -514,14 +555,20 @@ int tts_loss_partials_count(int H, int W, int* n_ssim) {
   return 2 * nb;
 }
 
+int tts_loss_value(const float* partials, int H, int W, double lambda, float* loss,
+                   hipStream_t stream) {
+  if (!partials || !loss) return TTS_EINVAL;
+  if (!loss_size_ok(H, W)) return TTS_EINVAL;
+  k_loss_value<<<1, 1024, 0, stream>>>(partials, fused_items(H, W), 3.0 * H * W,
+                                       3.0 * (H - kHalo) * (W - kHalo), lambda, loss);
+  return launch_status();
+}
+
 int tts_loss_target_stats(const float* target, int H, int W, float* stats, hipStream_t stream) {
   if (!target || !stats) return TTS_EINVAL;
   if (!loss_size_ok(H, W)) return TTS_EINVAL;
   const int tx = (W - kHalo + kSW - 1) / kSW, ty = (H - kHalo + kSH - 1) / kSH;
   k_loss_target_stats<<<tx * ty * 3, 256, 0, stream>>>(target, H, W, tx, make_taps(), stats);
-  const int64_t n = (int64_t)H * W;
-  k_loss_target_planar<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(
-      target, n, stats + 6 * (size_t)(H - kHalo) * (size_t)(W - kHalo));
   return launch_status();
 }
 

@@ -13,6 +13,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libttsplat.
 
 _c_int, _c_float, _vp = ctypes.c_int, ctypes.c_float, ctypes.c_void_p
 _c_size, _c_i64, _c_u32 = ctypes.c_size_t, ctypes.c_int64, ctypes.c_uint32
+_c_dbl = ctypes.c_double
 
 # name -> (restype, argtypes); must match include/ttsplat.h
 SIGNATURES = {
@@ -58,6 +59,9 @@ SIGNATURES = {
     "tts_loss_grad_stats": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_float, _vp, _vp, _vp]),
     "tts_composite_random_bg": (_c_int, [_vp, _c_int, _c_int, _vp, _c_int, _c_u32, _vp, _vp,
                                          _vp]),
+    "tts_loss_value": (_c_int, [_vp, _c_int, _c_int, _c_dbl, _vp, _vp]),
+    "tts_background": (_c_int, [_vp, _vp, _vp, _vp]),
+    "tts_background_grad": (_c_int, [_vp, _c_int, _vp, _vp, _vp]),
     "tts_loss_partials_count": (_c_int, [_c_int, _c_int, ctypes.POINTER(_c_int)]),
     "tts_loss_grad": (_c_int, [_vp, _vp, _c_int, _c_int, _c_float, _vp, _vp, _vp, _c_size, _vp]),
     "tts_adam_advance": (_c_int, [_vp, _c_float, _c_float, _vp]),

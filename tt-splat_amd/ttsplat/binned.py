@@ -72,6 +72,21 @@ def background(model, device):
     return torch.cat([w_b, c_b]).contiguous()
 
 
+def _raw_background(model, device):
+    """The model's (w_b_raw, c_b) as fp32 tensors on `device` (differentiable conversions)."""
+    w_b_raw = torch.as_tensor(model.w_b_raw, dtype=F32, device=device)
+    c_b = torch.as_tensor(model.c_b, dtype=F32, device=device)
+    return (w_b_raw if w_b_raw.numel() == 1 else w_b_raw.reshape(1),
+            c_b if c_b.numel() == 3 else c_b.reshape(3))
+
+
+def _raw_background_grads(ctx, at, gwb, w_b_raw, c_b):
+    """Gradients of the inputs at positions `at`, `at + 1`: w_b_raw's from the partial sums of
+    dL/dw_b; c_b is a constant of the reference model, its gradient zero."""
+    gw = kernels.background_grad(gwb, w_b_raw) if ctx.needs_input_grad[at] else None
+    return gw, torch.zeros_like(c_b) if ctx.needs_input_grad[at + 1] else None
+
+
 @torch.no_grad()
 def assign_bins(mu2d, keep, tmap, R=1, K=128, span=None):
     """Per-tile gaussian lists (tools/m4_train_binned.py:75-127) in the reference layout:
@@ -178,22 +193,27 @@ class BinnedRender(torch.autograd.Function):
     per-slot gradients -> slot->gaussian reduce (through the inverse table when the bins came
     with one, else an atomic scatter) -> geometry bwd.  proj: P's projection from this camera
     when the caller has it already; order: the tiles heaviest first, the splat kernels' dispatch
-    order (26.0 -> 19.0 us forward at G = 100k, 1264x832)."""
+    order (26.0 -> 19.0 us forward at G = 100k, 1264x832).  The background is either the block bg
+    [4] or, with bg None, made here from w_b_raw and c_b."""
 
     @staticmethod
-    def forward(ctx, P, camera, bg, idx32, v8, inv, H, W, S, k, proj=None, order=None):
+    def forward(ctx, P, camera, bg, idx32, v8, inv, H, W, S, k, proj=None, order=None,
+                w_b_raw=None, c_b=None):
         Pc = P.detach().contiguous()
+        if bg is None:
+            w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
+            bg = kernels.background(w_b_raw, c_b)
         if proj is None:
             proj, _ = kernels.geom_fwd(Pc, camera)
         img, den = kernels.splat_fwd(proj, idx32, v8, bg, H, W, S, k, order=order)
-        ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den)
+        ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw, c_b)
         ctx.inv, ctx.order = inv, order
         ctx.meta = (H, W, S, k)
         return img
 
     @staticmethod
     def backward(ctx, gimg):
-        Pc, camera, bg, idx32, v8, proj, img, den = ctx.saved_tensors
+        Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw, c_b = ctx.saved_tensors
         H, W, S, k = ctx.meta
         gwb = torch.empty(idx32.shape[0], device=Pc.device, dtype=F32)
         gslot = None
@@ -207,9 +227,13 @@ class BinnedRender(torch.autograd.Function):
         else:
             grad9 = kernels.slot_scatter(gslot, idx32, v8, Pc.shape[0])
         gP = kernels.geom_bwd(Pc, camera, grad9)
-        gbg = torch.zeros(4, device=Pc.device, dtype=F32)
-        gbg[0] = gwb.sum()
-        return gP, None, gbg, None, None, None, None, None, None, None, None, None
+        gbg = gw = gc = None
+        if w_b_raw is not None:
+            gw, gc = _raw_background_grads(ctx, 12, gwb, w_b_raw, c_b)
+        else:
+            gbg = torch.zeros(4, device=Pc.device, dtype=F32)
+            gbg[0] = gwb.sum()
+        return gP, None, gbg, None, None, None, None, None, None, None, None, None, gw, gc
 
 
 def render_binned_device(model, cam, tmap, R=1, K=128, cached_bins=None, return_bins=False,
@@ -231,6 +255,6 @@ def render_binned_device(model, cam, tmap, R=1, K=128, cached_bins=None, return_
     else:
         bins = cached_bins
         idx32, v8 = _checked_bins(bins, P.shape[0])
-    img = BinnedRender.apply(P, camera, background(model, dev), idx32, v8, inv, tmap.H, tmap.W,
-                             tmap.S, float(k), proj, order)
+    img = BinnedRender.apply(P, camera, None, idx32, v8, inv, tmap.H, tmap.W, tmap.S, float(k),
+                             proj, order, *_raw_background(model, dev))
     return (img, bins) if return_bins else img

@@ -30,6 +30,27 @@ def version():
 
 
 # ------------------------------------------------------------------------------- geometry --
+def background(w_b_raw, c_b):
+    """bg block [softplus(w_b_raw), c_b r, g, b] from two device tensors of 1 and 3 elements."""
+    dev = w_b_raw.device
+    require(w_b_raw, "w_b_raw", F32)
+    require(c_b, "c_b", F32, None, dev)
+    if w_b_raw.numel() != 1 or c_b.numel() != 3:
+        raise ValueError("w_b_raw must hold one element and c_b three")
+    bg = torch.empty(4, device=dev, dtype=F32)
+    call("tts_background", ptr(w_b_raw), ptr(c_b), ptr(bg), stream())
+    return bg
+
+
+def background_grad(gwb, w_b_raw):
+    """dL/dw_b_raw, shaped like it, from the partial sums gwb of dL/dw_b."""
+    require(gwb, "gwb", F32)
+    require(w_b_raw, "w_b_raw", F32, None, gwb.device)
+    g = torch.empty_like(w_b_raw)
+    call("tts_background_grad", ptr(gwb), gwb.numel(), ptr(w_b_raw), ptr(g), stream())
+    return g
+
+
 SH_REST = 15   # rest coefficients per channel (SH degrees 1-3)
 
 
@@ -625,12 +646,15 @@ def loss_grad_stats(image, target, stats, lam=0.2, gimage=None, partials=None):
 
 def loss_from_partials(partials, H, W, lam=0.2):
     """Loss value from the partial sums written by loss_grad (a device scalar)."""
-    _, ns = loss_partials_count(H, W)
-    s_sum = partials[:ns].double().sum()
-    l1_sum = partials[ns:].double().sum()
-    n = 3.0 * H * W
-    n_s = 3.0 * (H - 10) * (W - 10)
-    return ((1.0 - lam) * l1_sum / n + lam * (1.0 - s_sum / n_s)).float()
+    n, ns = loss_partials_count(H, W)
+    if not (partials.is_cuda and partials.dtype == F32 and partials.is_contiguous()
+            and partials.numel() == n):    # partials moved or converted by the caller
+        l1_sum, s_sum = partials[ns:].double().sum(), partials[:ns].double().sum()
+        return ((1.0 - lam) * l1_sum / (3.0 * H * W)
+                + lam * (1.0 - s_sum / (3.0 * (H - 10) * (W - 10)))).float()
+    loss = torch.empty((), device=partials.device, dtype=F32)
+    call("tts_loss_value", ptr(partials), H, W, float(lam), ptr(loss), stream())
+    return loss
 
 
 # ----------------------------------------------------------------------------------- adam --

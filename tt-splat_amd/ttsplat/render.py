@@ -23,7 +23,7 @@ constant (a registered buffer in the reference model, spike/model.py:51): its gr
 import torch
 
 from . import kernels
-from .binned import background, params_of
+from .binned import _raw_background, _raw_background_grads, params_of
 
 F32 = torch.float32
 ARMS = ("A", "B", "SZ", "RV")
@@ -39,10 +39,12 @@ def _check_arm(arm, sh_degree=0):
 class DenseRender(torch.autograd.Function):
     """bt: (depth_beta, depth_tau) [2] for arm B, or None; szb: softz_beta [1] for arm SZ, or
     None; rest: the SH rest coefficients in the library layout [15,3,G] (sh_degree > 0), or
-    None; blend: "A", "SZ" or "RV" (arm B blends as A)."""
+    None; blend: "A", "SZ" or "RV" (arm B blends as A).  The background is either the block bg [4]
+    or, with bg None, made here from w_b_raw and c_b."""
 
     @staticmethod
-    def forward(ctx, P, camera, bg, bt, szb, rest, sh_degree, blend, H, W, k, blur, near):
+    def forward(ctx, P, camera, bg, bt, szb, rest, sh_degree, blend, H, W, k, blur, near,
+                w_b_raw=None, c_b=None):
         Pc = P.detach().contiguous()
         btc = None if bt is None else bt.detach().float().contiguous()
         szc = None if szb is None else szb.detach().float().reshape(1).contiguous()
@@ -50,19 +52,23 @@ class DenseRender(torch.autograd.Function):
         deg = int(sh_degree) if rc is not None else 0
         proj, _ = kernels.geom_fwd(Pc, camera, near=near, blur=blur, depth_bt=btc, sh_rest=rc,
                                    sh_degree=deg)
+        if bg is None:
+            w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
+            bg = kernels.background(w_b_raw, c_b)
         bgc = bg.detach().contiguous()
         if blend == "A":
             img, den = kernels.render_dense(proj, H, W, k, bgc)
             aux = None
         else:
             img, den, aux = kernels.render_dense_arm(proj, H, W, k, bgc, blend, szc)
-        ctx.save_for_backward(Pc, camera, bg, proj, img, den, btc, szc, aux, rc)
+        ctx.save_for_backward(Pc, camera, bg, proj, img, den, btc, szc, aux, rc,
+                              w_b_raw, c_b)
         ctx.meta = (H, W, k, blur, near, blend, deg)
         return img
 
     @staticmethod
     def backward(ctx, gimg):
-        Pc, camera, bg, proj, img, den, btc, szc, aux, rc = ctx.saved_tensors
+        Pc, camera, bg, proj, img, den, btc, szc, aux, rc, w_b_raw, c_b = ctx.saved_tensors
         H, W, k, blur, near, blend, deg = ctx.meta
         bgc = bg.detach().contiguous()
         gi = gimg.float().contiguous()
@@ -84,8 +90,13 @@ class DenseRender(torch.autograd.Function):
                                               sh_rest=rc, sh_degree=deg, sh_dirgrad=True)
             if gdw is not None:
                 gbt = gdw.sum(0)
-        gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
-        return gP, None, gbg, gbt, gszb, grest, None, None, None, None, None, None, None
+        gbg = gw = gc = None
+        if w_b_raw is not None:
+            gw, gc = _raw_background_grads(ctx, 13, gwb, w_b_raw, c_b)
+        else:
+            gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
+        return (gP, None, gbg, gbt, gszb, grest, None, None, None, None, None, None, None, gw,
+                gc)
 
 
 def render(model, cam, arm, k=4.0, blur_eps=0.3, near=0.2, sh_degree=0):
@@ -104,6 +115,6 @@ def render(model, cam, arm, k=4.0, blur_eps=0.3, near=0.2, sh_degree=0):
     color_rest = getattr(model, "color_rest", None)
     if int(sh_degree) > 0 and color_rest is not None:        # spike/render.py:23-25
         rest = kernels.sh_rest_layout(color_rest.to(dev, F32))
-    return DenseRender.apply(P, cam.device_block(dev), background(model, dev), bt, szb, rest,
-                             int(sh_degree), blend, cam.H, cam.W, float(k), float(blur_eps),
-                             float(near))
+    return DenseRender.apply(P, cam.device_block(dev), None, bt, szb, rest, int(sh_degree), blend,
+                             cam.H, cam.W, float(k), float(blur_eps), float(near),
+                             *_raw_background(model, dev))
