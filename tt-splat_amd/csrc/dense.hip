@@ -13,10 +13,10 @@
 // Quad forward: a block per tile of pixels, the gaussians whose support reaches it listed in LDS
 // (DenseWalk below).  Quad backward: a pass over the pixels for their WSR gradients (gnum = gC/den,
 // gden = -(gC.C)/den), then waves per gaussian over the pixels of its support box.
-// theta forward: one thread per pixel, gaussians staged through LDS 256 at a time.
-// theta backward: one thread per gaussian; the pixels are cut into bands, each (gaussian chunk,
-// band) block stages its band's per-pixel WSR gradients in LDS and accumulates the gaussian's sums
-// over the band.  Band partials go to a workspace and are summed in band order by a second kernel.
+// theta forward: the waves of a block share its pixels and split the gaussians, staged in LDS.
+// theta backward: a block owns 64 gaussians and a band of pixels, whose WSR gradients it stages in
+// LDS; its waves split the pixels.  Band partials go to a workspace and are summed in band order
+// by a second kernel.
 // All results are deterministic and there are no floating-point atomics.
 //
 // The quad form also renders the two per-pixel occlusion arms of spike/arms.py (ARM template):
@@ -32,21 +32,25 @@
 
 namespace tts {
 
-constexpr int kDenseChunk = 256;
 constexpr int kArmA = 0, kArmSZ = 1, kArmRV = 2;   // TTS_ARM_* values
 constexpr int kQuadComp = 9;    // a, b, c, mu_x, mu_y, col_o r, g, b, o_col
 constexpr int kThetaComp = 10;  // theta 0..5, o, color r, g, b
 constexpr int kDenseTargetBlocks = 2048;
 constexpr size_t kDenseMaxWorkspace = size_t(1) << 30;
 
-// Pixels per band (a multiple of 256) for G gaussians over P pixels.
+// Pixels per band of the theta form's backward (a multiple of 256) for G gaussians over P pixels:
+// up to 2048 (64 gaussians, band) blocks of 16 waves, but bands of whole 1024-pixel stagings where
+// those still give each CU two blocks.  Measured, about 512 / 1024 / 2048 blocks (us, band sums
+// included): G 2000, 128x128 26 / 28 / 34; G 6000, 100x100 45 / 43 / 45; 200x200 135 / 131 / 122;
+// G 2000, 600x600 360 / 350 / 346.
 inline int dense_band_pixels(int G, int P) {
-  const int gchunks = (G + kDenseChunk - 1) / kDenseChunk;
+  const int gchunks = (G + 63) / 64;
   int nb = kDenseTargetBlocks / (gchunks > 0 ? gchunks : 1);
   if (nb < 1) nb = 1;
   int pb = (P + nb - 1) / nb;
   pb = ((pb + 255) / 256) * 256;
   if (pb < 256) pb = 256;
+  if (pb < 1024 && (int64_t)gchunks * ((P + 1023) / 1024) >= 512) pb = 1024;
   // keep the partials within the workspace cap
   while ((size_t)((P + pb - 1) / pb) * (size_t)G * kThetaComp * 4 > kDenseMaxWorkspace) pb *= 2;
   return pb;
@@ -334,55 +338,86 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
   }
 }
 
-__global__ __launch_bounds__(256) void k_wsr_dense(const float* __restrict__ theta,
-                                                   const float* __restrict__ o,
-                                                   const float* __restrict__ color,
-                                                   const uint8_t* __restrict__ keep,
-                                                   const float* __restrict__ phi, int G, int P,
-                                                   const float* __restrict__ bg,
-                                                   float* __restrict__ C,
-                                                   float* __restrict__ den_out) {
-  __shared__ float4 s_a[kDenseChunk];  // theta 0..3
-  __shared__ float4 s_b[kDenseChunk];  // theta 4, 5, -, -
-  __shared__ float4 s_c[kDenseChunk];  // o*keep*color, o*keep
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  float f[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (p < P) {
+// theta form, forward: 16 waves share a block's 64 * PX pixels (PX per lane), the gaussians are
+// dealt to the waves in runs and the waves' sums joined in wave order.  Every pair counts (the
+// basis is arbitrary, so there is no support box): bound by the 10 CU cycles of LDS a gaussian's
+// 40 bytes take per wave and, with PX pixels sharing them, by the VALU (13 instructions a pair).
+constexpr int kThetaThreads = 1024;
+constexpr int kThetaWaves = kThetaThreads / 64;
+
+template <int PX>
+__global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
+    const float* __restrict__ theta, const float* __restrict__ o, const float* __restrict__ color,
+    const uint8_t* __restrict__ keep, const float* __restrict__ phi, int G, int P,
+    const float* __restrict__ bg, float* __restrict__ C, float* __restrict__ den_out) {
+  __shared__ float4 s_a[kThetaThreads];  // theta 0..3
+  __shared__ float4 s_c[kThetaThreads];  // o*keep*color, o*keep
+  __shared__ float2 s_b[kThetaThreads];  // theta 4, 5
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int p0 = blockIdx.x * 64 * PX + lane;
+  float f[PX][6], n[PX][4];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) f[i] = phi[(int64_t)p * 6 + i];
+  for (int i = 0; i < PX; ++i) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) f[i][k] = p0 + i * 64 < P ? phi[(int64_t)(p0 + i * 64) * 6 + k] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) n[i][k] = 0.f;
   }
-  float nr = 0.f, ng = 0.f, nb = 0.f, nd = 0.f;
-  for (int g0 = 0; g0 < G; g0 += kDenseChunk) {
-    const int n = min(kDenseChunk, G - g0);
+  for (int g0 = 0; g0 < G; g0 += kThetaThreads) {
+    const int cnt = min(kThetaThreads, G - g0);
     __syncthreads();
-    if ((int)threadIdx.x < n) {
+    if ((int)threadIdx.x < cnt) {
       const int g = g0 + threadIdx.x;
       const float* th = theta + (int64_t)g * 6;
       const float ok = (keep && !keep[g]) ? 0.0f : o[g];
       s_a[threadIdx.x] = make_float4(th[0], th[1], th[2], th[3]);
-      s_b[threadIdx.x] = make_float4(th[4], th[5], 0.f, 0.f);
+      s_b[threadIdx.x] = make_float2(th[4], th[5]);
       s_c[threadIdx.x] = make_float4(ok * color[(int64_t)g * 3 + 0], ok * color[(int64_t)g * 3 + 1],
                                      ok * color[(int64_t)g * 3 + 2], ok);
     }
     __syncthreads();
-    for (int j = 0; j < n; ++j) {
-      const float4 A = s_a[j], B = s_b[j], Cc = s_c[j];
-      const float u = f[0] * A.x + f[1] * A.y + f[2] * A.z + f[3] * A.w + f[4] * B.x + f[5] * B.y;
-      const float r = relu_nan(u);
-      const float w = r * r;
-      nr += w * Cc.x;
-      ng += w * Cc.y;
-      nb += w * Cc.z;
-      nd += w * Cc.w;
+    const int j1 = (int)((wave + 1) * cnt) / kThetaWaves;
+#pragma unroll 4
+    for (int j = (int)(wave * cnt) / kThetaWaves; j < j1; ++j) {
+      const float4 A = s_a[j], Cc = s_c[j];
+      const float2 B = s_b[j];
+#pragma unroll
+      for (int i = 0; i < PX; ++i) {
+        const float u = f[i][0] * A.x + f[i][1] * A.y + f[i][2] * A.z + f[i][3] * A.w +
+                        f[i][4] * B.x + f[i][5] * B.y;
+        const float r = relu_nan(u);
+        const float w = r * r;
+        n[i][0] += w * Cc.x;
+        n[i][1] += w * Cc.y;
+        n[i][2] += w * Cc.z;
+        n[i][3] += w * Cc.w;
+      }
     }
   }
-  if (p < P) {
-    const float wb = bg[0];
-    const float d = nd + wb;
-    C[(int64_t)p * 3 + 0] = (nr + wb * bg[1]) / d;
-    C[(int64_t)p * 3 + 1] = (ng + wb * bg[2]) / d;
-    C[(int64_t)p * 3 + 2] = (nb + wb * bg[3]) / d;
-    if (den_out) den_out[p] = d;
+  // joined per PX: [wave][4][64] floats fill s_a
+  float* s = reinterpret_cast<float*>(s_a);
+#pragma unroll
+  for (int i = 0; i < PX; ++i) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[(wave * 4 + k) * 64 + lane] = n[i][k];
+    __syncthreads();
+    if (wave != i) continue;   // wave i finishes the block's i-th run of pixels
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kThetaWaves; ++w) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] += s[(w * 4 + k) * 64 + lane];
+    }
+    const int64_t p = p0 + i * 64;
+    if (p < P) {
+      const float wb = bg[0];
+      const float d = v[3] + wb;
+      C[p * 3 + 0] = (v[0] + wb * bg[1]) / d;
+      C[p * 3 + 1] = (v[1] + wb * bg[2]) / d;
+      C[p * 3 + 2] = (v[2] + wb * bg[3]) / d;
+      if (den_out) den_out[p] = d;
+    }
   }
 }
 
@@ -649,17 +684,25 @@ __global__ __launch_bounds__(256) void k_render_dense_bwd(
   out[((int64_t)blockIdx.y * G + g) * NC + lane] = o;
 }
 
-__global__ __launch_bounds__(256) void k_wsr_dense_bwd(
+// theta form, backward: a block owns 64 gaussians (one per lane) and a band of pixels, 1024 of
+// which it stages at a time with their WSR gradients; the 16 waves take runs of them and their
+// sums are joined in wave order into the band's partial.  Bound by the VALU (24 instructions a
+// pair).  256-thread blocks of 256 gaussians over 64 bands, and their 64 partials a gaussian, took
+// 44 us at G 2000, 128x128 (17 of it the band sums), 55 at G 6000, 100x100, 151 at 200x200; this
+// takes 26, 43 and 122.
+__global__ __launch_bounds__(kThetaThreads) void k_wsr_dense_bwd(
     const float* __restrict__ theta, const float* __restrict__ o, const float* __restrict__ color,
     const uint8_t* __restrict__ keep, const float* __restrict__ phi, int G, int P, int PB,
     const float* __restrict__ bg, const float* __restrict__ C, const float* __restrict__ den,
     const float* __restrict__ gC, float* __restrict__ part, float* __restrict__ gwb_part) {
-  __shared__ float4 s_px[256];
-  __shared__ float4 s_fa[256];  // phi 0..3
-  __shared__ float2 s_fb[256];  // phi 4..5
-  __shared__ float s_ftmp[4];
+  __shared__ float s_all[kThetaThreads * kThetaComp];
+  __shared__ float s_wb[kThetaWaves];
+  float4* s_px = reinterpret_cast<float4*>(s_all);
+  float4* s_fa = s_px + kThetaThreads;                                // phi 0..3
+  float2* s_fb = reinterpret_cast<float2*>(s_fa + kThetaThreads);     // phi 4..5
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int band = blockIdx.y;
-  const int g = blockIdx.x * 256 + threadIdx.x;
+  const int g = blockIdx.x * 64 + lane;
   const bool act = g < G;
   float th[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float og = 0.f, kp = 0.f, col[3] = {0.f, 0.f, 0.f};
@@ -673,11 +716,10 @@ __global__ __launch_bounds__(256) void k_wsr_dense_bwd(
   }
   const float ok = og * kp;
   const float cr = ok * col[0], cg = ok * col[1], cb = ok * col[2];
-  float st[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  float gr = 0.f, gg = 0.f, gbl = 0.f, gd = 0.f;
+  float v[kThetaComp] = {};   // theta 0..5, then sums of w q: r, g, b, den
   float wpart = 0.f;
   const int pend = min(P, (band + 1) * PB);
-  for (int p0 = band * PB; p0 < pend; p0 += 256) {
+  for (int p0 = band * PB; p0 < pend; p0 += kThetaThreads) {
     __syncthreads();
     const int pp = p0 + threadIdx.x;
     const bool in = pp < pend;
@@ -692,8 +734,10 @@ __global__ __launch_bounds__(256) void k_wsr_dense_bwd(
     s_fa[threadIdx.x] = fa;
     s_fb[threadIdx.x] = fb;
     __syncthreads();
-    const int n = min(256, pend - p0);
-    for (int j = 0; j < n; ++j) {
+    const int n = min(kThetaThreads, pend - p0);
+    const int j1 = (wave + 1) * n / kThetaWaves;
+#pragma unroll 2
+    for (int j = wave * n / kThetaWaves; j < j1; ++j) {
       const float4 q = s_px[j];
       const float4 fa2 = s_fa[j];
       const float2 fb2 = s_fb[j];
@@ -701,27 +745,47 @@ __global__ __launch_bounds__(256) void k_wsr_dense_bwd(
                       fb2.x * th[4] + fb2.y * th[5];
       const float r = relu_nan(u);
       const float w = r * r;
-      gr += w * q.x;
-      gg += w * q.y;
-      gbl += w * q.z;
-      gd += w * q.w;
+      v[6] += w * q.x;
+      v[7] += w * q.y;
+      v[8] += w * q.z;
+      v[9] += w * q.w;
       const float gu = r * (q.x * cr + q.y * cg + q.z * cb + q.w * ok);  // half of dL/du
-      st[0] += gu * fa2.x;
-      st[1] += gu * fa2.y;
-      st[2] += gu * fa2.z;
-      st[3] += gu * fa2.w;
-      st[4] += gu * fb2.x;
-      st[5] += gu * fb2.y;
+      v[0] += gu * fa2.x;
+      v[1] += gu * fa2.y;
+      v[2] += gu * fa2.z;
+      v[3] += gu * fa2.w;
+      v[4] += gu * fb2.x;
+      v[5] += gu * fb2.y;
     }
   }
   if (blockIdx.x == 0) {
-    const float tot = block_sum256(wpart, s_ftmp);
-    if (threadIdx.x == 0) gwb_part[band] = tot;
+    const float t = wave_sum(wpart);
+    if (lane == 0) s_wb[wave] = t;
   }
-  if (act) {
+  __syncthreads();
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < kThetaWaves; ++w) t += s_wb[w];
+    gwb_part[band] = t;
+  }
+#pragma unroll
+  for (int k = 0; k < kThetaComp; ++k) s_all[(wave * kThetaComp + k) * 64 + lane] = v[k];
+  __syncthreads();
+  float t = 0.f;
+  if (wave < kThetaComp) {   // wave k sums component k
+#pragma unroll
+    for (int w = 0; w < kThetaWaves; ++w) t += s_all[(w * kThetaComp + wave) * 64 + lane];
+  }
+  __syncthreads();
+  if (wave < kThetaComp) s_all[wave * 64 + lane] = t;
+  __syncthreads();
+  if (wave == 0 && act) {
     float* dst = part + ((int64_t)band * G + g) * kThetaComp;
 #pragma unroll
-    for (int i = 0; i < 6; ++i) dst[i] = 2.0f * st[i];
+    for (int i = 0; i < 6; ++i) dst[i] = 2.0f * s_all[i * 64 + lane];
+    const float gr = s_all[6 * 64 + lane], gg = s_all[7 * 64 + lane], gbl = s_all[8 * 64 + lane],
+                gd = s_all[9 * 64 + lane];
     // num = sum w_geo*o*keep*color, den = sum w_geo*o*keep + w_b
     dst[6] = kp * (col[0] * gr + col[1] * gg + col[2] * gbl + gd);  // dL/do
     dst[7] = ok * gr;                                              // dL/dcolor
@@ -740,13 +804,15 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
   const int64_t n = (int64_t)G * ncomp;
   if (i < n) {
     float s = 0.f;
+#pragma unroll 8
     for (int b = 0; b < nb; ++b) s += part[(int64_t)b * n + i];
     out[i] = s;
   }
-  if (i == 0 && gwb) {
+  if (blockIdx.x == 0 && threadIdx.x < 64 && gwb) {   // wave 0: lanes over the bands
     float s = 0.f;
-    for (int b = 0; b < nb; ++b) s += gwb_part[b];
-    gwb[0] = s;
+    for (int b = threadIdx.x; b < nb; b += 64) s += gwb_part[b];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) gwb[0] = s;
   }
 }
 
@@ -936,7 +1002,16 @@ int tts_wsr_dense(const float* theta, const float* o, const float* color, const 
   if ((G > 0 && (!theta || !o || !color)) || !phi || !bg || !C || P <= 0 || G < 0)
     return TTS_EINVAL;
   if (G > (1 << 30) || P > (1 << 30)) return TTS_EINVAL;
-  k_wsr_dense<<<grid1d(P, 256), 256, 0, stream>>>(theta, o, color, keep, phi, G, P, bg, C, den);
+  // Pixels per lane: four read the gaussians' LDS records a quarter as often, one makes four times
+  // the blocks.  Measured, one / four (us): G 2000, 128x128 19 / 37; G 6000, 100x100 45 / 94,
+  // 200x200 116 / 95; G 2000, 600x600 263 / 209 (one thread per pixel, a chain over G: 79, 230, 230
+  // and 278).
+  if (P <= 32768)
+    k_wsr_dense<1><<<grid1d(P, 64), kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P,
+                                                                bg, C, den);
+  else
+    k_wsr_dense<4><<<grid1d(P, 256), kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P,
+                                                                 bg, C, den);
   return launch_status();
 }
 
@@ -952,9 +1027,9 @@ int tts_wsr_dense_bwd(const float* theta, const float* o, const float* color,
   int PB;
   const int nb = theta_ws(workspace, workspace_bytes, G, P, &part, &gwbp, &PB);
   if (nb < 0) return nb;
-  dim3 grid(grid1d(G, 256), nb);
-  k_wsr_dense_bwd<<<grid, 256, 0, stream>>>(theta, o, color, keep, phi, G, P, PB, bg, C, den, gC,
-                                            part, gwbp);
+  dim3 grid(grid1d(G, 64), nb);
+  k_wsr_dense_bwd<<<grid, kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P, PB, bg, C,
+                                                      den, gC, part, gwbp);
   k_dense_reduce<<<grid1d((int64_t)G * kThetaComp, 256), 256, 0, stream>>>(
       part, nb, G, kThetaComp, gwbp, gtheta10, gwb);
   return launch_status();

@@ -37,6 +37,8 @@ def _bg(w_b, c_b, device):
 def _keep_u8(keep):
     if keep is None:
         return None
+    if keep.dtype == torch.bool:        # a bool's bytes are 0 and 1 already
+        return keep.contiguous().view(torch.uint8)
     return (keep != 0).to(torch.uint8).contiguous()
 
 
