@@ -19,7 +19,7 @@
 //   4 transposed vertical filter (a thread = one gradient column, a run of rows, so its image
 //     loads and gradient stores are coalesced), combined as dmeanS/dx = (T'A + 2 x T'B +
 //     y T'C) / Ns, gated by 0 <= x <= 1 (the clamp), plus the L1 term (1-l) sign(x-y) / N.
-// V, D and T share one 51 KB LDS buffer (each written after a barrier that ends the reads of
+// V, D and T share one LDS buffer (51 KB at 40 rows; each written after a barrier that ends the reads of
 // the one before; three blocks fit a CU); the loads a phase needs from global memory are issued
 // a phase ahead.  Each block also sums S over the map pixels of its tile and |x - y| over its
 // pixels.  Nothing is exchanged between blocks: the kernel needs no workspace.
@@ -33,10 +33,6 @@ constexpr int kHalo = kWin - 1;
 constexpr int kTW = 64;                 // gradient tile width
 constexpr int kMC = kTW + kHalo;        // 74 map columns
 constexpr int kIC = kTW + 2 * kHalo;    // 84 input columns
-constexpr int kVS = kIC + 1;            // LDS row strides (odd: column walks spread over banks)
-constexpr int kDS = kMC + 1;
-constexpr int kHC = 15;                 // phase 2: map columns per thread (5 runs cover 74)
-constexpr int kHC3 = 13;                // phase 3: gradient columns per thread (5 runs cover 64)
 constexpr int kTS = kTW + 1;
 constexpr float kC1 = 1e-4f;
 constexpr float kC2 = 9e-4f;
@@ -205,21 +201,27 @@ __device__ __forceinline__ int strip_tile(int s, int tiles_x, int tiles_y) {
   return row * tiles_x + k * kStrip + (r - row * w);
 }
 
-template <int TH>
+// A tile of TH gradient rows; phase 2 and 3 take runs of HC map and HC3 gradient columns.
+template <int TH_, int HC_, int HC3_>
 struct FGeo {
+  static constexpr int TH = TH_, HC = HC_, HC3 = HC3_;
   static constexpr int MR = TH + kHalo;              // map rows of the region
   static constexpr int VR = (MR + 2) / 3;            // phase 1: map rows per thread (3 runs)
   static constexpr int TR4 = (TH + 3) / 4;           // phase 4: gradient rows per thread
-  static constexpr int N2 = 5 * MR;                  // phase 2 and 3 threads
+  static constexpr int R2 = (kMC + HC - 1) / HC, R3 = (kTW + HC3 - 1) / HC3;   // runs per row
+  static constexpr int N2 = R2 * MR, N3 = R3 * MR;   // phase 2 and 3 threads
+  // LDS row strides: odd (column walks spread over banks), past the last run's reads
+  static constexpr int VS = (R2 * HC + kHalo > kIC ? R2 * HC + kHalo : kIC) | 1;
+  static constexpr int DS = (R3 * HC3 + kHalo > kMC ? R3 * HC3 + kHalo : kMC) | 1;
   static constexpr int TP = 4 * TR4 + kHalo;         // T rows per plane (phase 4 reads past MR)
-  static constexpr int kV = 3 * MR * kVS;            // floats of V
-  static_assert(3 * MR * kDS + kDS <= kV && 3 * TP * kTS <= kV, "D and T reuse V's space");
-  static_assert(3 * kIC <= 256 && N2 <= 256, "one pass each");
-  static_assert(5 * kHC >= kMC && 5 * kHC3 >= kTW && 3 * VR >= MR && 4 * TR4 >= TH, "cover");
+  static constexpr int kV = 3 * MR * VS;             // floats of V
+  static_assert(3 * MR * DS <= kV && 3 * TP * kTS <= kV, "D and T reuse V's space");
+  static_assert(3 * kIC <= 256 && N2 <= 256 && N3 <= 256, "one pass each");
+  static_assert(3 * VR >= MR && 4 * TR4 >= TH, "cover");
   static constexpr size_t lds_bytes = sizeof(float) * (size_t)kV;
 };
 
-template <int TH>
+template <class G>
 __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
                                                     const float* __restrict__ y,
                                                     const float* __restrict__ stats, int H,
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
                                                     float lambda, float inv_n, float inv_ns,
                                                     float* __restrict__ gout,
                                                     float* __restrict__ partials) {
-  using G = FGeo<TH>;
+  constexpr int TH = G::TH, kHC = G::HC, kHC3 = G::HC3, kVS = G::VS, kDS = G::DS;
   extern __shared__ float s_lds[];
   float* V = s_lds;
   float* D = s_lds;
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
   const Rsrc ys = rsrc(stats + 6 * (size_t)Ho * Wo + (size_t)ch * npix, npix * 4);
   const Rsrc ss = rsrc(stats, (size_t)Ho * Wo * 24);
   const unsigned plane4 = (unsigned)(Ho * Wo) * 4u;
-  // phase-2 role: map row m2, columns [q2, q2 + 15); its target statistics loaded up front
+  // phase-2 role: map row m2, columns [q2, q2 + kHC); its target statistics loaded up front
   const int m2 = tid % G::MR, q2 = (tid / G::MR) * kHC;
   const bool act2 = tid < G::N2;
   const int gm2 = R0 - kHalo + m2;
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
     for (int o = 0; o < kHC; ++o) dv[0][o] = dv[1][o] = dv[2][o] = 0.f;
 #pragma unroll
     for (int k = 0; k < kHC + kHalo; ++k) {
-      const int c = q2 + k;   // <= 84 < kVS: the row padding, feeding only dropped columns
+      const int c = q2 + k;   // < kVS: the row padding, feeding only dropped columns
       float vv[3];
 #pragma unroll
       for (int qn = 0; qn < 3; ++qn) vv[qn] = V[(qn * G::MR + m2) * kVS + c];
@@ -396,13 +398,13 @@ __global__ __launch_bounds__(256) void k_loss_fused(const float* __restrict__ x,
   //      gradient column c receives map columns c..c+10 through tap 10 - (q - c)
   float ta[3][kHC3];
   const int m3 = tid % G::MR, c3 = (tid / G::MR) * kHC3;
-  const bool act3 = tid < 5 * G::MR;
+  const bool act3 = tid < G::N3;
   if (act3) {
 #pragma unroll
     for (int o = 0; o < kHC3; ++o) ta[0][o] = ta[1][o] = ta[2][o] = 0.f;
 #pragma unroll
     for (int k = 0; k < kHC3 + kHalo; ++k) {
-      const int q = c3 + k;   // <= 74 < kDS: the row padding, feeding only dropped columns
+      const int q = c3 + k;   // < kDS: the row padding, feeding only dropped columns
       float dd[3];
 #pragma unroll
       for (int qn = 0; qn < 3; ++qn) dd[qn] = D[(qn * G::MR + m3) * kDS + q];
@@ -512,10 +514,35 @@ __global__ __launch_bounds__(1024) void k_loss_value(const float* __restrict__ p
 // the threads (5 runs on each of the 50 map rows), and V's 51 KB still lets three blocks share
 // a CU.  Measured at 1264x832: 34 rows 32.4 us, 38 rows 32.5, 40 rows 30.4, 41 rows 30.4 (42
 // rows would need 260 threads in phases 2 and 3).
-constexpr int kTH = 40;
+// Smaller tiles repeat more of the halo's work but give a small image enough blocks, and each
+// block a shorter chain: at 128x128 40 rows (24 blocks) 11.5 us, 24 rows 9.2, 16 rows 8.0, 8 rows
+// 6.5; at 320x480 11.5, 11.7, 10.1, 11.0; at 600x800 18.8, 17.7, 20.1, 23.9; at 832x1264 30.2,
+// 33.9, 37.0, 45.6.  A launch takes about a + b n with n = blocks per CU, rounded up (fitted to 15
+// sizes from 24x24 to 1072x1920, within 8 %); the rows with the least of it are taken.
+using Tile40 = FGeo<40, 15, 13>;
+using Tile24 = FGeo<24, 11, 10>;
+using Tile16 = FGeo<16, 9, 8>;
+using Tile8 = FGeo<8, 6, 5>;
 
 inline int fused_tiles_x(int W) { return (W + kTW - 1) / kTW; }
-inline int fused_items(int H, int W) { return 3 * fused_tiles_x(W) * ((H + kTH - 1) / kTH); }
+inline int loss_items(int H, int W, int rows) {
+  return 3 * fused_tiles_x(W) * ((H + rows - 1) / rows);
+}
+inline int loss_rows(int H, int W) {
+  struct Cost { int rows; double a, b; };   // us
+  constexpr Cost cost[] = {{40, 6.5, 4.7}, {24, 6.0, 3.1}, {16, 5.9, 2.2}, {8, 5.3, 1.4}};
+  int best = 40;
+  double least = 1e30;
+  for (const Cost& c : cost) {
+    const double us = c.a + c.b * ((loss_items(H, W, c.rows) + 255) / 256);
+    if (us < least) {
+      least = us;
+      best = c.rows;
+    }
+  }
+  return best;
+}
+inline int fused_items(int H, int W) { return loss_items(H, W, loss_rows(H, W)); }
 
 inline Taps make_taps() {
   Taps taps;
@@ -591,8 +618,18 @@ int tts_loss_grad_stats(const float* image, const float* target, const float* st
   const int tx = fused_tiles_x(W), ni = fused_items(H, W);
   const float inv_n = 1.0f / (3.0f * (float)H * (float)W);
   const float inv_ns = 1.0f / (3.0f * (float)(H - kHalo) * (float)(W - kHalo));
-  k_loss_fused<kTH><<<ni, 256, FGeo<kTH>::lds_bytes, stream>>>(
-      image, target, stats, H, W, tx, ni, make_taps(), lambda, inv_n, inv_ns, gimage, partials);
+  auto launch = [&](auto geo) {
+    using G = decltype(geo);
+    k_loss_fused<G><<<ni, 256, G::lds_bytes, stream>>>(image, target, stats, H, W, tx, ni,
+                                                      make_taps(), lambda, inv_n, inv_ns, gimage,
+                                                      partials);
+  };
+  switch (loss_rows(H, W)) {
+    case 40: launch(Tile40{}); break;
+    case 24: launch(Tile24{}); break;
+    case 16: launch(Tile16{}); break;
+    default: launch(Tile8{}); break;
+  }
   return launch_status();
 }
 
