@@ -416,32 +416,32 @@ __device__ __forceinline__ Camera load_camera(const float* __restrict__ cam) {
 // a loop bounded by rows * W would wait out one memory round trip per word.
 constexpr int kGeoBlock = 256;
 constexpr int kSeamRow = 3 * 15 + 9;  // floats of one staged row of the step seam (params, m, v, inv)
-// tid: the thread's index among the kGeoBlock threads that copy these rows (threadIdx.x, or
+// tid: the thread's index among the NT threads that copy these rows (threadIdx.x, or
 // its index in its half of a 512-thread block).
-template <int W, typename T>
+template <int W, int NT = kGeoBlock, typename T>
 __device__ __forceinline__ void stage_load(const T* __restrict__ src, int g0, int rows, T (&r)[W],
                                            int tid = threadIdx.x) {
   const T* base = src + (int64_t)g0 * W;
   const int last = rows * W - 1;
 #pragma unroll
-  for (int k = 0; k < W; ++k) r[k] = base[min(tid + k * kGeoBlock, last)];
+  for (int k = 0; k < W; ++k) r[k] = base[min(tid + k * NT, last)];
 }
-template <int W, int SW, typename T>
+template <int W, int SW, int NT = kGeoBlock, typename T>
 __device__ __forceinline__ void stage_put(const T (&r)[W], int rows, T* s, int tid = threadIdx.x) {
   const int n = rows * W;
 #pragma unroll
   for (int k = 0; k < W; ++k) {
-    const int i = tid + k * kGeoBlock;
+    const int i = tid + k * NT;
     if (i < n) s[(i / W) * SW + i % W] = r[k];
   }
 }
-template <int W, int SW, typename T>
+template <int W, int SW, int NT = kGeoBlock, typename T>
 __device__ __forceinline__ void stage_in(const T* __restrict__ src, int g0, int rows, T* s) {
   T r[W];
-  stage_load<W>(src, g0, rows, r);
-  stage_put<W, SW>(r, rows, s);
+  stage_load<W, NT>(src, g0, rows, r);
+  stage_put<W, SW, NT>(r, rows, s);
 }
-template <int W, int SW, typename T>
+template <int W, int SW, int NT = kGeoBlock, typename T>
 __device__ __forceinline__ void stage_out(T* __restrict__ dst, int g0, int rows, const T* s,
                                           int tid = threadIdx.x) {
   T* base = dst + (int64_t)g0 * W;
@@ -449,12 +449,12 @@ __device__ __forceinline__ void stage_out(T* __restrict__ dst, int g0, int rows,
   T r[W];
 #pragma unroll
   for (int k = 0; k < W; ++k) {
-    const int i = min(tid + k * kGeoBlock, n - 1);
+    const int i = min(tid + k * NT, n - 1);
     r[k] = s[(i / W) * SW + i % W];
   }
 #pragma unroll
   for (int k = 0; k < W; ++k) {
-    const int i = tid + k * kGeoBlock;
+    const int i = tid + k * NT;
     if (i < n) base[i] = r[k];
   }
 }
@@ -935,38 +935,44 @@ __device__ __forceinline__ void bwd_adam_row(
   }
 }
 
+// One wave per block: its 64 rows of LDS let eleven blocks share a CU (256 threads: two, eight
+// waves), no wave waits at a barrier for another's rows, and a small G reaches more CUs.  Training
+// step with 256 / 128 / 64 threads: G 10000, 800x800, bins kept 77.3 / 73.9 / 73.4 us; G 2000,
+// 128x128 67.1 / 66.5 / 65.6; G 60000, SH 2 113.0 / 112.5 / 111.6; G 100000, SH 3 + MCMC 175.7 /
+// 172.6 / 173.6.
+constexpr int kAdamBlock = 64;
 template <bool SH, bool MC>
-__global__ __launch_bounds__(256) void k_geom_bwd_adam(
+__global__ __launch_bounds__(kAdamBlock) void k_geom_bwd_adam(
     float* __restrict__ params, int G, float* __restrict__ rest, float* __restrict__ sh_m,
     float* __restrict__ sh_v, int n_rest, const float* __restrict__ camera, float near_z,
     float blur, const float* __restrict__ gslot, const int32_t* __restrict__ inv,
     float* __restrict__ gparams, float* __restrict__ m, float* __restrict__ v,
     const float* __restrict__ lr, const float* __restrict__ lr_sh,
     const int32_t* __restrict__ step, float b1, float b2, float eps, McmcArgs mc, DepthW dwa) {
-  __shared__ float s_p[kGeoBlock * 15], s_m[kGeoBlock * 15], s_v[kGeoBlock * 15];
-  __shared__ int s_inv[kGeoBlock * 9];
-  const int g0 = blockIdx.x * kGeoBlock, rows = min(kGeoBlock, G - g0);
+  __shared__ float s_p[kAdamBlock * 15], s_m[kAdamBlock * 15], s_v[kAdamBlock * 15];
+  __shared__ int s_inv[kAdamBlock * 9];
+  const int g0 = blockIdx.x * kAdamBlock, rows = min(kAdamBlock, G - g0);
   const int g = g0 + threadIdx.x;
   {  // all four row copies in flight at once
     int ri[9];
     float rp[14], rm[14], rv[14];
-    stage_load<9>(inv, g0, rows, ri);
-    stage_load<14>(params, g0, rows, rp);
-    stage_load<14>(m, g0, rows, rm);
-    stage_load<14>(v, g0, rows, rv);
-    stage_put<9, 9>(ri, rows, s_inv);
-    stage_put<14, 15>(rp, rows, s_p);
-    stage_put<14, 15>(rm, rows, s_m);
-    stage_put<14, 15>(rv, rows, s_v);
+    stage_load<9, kAdamBlock>(inv, g0, rows, ri);
+    stage_load<14, kAdamBlock>(params, g0, rows, rp);
+    stage_load<14, kAdamBlock>(m, g0, rows, rm);
+    stage_load<14, kAdamBlock>(v, g0, rows, rv);
+    stage_put<9, 9, kAdamBlock>(ri, rows, s_inv);
+    stage_put<14, 15, kAdamBlock>(rp, rows, s_p);
+    stage_put<14, 15, kAdamBlock>(rm, rows, s_m);
+    stage_put<14, 15, kAdamBlock>(rv, rows, s_v);
   }
   __syncthreads();
   if ((int)threadIdx.x < rows)
     bwd_adam_row<SH, MC>(threadIdx.x, g, G, s_p, s_m, s_v, s_inv, rest, sh_m, sh_v, n_rest, camera,
                          near_z, blur, gslot, gparams, lr, lr_sh, step, b1, b2, eps, mc, dwa);
   __syncthreads();
-  stage_out<14, 15>(params, g0, rows, s_p);
-  stage_out<14, 15>(m, g0, rows, s_m);
-  stage_out<14, 15>(v, g0, rows, s_v);
+  stage_out<14, 15, kAdamBlock>(params, g0, rows, s_p);
+  stage_out<14, 15, kAdamBlock>(m, g0, rows, s_m);
+  stage_out<14, 15, kAdamBlock>(v, g0, rows, s_v);
 }
 
 // The seam between two training steps in one launch: step i's geometry backward + Adam
@@ -1476,7 +1482,7 @@ int tts_geom_bwd_adam(float* params, int G, const float* camera, float near_z, f
     return TTS_EINVAL;
   if (G >= (1 << 30)) return TTS_EG;
   if (G == 0) return TTS_OK;
-  k_geom_bwd_adam<false, false><<<grid1d(G, 256), 256, 0, stream>>>(
+  k_geom_bwd_adam<false, false><<<grid1d(G, kAdamBlock), kAdamBlock, 0, stream>>>(
       params, G, nullptr, nullptr, nullptr, 0, camera, near_z, blur, gslot, inv, gparams, m, v,
       lr, nullptr, step, beta1, beta2, eps, McmcArgs{0.0f, 0.0f, 0.0f, 0u},
       DepthW{nullptr, nullptr, 1.0f, 0, 0});
@@ -1501,9 +1507,9 @@ int tts_geom_bwd_adam_ex(float* params, float* sh_rest, float* sh_m, float* sh_v
   const DepthW dwa{depth_bt, gdepth, 1.0f, 0, 0};
   const bool use_mc = lambda_o > 0.0f || lambda_s > 0.0f || noise_lr > 0.0f;
   const int n_rest = sh_rest_count(sh_degree);
-  const dim3 grid = grid1d(G, 256);
+  const dim3 grid = grid1d(G, kAdamBlock);
 #define TTS_LAUNCH_BWD_ADAM(SH, MC)                                                          \
-  k_geom_bwd_adam<SH, MC><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_m, sh_v, n_rest,   \
+  k_geom_bwd_adam<SH, MC><<<grid, kAdamBlock, 0, stream>>>(params, G, sh_rest, sh_m, sh_v, n_rest,   \
                                                     camera, near_z, blur, gslot, inv, gparams, \
                                                     m, v, lr, lr_sh, step, beta1, beta2, eps,  \
                                                     mc, dwa)
