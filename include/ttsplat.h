@@ -428,6 +428,14 @@ int tts_geom_bwd_ex(const float* params, const float* sh_rest, int sh_degree,
                     float near_z, float blur, const float* grad9, float* gparams,
                     float* gsh_rest, float* gdepth, hipStream_t stream);
 
+/* The last view of a batch and the batch's Adam update in one launch: Adam takes the gradient
+ * gacc + scale * dL/dparams of this view, and gacc is left at zero.  The same results as
+ * tts_geom_bwd_accum, tts_adam and tts_zero(gacc); the step block must have been advanced. */
+int tts_geom_bwd_adam_acc(float* params, int G, const float* camera, float near_z, float blur,
+                          const float* gslot, const int32_t* inv, float* gacc, float scale,
+                          float* m, float* v, const float* lr, const int32_t* step, float beta1,
+                          float beta2, float eps, hipStream_t stream);
+
 /* tts_geom_bwd_adam with the optional extensions of the device step, in one kernel:
  *  - SH colour (sh_degree > 0): the rest coefficients and their Adam moments sh_m, sh_v (rest
  *    layout) take the same Adam step with learning rate lr_sh[0] (device scalar; the reference

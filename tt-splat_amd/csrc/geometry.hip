@@ -863,20 +863,25 @@ struct McmcArgs {
 // stride 15, s_inv at stride 9), gaussian g.  The slot gradients are gathered through the
 // row's inverse-table entries, the forward recomputed, the chain rule applied (plus the MCMC
 // regulariser), and the new parameters and moments written back over the row.
-template <bool SH, bool MC>
+template <bool SH, bool MC, bool ACC = false>
 __device__ __forceinline__ void bwd_adam_row(
     int t, int g, int G, float* s_p, float* s_m, float* s_v, const int* s_inv,
     float* __restrict__ rest, float* __restrict__ sh_m, float* __restrict__ sh_v, int n_rest,
     const float* __restrict__ camera, float near_z, float blur, const float* __restrict__ gslot,
     float* __restrict__ gparams, const float* __restrict__ lr, const float* __restrict__ lr_sh,
     const int32_t* __restrict__ step, float b1, float b2, float eps, const McmcArgs& mc,
-    const DepthW& dwa) {
+    const DepthW& dwa, float* __restrict__ gacc = nullptr, float scale = 1.0f) {
   int e[9];
 #pragma unroll
   for (int j = 0; j < 9; ++j) e[j] = s_inv[t * 9 + j];
   float gin[9], gout[14], gcol[3];
   SlotRecs recs;
   slot_loads(gslot, e, recs);  // in flight during the forward recompute below
+  float ga[ACC ? 14 : 1];
+  if (ACC) {
+#pragma unroll
+    for (int i = 0; i < 14; ++i) ga[i] = gacc[(int64_t)g * 14 + i];
+  }
   float pl[14], mm[14], vv[14];
 #pragma unroll
   for (int i = 0; i < 14; ++i) {
@@ -897,6 +902,13 @@ __device__ __forceinline__ void bwd_adam_row(
   float gdw[2];
   slot_sum(e, recs, gin);
   geo_backward(pl, cam, s, gin, gout, gcol, gdw, dwa.zgrad != 0);
+  if (ACC) {   // the batch's mean gradient: the earlier views' sum and this one's share
+#pragma unroll
+    for (int i = 0; i < 14; ++i) {
+      gout[i] = ga[i] + scale * gout[i];
+      gacc[(int64_t)g * 14 + i] = 0.0f;
+    }
+  }
   depthw_store(dwa, g, gdw);
   if (MC) reg_add(pl, mc.reg_o, mc.reg_s, gout);
   const float* f = reinterpret_cast<const float*>(step);
@@ -941,14 +953,19 @@ __device__ __forceinline__ void bwd_adam_row(
 // 128x128 67.1 / 66.5 / 65.6; G 60000, SH 2 113.0 / 112.5 / 111.6; G 100000, SH 3 + MCMC 175.7 /
 // 172.6 / 173.6.
 constexpr int kAdamBlock = 64;
-template <bool SH, bool MC>
+// ACC: the last view of a batch -- gacc, the earlier views' accumulated gradient, plus scale times
+// this view's is what Adam takes, and gacc is left at zero for the next batch.  In place of three
+// launches that write, read and clear the sum (k_geom_bwd_accum, k_adam, k_zero: 58 + 59 + 15 us at
+// G = 1M).
+template <bool SH, bool MC, bool ACC = false>
 __global__ __launch_bounds__(kAdamBlock) void k_geom_bwd_adam(
     float* __restrict__ params, int G, float* __restrict__ rest, float* __restrict__ sh_m,
     float* __restrict__ sh_v, int n_rest, const float* __restrict__ camera, float near_z,
     float blur, const float* __restrict__ gslot, const int32_t* __restrict__ inv,
     float* __restrict__ gparams, float* __restrict__ m, float* __restrict__ v,
     const float* __restrict__ lr, const float* __restrict__ lr_sh,
-    const int32_t* __restrict__ step, float b1, float b2, float eps, McmcArgs mc, DepthW dwa) {
+    const int32_t* __restrict__ step, float b1, float b2, float eps, McmcArgs mc, DepthW dwa,
+    float* __restrict__ gacc = nullptr, float scale = 1.0f) {
   __shared__ float s_p[kAdamBlock * 15], s_m[kAdamBlock * 15], s_v[kAdamBlock * 15];
   __shared__ int s_inv[kAdamBlock * 9];
   const int g0 = blockIdx.x * kAdamBlock, rows = min(kAdamBlock, G - g0);
@@ -967,8 +984,8 @@ __global__ __launch_bounds__(kAdamBlock) void k_geom_bwd_adam(
   }
   __syncthreads();
   if ((int)threadIdx.x < rows)
-    bwd_adam_row<SH, MC>(threadIdx.x, g, G, s_p, s_m, s_v, s_inv, rest, sh_m, sh_v, n_rest, camera,
-                         near_z, blur, gslot, gparams, lr, lr_sh, step, b1, b2, eps, mc, dwa);
+    bwd_adam_row<SH, MC, ACC>(threadIdx.x, g, G, s_p, s_m, s_v, s_inv, rest, sh_m, sh_v, n_rest, camera,
+                         near_z, blur, gslot, gparams, lr, lr_sh, step, b1, b2, eps, mc, dwa, gacc, scale);
   __syncthreads();
   stage_out<14, 15, kAdamBlock>(params, g0, rows, s_p);
   stage_out<14, 15, kAdamBlock>(m, g0, rows, s_m);
@@ -1471,6 +1488,23 @@ int tts_geom_bwd_accum_ex(const float* params, const float* sh_rest, int sh_degr
   else
     k_geom_bwd_accum<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z,
                                                       blur, gslot, inv, scale, gacc, nullptr);
+  return launch_status();
+}
+
+// The last view of a batch and its Adam update in one launch.
+int tts_geom_bwd_adam_acc(float* params, int G, const float* camera, float near_z, float blur,
+                          const float* gslot, const int32_t* inv, float* gacc, float scale,
+                          float* m, float* v, const float* lr, const int32_t* step, float beta1,
+                          float beta2, float eps, hipStream_t stream) {
+  if (G < 0 ||
+      (G > 0 && (!params || !camera || !gslot || !inv || !gacc || !m || !v || !lr || !step)))
+    return TTS_EINVAL;
+  if (G >= (1 << 30)) return TTS_EG;
+  if (G == 0) return TTS_OK;
+  k_geom_bwd_adam<false, false, true><<<grid1d(G, kAdamBlock), kAdamBlock, 0, stream>>>(
+      params, G, nullptr, nullptr, nullptr, 0, camera, near_z, blur, gslot, inv, nullptr, m, v, lr,
+      nullptr, step, beta1, beta2, eps, McmcArgs{0.0f, 0.0f, 0.0f, 0u},
+      DepthW{nullptr, nullptr, 1.0f, 0, 0}, gacc, scale);
   return launch_status();
 }
 

@@ -95,6 +95,9 @@ SIGNATURES = {
                                       _vp]),
     "tts_geom_bwd_accum_ex": (_c_int, [_vp, _vp, _c_int, _vp, _c_int, _vp, _c_float, _c_float, _vp,
                                        _vp, _c_float, _vp, _vp, _vp, _vp]),
+    "tts_geom_bwd_adam_acc": (_c_int, [_vp, _c_int, _vp, _c_float, _c_float, _vp, _vp, _vp,
+                                       _c_float, _vp, _vp, _vp, _vp, _c_float, _c_float, _c_float,
+                                       _vp]),
     "tts_depth_weight_workspace_bytes": (_c_size, [_c_int]),
     "tts_depth_weight_adam": (_c_int, [_vp, _c_int, _vp, _vp, _vp, _vp, _c_float, _c_float,
                                        _c_float, _vp, _c_size, _vp]),

@@ -718,6 +718,24 @@ def geom_bwd_accum(params, camera, gslot, inv, gacc, scale=1.0, near=NEAR, blur=
     return gacc
 
 
+def geom_bwd_adam_acc(params, camera, gslot, inv, gacc, scale, m, v, lr, step, near=NEAR,
+                      blur=BLUR, b1=BETA1, b2=BETA2, eps=EPS):
+    """The last view of a batch: Adam on gacc + scale * dL/dparams of this view (gacc as the
+    earlier views' geom_bwd_accum left it; zero afterwards)."""
+    G = params.shape[0]
+    dev = params.device
+    require(params, "params", F32, (G, 14))
+    require(camera, "camera", F32, (16,), dev)
+    require(gslot, "gslot", F32, None, dev)
+    require(inv, "inv", I32, (G, 9), dev)
+    for t, n in ((gacc, "gacc"), (m, "m"), (v, "v")):
+        require(t, n, F32, (G, 14), dev)
+    require(lr, "lr", F32, (14,), dev)
+    require(step, "step", I32, (4,), dev)
+    call("tts_geom_bwd_adam_acc", ptr(params), G, ptr(camera), near, blur, ptr(gslot), ptr(inv),
+         ptr(gacc), float(scale), ptr(m), ptr(v), ptr(lr), ptr(step), b1, b2, eps, stream())
+
+
 def geom_bwd_adam(params, camera, gslot, inv, m, v, lr, step, near=NEAR, blur=BLUR, gparams=None,
                   b1=BETA1, b2=BETA2, eps=EPS, sh_rest=None, sh_m=None, sh_v=None, lr_sh=None,
                   sh_degree=0, lambda_o=0.0, lambda_s=0.0, noise_lr=0.0, seed=0, depth_bt=None,

@@ -331,12 +331,21 @@ class TrainStep:
             self._geometry_backward_adam(i)
             return
         scale = 1.0 / self.batch
-        for ci in range(i * self.batch, (i + 1) * self.batch):
-            self._view_backward(ci)
+        # the plain step's last view goes to Adam with the others' sum, in one launch
+        plain = (self.sh_degree == 0 and self.dw is None
+                 and not (mc["lambda_o"] or mc["lambda_s"] or mc["noise_lr"]))
+        last = (i + 1) * self.batch - 1
+        for ci in range(i * self.batch, last + 1):
+            # the step advance rides on the last view's geometry launch (after its background's
+            # draw, keyed by the completed steps)
+            self._view_backward(ci, advance=ci == last)
+            if plain and ci == last:
+                kernels.geom_bwd_adam_acc(self.P, self.cams[ci], self.gslot, self.inv, self.gacc,
+                                          scale, self.m, self.v, self.lr, self.step_block)
+                return
             kernels.geom_bwd_accum(self.P, self.cams[ci], self.gslot, self.inv, self.gacc, scale,
                                    gacc_sh=self.gacc_sh, depth_bt=self.dw, gacc_depth=self.gdw,
                                    **sh)
-        kernels.adam_advance(self.step_block)
         if mc["lambda_o"] or mc["lambda_s"]:
             kernels.mcmc_reg_grad(self.P, self.gacc, mc["lambda_o"], mc["lambda_s"])
         kernels.adam(self.P, self.m, self.v, self.gacc, self.lr, self.step_block)
