@@ -387,6 +387,31 @@ int tts_geom_fwd_assign_bins(const float* params, const float* sh_rest, int sh_d
                              int32_t* pos_count, void* workspace, size_t workspace_bytes,
                              hipStream_t stream);
 
+/* tts_geom_fwd_ex and tts_geom_fwd_assign_bins that also write the background block tts_background
+ * makes (bg, from w_b_raw and c_b; NULL: not), and tts_geom_bwd_ex that also makes
+ * tts_background_grad's gradient (gw_b_raw; NULL: not) and takes the projected gradients either as
+ * rows grad_stride >= 9 floats apart (inv NULL) or as slot gradients [T,K,9] through the inverse
+ * table inv (tts_slot_reduce's sum; no SH, no depth weight): one launch each. */
+int tts_geom_fwd_bg(const float* params, const float* sh_rest, int sh_degree,
+                    const float* depth_bt, int G, const float* camera, float near_z, float blur,
+                    float* proj, uint8_t* keep, int32_t* step_adv, float beta1, float beta2,
+                    const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream);
+int tts_geom_fwd_assign_bins_bg(const float* params, const float* sh_rest, int sh_degree,
+                                const float* depth_bt, int G, const float* camera, float near_z,
+                                float blur, float* proj, uint8_t* keep, int32_t* step_adv,
+                                float beta1, float beta2, int H, int W, int S, int R, int K,
+                                int span, int32_t* idx, uint8_t* valid, int32_t* count,
+                                int32_t* ncand, int32_t* inv, int32_t* order, float* slot_rec,
+                                int32_t* pos_count, void* workspace, size_t workspace_bytes,
+                                const float* w_b_raw, const float* c_b, float* bg,
+                                hipStream_t stream);
+int tts_geom_bwd_render(const float* params, const float* sh_rest, int sh_degree,
+                        const float* depth_bt, int depth_zgrad, int G, const float* camera,
+                        float near_z, float blur, const float* grad, int grad_stride,
+                        const int32_t* inv, float* gparams, float* gsh_rest, float* gdepth,
+                        const float* gwb, int n_gwb, const float* w_b_raw, float* gw_b_raw,
+                        hipStream_t stream);
+
 /* The seam between two training steps in one launch: tts_geom_bwd_adam of step i (camera_bwd,
  * its slot gradients gslot through inv; gparams may be NULL) followed by the geometry forward
  * of step i+1 (camera_fwd, into proj and keep) and the count pass of its binning into the

@@ -82,3 +82,32 @@ def test_loss_fn_value_and_gradient_scale():
     (g1,) = torch.autograd.grad(loss, x, retain_graph=True)
     (g2,) = torch.autograd.grad(loss * 3.0, x)
     assert torch.allclose(3.0 * g1, g2, rtol=1e-6)
+
+
+@pytest.mark.parametrize("G", [0, 1, 255, 256, 257, 1000])
+def test_geometry_launches_carry_the_background(G):
+    """geom_fwd writes the block background() makes; geom_bwd writes background_grad's result, takes
+    rows of 10 and slot gradients through the inverse table."""
+    from helpers import config_inputs
+    _, P, cam = config_inputs("c1_ref", G=max(G, 1))
+    P, camb = P[:G].cuda(), cam.device_block("cuda")
+    w, c = torch.tensor(-1.5).cuda(), torch.tensor([0.2, 0.4, 0.9]).cuda()
+    bg = torch.full((4,), -1.0, device="cuda")
+    proj, keep = kernels.geom_fwd(P, camb, background=(w, c, bg))
+    assert torch.equal(bg, kernels.background(w, c))
+    if G == 0:
+        return
+    assert torch.equal(proj, kernels.geom_fwd(P, camb)[0])
+    g = torch.Generator().manual_seed(G)
+    gwb = torch.randn(77, generator=g).cuda()
+    g10 = torch.randn(G, 10, generator=g).cuda()
+    want = kernels.geom_bwd(P, camb, g10[:, :9].contiguous())
+    gw = torch.empty_like(w)
+    assert torch.equal(kernels.geom_bwd(P, camb, g10, background=(gwb, w, gw)), want)
+    assert torch.equal(gw, kernels.background_grad(gwb, w))
+    gslot = torch.randn(8, 16, 9, generator=g).cuda()
+    inv = torch.randint(-1, 128, (G, 9), generator=g, dtype=torch.int32).cuda()
+    ref = kernels.geom_bwd(P, camb, kernels.slot_reduce(gslot, inv))
+    got = kernels.geom_bwd(P, camb, gslot, inv=inv)
+    # the same sum and formulas, contracted by the compiler per kernel
+    assert torch.allclose(got, ref, rtol=1e-4, atol=1e-5 * float(ref.abs().max()))

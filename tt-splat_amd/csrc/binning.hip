@@ -114,12 +114,14 @@ __global__ __launch_bounds__(1024) void k_bin_colscan(int* __restrict__ mat, int
                                                       int* __restrict__ within,
                                                       int* __restrict__ chunk_tot,
                                                       int* __restrict__ cls_ctr, int n_ctr,
-                                                      int32_t* adv, float b1, float b2) {
+                                                      int32_t* adv, float b1, float b2,
+                                                      BgArgs bga) {
   __shared__ int s_seg[16][kChunk];
   // the scatter pass's list counters start from zero
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < n_ctr; i += 1024) cls_ctr[i] = 0;
   if (adv && blockIdx.x == 0 && threadIdx.x == 0) advance_step(adv, b1, b2);
+  if (bga.out && blockIdx.x == 0) write_background(bga);
   const int col = threadIdx.x & (kChunk - 1), seg = threadIdx.x >> 6;
   const int x = blockIdx.x * kChunk + col;
   const int rows = (nblk + 15) / 16;
@@ -1287,7 +1289,7 @@ static int bin_run(const float* mu2d, int mu_stride, const uint8_t* keep, int ke
                    int32_t* count, int32_t* ncand, int32_t* inv, int32_t* order,
                    const float* proj, float* rec, int32_t* pos_count, const BinWorkspace& ws,
                    bool counted, hipStream_t stream, int32_t* adv = nullptr, float b1 = 0.f,
-                   float b2 = 0.f, int64_t* idx64 = nullptr) {
+                   float b2 = 0.f, int64_t* idx64 = nullptr, BgArgs bga = BgArgs{}) {
   const int ntx = W / S, nty = H / S, T = ntx * nty;
   const float Sf = static_cast<float>(S);
   const int NB = ws.NB, Tpad = ws.Tpad, nblk = ws.nblk;
@@ -1314,7 +1316,7 @@ static int bin_run(const float* mu2d, int mu_stride, const uint8_t* keep, int ke
   }
   k_bin_colscan<<<(X + kChunk - 1) / kChunk, 1024, 0, stream>>>(ws.mat, nblk, X, ws.tot,
                                                                 ws.within, ws.chunk_tot,
-                                                                ws.nlist, 2, adv, b1, b2);
+                                                                ws.nlist, 2, adv, b1, b2, bga);
   const int ncls = (T + 1023) / 1024;
   ScatterArgs sc{mu2d, mu_stride, G, ntx, nty, NB, Tpad, K, ws.cblock, ncls, ws.cell_slot,
                  ws.mat, ws.tot, ws.within, ws.chunk_tot, ws.cell_start, ws.far_start, ws.recs,
@@ -1432,15 +1434,18 @@ int tts_tile_order(const int32_t* count, int T, int K, int32_t* order, hipStream
 // Geometry forward + binning of one view (tts_geom_fwd_ex, then tts_assign_bins on proj's
 // means and keep): with count blocks of 512 gaussians (G <= 131072) the count pass runs inside
 // the geometry launch (k_geom_fwd_count), otherwise the two run as their own launches.  With
-// slot_rec the select pass also writes the slot records and per-position counts.
-int tts_geom_fwd_assign_bins(const float* params, const float* sh_rest, int sh_degree,
-                             const float* depth_bt, int G, const float* camera, float near_z,
-                             float blur, float* proj, uint8_t* keep, int32_t* step_adv,
-                             float beta1, float beta2, int H, int W, int S, int R, int K,
-                             int span, int32_t* idx, uint8_t* valid, int32_t* count,
-                             int32_t* ncand, int32_t* inv, int32_t* order, float* slot_rec,
-                             int32_t* pos_count, void* workspace, size_t workspace_bytes,
-                             hipStream_t stream) {
+// slot_rec the select pass also writes the slot records and per-position counts; with bg the
+// column scan writes the render's background block.
+int tts_geom_fwd_assign_bins_bg(const float* params, const float* sh_rest, int sh_degree,
+                                const float* depth_bt, int G, const float* camera, float near_z,
+                                float blur, float* proj, uint8_t* keep, int32_t* step_adv,
+                                float beta1, float beta2, int H, int W, int S, int R, int K,
+                                int span, int32_t* idx, uint8_t* valid, int32_t* count,
+                                int32_t* ncand, int32_t* inv, int32_t* order, float* slot_rec,
+                                int32_t* pos_count, void* workspace, size_t workspace_bytes,
+                                const float* w_b_raw, const float* c_b, float* bg,
+                                hipStream_t stream) {
+  if (bg && (!w_b_raw || !c_b)) return TTS_EINVAL;
   if (G < 0 || (G > 0 && (!params || !camera || !proj || !keep))) return TTS_EINVAL;
   if (slot_rec && (!pos_count || !order)) return TTS_EINVAL;
   if (sh_degree < 0 || sh_degree > 3 || (sh_degree > 0 && !sh_rest)) return TTS_ESH;
@@ -1455,23 +1460,39 @@ int tts_geom_fwd_assign_bins(const float* params, const float* sh_rest, int sh_d
   // the count pass inside the geometry launch: blocks of 512 (small) or 4096 (large) gaussians
   const bool small = ws.cblock == CountSmall::kBlock;
   const bool fused = G > 0 && (small ? geom_fwd_count_lds(ws.NB, ws.Tpad)
-                                     : geom_fwd_count_large_lds(ws.NB, ws.Tpad)) <= kMaxLdsBytes;
+                                        : geom_fwd_count_large_lds(ws.NB, ws.Tpad)) <= kMaxLdsBytes;
   const float Sf = static_cast<float>(S);
   int e;
   if (fused && small)
     e = launch_geom_fwd_count(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur, proj,
-                              keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB, ws.Tpad,
-                              ws.mat, ws.cell_slot, stream);
+                                 keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB, ws.Tpad,
+                                 ws.mat, ws.cell_slot, stream);
   else if (fused)
     e = launch_geom_fwd_count_large(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur,
-                                    proj, keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB,
-                                    ws.Tpad, ws.mat, ws.cell_slot, stream);
+                                       proj, keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB,
+                                       ws.Tpad, ws.mat, ws.cell_slot, stream);
   else
     e = tts_geom_fwd_ex(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur, proj, keep,
                         step_adv, beta1, beta2, stream);
   if (e != TTS_OK) return e;
   return bin_run(proj, 12, keep, 1, G, H, W, S, K, span, idx, valid, count, ncand, inv, order,
-                 proj, slot_rec, pos_count, ws, fused, stream);
+                 proj, slot_rec, pos_count, ws, fused, stream, nullptr, 0.f, 0.f, nullptr,
+                 BgArgs{w_b_raw, c_b, bg});
+}
+
+int tts_geom_fwd_assign_bins(const float* params, const float* sh_rest, int sh_degree,
+                             const float* depth_bt, int G, const float* camera, float near_z,
+                             float blur, float* proj, uint8_t* keep, int32_t* step_adv,
+                             float beta1, float beta2, int H, int W, int S, int R, int K,
+                             int span, int32_t* idx, uint8_t* valid, int32_t* count,
+                             int32_t* ncand, int32_t* inv, int32_t* order, float* slot_rec,
+                             int32_t* pos_count, void* workspace, size_t workspace_bytes,
+                             hipStream_t stream) {
+  return tts_geom_fwd_assign_bins_bg(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur,
+                                     proj, keep, step_adv, beta1, beta2, H, W, S, R, K, span, idx,
+                                     valid, count, ncand, inv, order, slot_rec, pos_count,
+                                     workspace, workspace_bytes, nullptr, nullptr, nullptr,
+                                     stream);
 }
 
 // The seam between two training steps (k_geom_bwd_adam_fwd_count): tts_geom_bwd_adam for

@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void k_geom_fwd(const float* __restrict__ para
                                                   const float* __restrict__ camera, float near_z,
                                                   float blur, float* __restrict__ proj,
                                                   uint8_t* __restrict__ keep, int32_t* adv,
-                                                  float b1, float b2) {
+                                                  float b1, float b2, BgArgs bga) {
   __shared__ float s_p[kGeoBlock * 15];
   __shared__ float s_o[kGeoBlock * 13];
   const int g0 = blockIdx.x * kGeoBlock, rows = min(kGeoBlock, G - g0);
@@ -561,6 +561,7 @@ __global__ __launch_bounds__(256) void k_geom_fwd(const float* __restrict__ para
   __syncthreads();
   stage_out<12, 13>(proj, g0, rows, s_o);
   if (adv && blockIdx.x == 0 && threadIdx.x == 0) advance_step(adv, b1, b2);
+  if (bga.out && blockIdx.x == 0) write_background(bga);
 }
 
 // The geometry forward of 512 gaussians, one per thread (two 256-row halves staged by the two
@@ -729,15 +730,74 @@ __global__ __launch_bounds__(1024) void k_geom_fwd_count_large(
                         reinterpret_cast<int*>(s_dyn), mat, cell_slot);
 }
 
+// Sum of one gaussian's slot gradients, gathered through the inverse bin table inv[g][0..9)
+// (tile*K + slot, or -1) in stencil order: the slot->gaussian reduce of
+// tools/m9_scatter_oracle.py:35-42 / tools/resident_traced.py:383-395, without atomics and in a
+// fixed order (so the result is reproducible bit for bit).
+// Per-gaussian sum of its slot gradients, in stencil order j (a fixed order: deterministic).
+// Every load is issued before any is used (missing slots read row 0 and are masked), so the
+// gather costs one dependent round trip after the inverse-table load.
+__device__ __forceinline__ void gather_slot_grads(const float* __restrict__ gslot,
+                                                  const int32_t* __restrict__ inv, int g,
+                                                  float* gin) {
+  int e[9];
+#pragma unroll
+  for (int j = 0; j < 9; ++j) e[j] = inv[(int64_t)g * 9 + j];
+  float v[9][9];
+#pragma unroll
+  for (int j = 0; j < 9; ++j) {
+    const float* src = gslot + (int64_t)(e[j] >= 0 ? e[j] : 0) * 9;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) v[j][c] = src[c];
+  }
+#pragma unroll
+  for (int c = 0; c < 9; ++c) gin[c] = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 9; ++j)
+#pragma unroll
+    for (int c = 0; c < 9; ++c) gin[c] += e[j] >= 0 ? v[j][c] : 0.0f;
+}
+
+// dL/dw_b_raw from n partial sums of dL/dw_b (one block's work, summed in 64 bits in a fixed order).
+struct BgGrad {
+  const float* gwb;
+  int n;
+  const float* raw;
+  float* graw;
+};
+__device__ __forceinline__ void background_grad(const BgGrad& a) {
+  __shared__ double s_sum[4];
+  double v = 0.0;
+  for (int i = threadIdx.x; i < a.n; i += 256) v += (double)a.gwb[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const float g = (float)((s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3])), x = a.raw[0];
+    const float z = expf(x);
+    a.graw[0] = x > 20.0f ? g : g * z / (z + 1.0f);
+  }
+}
+
+// Gradient of one gaussian's nine projected quantities (grad, rows `stride` floats apart; GATHER:
+// summed here from the slot gradients through the inverse table, as k_slot_reduce) to its
+// parameters.  With bgg.graw the last block, past the gaussians', makes the background's gradient:
+// a render's backward then needs no launches of its own for either.
 // gsh (SH only): dL/drest in the rest layout; rows l >= n_rest are written as zero.
-template <bool SH>
+template <bool SH, bool GATHER = false>
 __global__ __launch_bounds__(256) void k_geom_bwd(const float* __restrict__ params, int G,
                                                   const float* __restrict__ rest, int n_rest,
                                                   DepthW dwa, const float* __restrict__ camera,
                                                   float near_z, float blur,
-                                                  const float* __restrict__ grad9,
+                                                  const float* __restrict__ grad, int stride,
+                                                  const int32_t* __restrict__ inv,
                                                   float* __restrict__ gparams,
-                                                  float* __restrict__ gsh) {
+                                                  float* __restrict__ gsh, BgGrad bgg) {
+  if (bgg.graw && blockIdx.x == gridDim.x - 1) {
+    background_grad(bgg);
+    return;
+  }
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= G) return;
   const Camera cam = load_camera(camera);
@@ -752,8 +812,12 @@ __global__ __launch_bounds__(256) void k_geom_bwd(const float* __restrict__ para
     sh_apply(p, b, rv, n_rest, s);
   }
   float gin[9], gout[14], gcol[3], gdw[2];
+  if (GATHER) {
+    gather_slot_grads(grad, inv, g, gin);
+  } else {
 #pragma unroll
-  for (int i = 0; i < 9; ++i) gin[i] = grad9[(int64_t)g * 9 + i];
+    for (int i = 0; i < 9; ++i) gin[i] = grad[(int64_t)g * stride + i];
+  }
   geo_backward(p, cam, s, gin, gout, gcol, gdw, (dwa.zgrad & TTS_GRAD_DEPTH_Z) != 0);
   if (SH && (dwa.zgrad & TTS_GRAD_SH_DIR)) sh_dir_grad(p, cam, rv, n_rest, gcol, gout);
 #pragma unroll
@@ -797,34 +861,6 @@ __global__ __launch_bounds__(256) void k_adam(float* __restrict__ params, float*
   params[i] = pp;
   m[i] = mm;
   v[i] = vv;
-}
-
-// Sum of one gaussian's slot gradients, gathered through the inverse bin table inv[g][0..9)
-// (tile*K + slot, or -1) in stencil order: the slot->gaussian reduce of
-// tools/m9_scatter_oracle.py:35-42 / tools/resident_traced.py:383-395, without atomics and in a
-// fixed order (so the result is reproducible bit for bit).
-// Per-gaussian sum of its slot gradients, in stencil order j (a fixed order: deterministic).
-// Every load is issued before any is used (missing slots read row 0 and are masked), so the
-// gather costs one dependent round trip after the inverse-table load.
-__device__ __forceinline__ void gather_slot_grads(const float* __restrict__ gslot,
-                                                  const int32_t* __restrict__ inv, int g,
-                                                  float* gin) {
-  int e[9];
-#pragma unroll
-  for (int j = 0; j < 9; ++j) e[j] = inv[(int64_t)g * 9 + j];
-  float v[9][9];
-#pragma unroll
-  for (int j = 0; j < 9; ++j) {
-    const float* src = gslot + (int64_t)(e[j] >= 0 ? e[j] : 0) * 9;
-#pragma unroll
-    for (int c = 0; c < 9; ++c) v[j][c] = src[c];
-  }
-#pragma unroll
-  for (int c = 0; c < 9; ++c) gin[c] = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 9; ++j)
-#pragma unroll
-    for (int c = 0; c < 9; ++c) gin[c] += e[j] >= 0 ? v[j][c] : 0.0f;
 }
 
 __global__ __launch_bounds__(256) void k_slot_reduce(const float* __restrict__ gslot,
@@ -1303,37 +1339,11 @@ int launch_geom_seam(float* params, int G, const float* cam_b, const float* cam_
   return launch_status();
 }
 
-// The blend's background block [w_b, c_b], w_b = softplus(w_b_raw) (spike/render.py:28), and the
-// gradient back to w_b_raw from per-tile partial sums of dL/dw_b (summed in 64 bits, a fixed
-// order).  Latency-bound launches of one wave, in place of two (forward) and eight (backward)
-// tensor operations on four floats.
-__global__ __launch_bounds__(64) void k_background(const float* __restrict__ raw,
-                                                   const float* __restrict__ c_b,
-                                                   float* __restrict__ bg) {
-  if (threadIdx.x == 0) {
-    const float x = raw[0];
-    bg[0] = x > 20.0f ? x : log1pf(expf(x));
-  } else if (threadIdx.x < 4) {
-    bg[threadIdx.x] = c_b[threadIdx.x - 1];
-  }
-}
+// The background block alone (a launch of one wave; the renders write it inside the geometry or
+// binning launch).
+__global__ __launch_bounds__(64) void k_background(BgArgs a) { write_background(a); }
 
-__global__ __launch_bounds__(256) void k_background_grad(const float* __restrict__ gwb, int n,
-                                                         const float* __restrict__ raw,
-                                                         float* __restrict__ graw) {
-  __shared__ double s_sum[4];
-  double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) v += (double)gwb[i];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const float g = (float)((s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3])), x = raw[0];
-    const float z = expf(x);
-    graw[0] = x > 20.0f ? g : g * z / (z + 1.0f);
-  }
-}
+__global__ __launch_bounds__(256) void k_background_grad(BgGrad a) { background_grad(a); }
 
 }  // namespace tts
 
@@ -1366,7 +1376,7 @@ int tts_geom_fwd(const float* params, int G, const float* camera, float near_z, 
   if (G == 0) return TTS_OK;
   k_geom_fwd<false><<<grid1d(G, 256), 256, 0, stream>>>(params, G, nullptr, 0, nullptr, camera,
                                                         near_z, blur, proj, keep, nullptr, 0.f,
-                                                        0.f);
+                                                        0.f, BgArgs{});
   return launch_status();
 }
 
@@ -1377,26 +1387,37 @@ static int sh_args(int deg, const void* rest) {
   return TTS_OK;
 }
 
+int tts_geom_fwd_bg(const float* params, const float* sh_rest, int sh_degree,
+                    const float* depth_bt, int G, const float* camera, float near_z, float blur,
+                    float* proj, uint8_t* keep, int32_t* step_adv, float beta1, float beta2,
+                    const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream) {
+  if (G < 0 || (G > 0 && (!params || !camera || !proj || !keep))) return TTS_EINVAL;
+  if (bg && (!w_b_raw || !c_b)) return TTS_EINVAL;
+  if (const int e = sh_args(sh_degree, sh_rest)) return e;
+  if (G >= (1 << 30)) return TTS_EG;
+  if (G == 0) {  // no rows: the advance and the background alone
+    if (step_adv) k_adam_advance<<<1, 64, 0, stream>>>(step_adv, beta1, beta2);
+    if (bg) k_background<<<1, 64, 0, stream>>>(BgArgs{w_b_raw, c_b, bg});
+    return launch_status();
+  }
+  const dim3 grid = grid1d(G, 256);
+  const BgArgs bga{w_b_raw, c_b, bg};
+  if (sh_degree > 0)
+    k_geom_fwd<true><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_rest_count(sh_degree),
+                                               depth_bt, camera, near_z, blur, proj, keep,
+                                               step_adv, beta1, beta2, bga);
+  else
+    k_geom_fwd<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, depth_bt, camera, near_z,
+                                                blur, proj, keep, step_adv, beta1, beta2, bga);
+  return launch_status();
+}
+
 int tts_geom_fwd_ex(const float* params, const float* sh_rest, int sh_degree,
                     const float* depth_bt, int G, const float* camera, float near_z, float blur,
                     float* proj, uint8_t* keep, int32_t* step_adv, float beta1, float beta2,
                     hipStream_t stream) {
-  if (G < 0 || (G > 0 && (!params || !camera || !proj || !keep))) return TTS_EINVAL;
-  if (const int e = sh_args(sh_degree, sh_rest)) return e;
-  if (G >= (1 << 30)) return TTS_EG;
-  if (G == 0) {  // no rows: the advance alone
-    if (step_adv) k_adam_advance<<<1, 64, 0, stream>>>(step_adv, beta1, beta2);
-    return launch_status();
-  }
-  const dim3 grid = grid1d(G, 256);
-  if (sh_degree > 0)
-    k_geom_fwd<true><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_rest_count(sh_degree),
-                                               depth_bt, camera, near_z, blur, proj, keep,
-                                               step_adv, beta1, beta2);
-  else
-    k_geom_fwd<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, depth_bt, camera, near_z,
-                                                blur, proj, keep, step_adv, beta1, beta2);
-  return launch_status();
+  return tts_geom_fwd_bg(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur, proj, keep,
+                         step_adv, beta1, beta2, nullptr, nullptr, nullptr, stream);
 }
 
 int tts_geom_bwd(const float* params, int G, const float* camera, float near_z, float blur,
@@ -1406,8 +1427,41 @@ int tts_geom_bwd(const float* params, int G, const float* camera, float near_z, 
   if (G == 0) return TTS_OK;
   k_geom_bwd<false><<<grid1d(G, 256), 256, 0, stream>>>(params, G, nullptr, 0,
                                                         DepthW{nullptr, nullptr, 1.0f, 0, 0},
-                                                        camera, near_z, blur, grad9, gparams,
-                                                        nullptr);
+                                                        camera, near_z, blur, grad9, 9, nullptr,
+                                                        gparams, nullptr, BgGrad{});
+  return launch_status();
+}
+
+int tts_geom_bwd_render(const float* params, const float* sh_rest, int sh_degree,
+                        const float* depth_bt, int depth_zgrad, int G, const float* camera,
+                        float near_z, float blur, const float* grad, int grad_stride,
+                        const int32_t* inv, float* gparams, float* gsh_rest, float* gdepth,
+                        const float* gwb, int n_gwb, const float* w_b_raw, float* gw_b_raw,
+                        hipStream_t stream) {
+  if (G < 0 || (G > 0 && (!params || !camera || !grad || !gparams))) return TTS_EINVAL;
+  if (const int e = sh_args(sh_degree, sh_rest)) return e;
+  if (sh_degree > 0 && !gsh_rest) return TTS_EINVAL;
+  if (inv && (sh_degree > 0 || depth_bt)) return TTS_EINVAL;  // the binned render has neither
+  if (!inv && grad_stride < 9) return TTS_EINVAL;
+  if (gw_b_raw && (n_gwb < 0 || (n_gwb > 0 && !gwb) || !w_b_raw)) return TTS_EINVAL;
+  if (G >= (1 << 30)) return TTS_EG;
+  const BgGrad bgg{gwb, n_gwb, w_b_raw, gw_b_raw};
+  if (G == 0) {
+    if (gw_b_raw) k_background_grad<<<1, 256, 0, stream>>>(bgg);
+    return launch_status();
+  }
+  const DepthW dwa{depth_bt, gdepth, 1.0f, 0, depth_zgrad & (TTS_GRAD_DEPTH_Z | TTS_GRAD_SH_DIR)};
+  const dim3 grid = grid1d(G, 256) + (gw_b_raw ? 1 : 0);
+  if (sh_degree > 0)
+    k_geom_bwd<true><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_rest_count(sh_degree), dwa,
+                                               camera, near_z, blur, grad, grad_stride, nullptr,
+                                               gparams, gsh_rest, bgg);
+  else if (inv)
+    k_geom_bwd<false, true><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z,
+                                                      blur, grad, 9, inv, gparams, nullptr, bgg);
+  else
+    k_geom_bwd<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z, blur,
+                                                grad, grad_stride, nullptr, gparams, nullptr, bgg);
   return launch_status();
 }
 
@@ -1415,20 +1469,9 @@ int tts_geom_bwd_ex(const float* params, const float* sh_rest, int sh_degree,
                     const float* depth_bt, int depth_zgrad, int G, const float* camera,
                     float near_z, float blur, const float* grad9, float* gparams,
                     float* gsh_rest, float* gdepth, hipStream_t stream) {
-  if (G < 0 || (G > 0 && (!params || !camera || !grad9 || !gparams))) return TTS_EINVAL;
-  if (const int e = sh_args(sh_degree, sh_rest)) return e;
-  if (sh_degree > 0 && !gsh_rest) return TTS_EINVAL;
-  if (G >= (1 << 30)) return TTS_EG;
-  if (G == 0) return TTS_OK;
-  const DepthW dwa{depth_bt, gdepth, 1.0f, 0, depth_zgrad & (TTS_GRAD_DEPTH_Z | TTS_GRAD_SH_DIR)};
-  const dim3 grid = grid1d(G, 256);
-  if (sh_degree > 0)
-    k_geom_bwd<true><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_rest_count(sh_degree), dwa,
-                                               camera, near_z, blur, grad9, gparams, gsh_rest);
-  else
-    k_geom_bwd<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z, blur,
-                                                grad9, gparams, nullptr);
-  return launch_status();
+  return tts_geom_bwd_render(params, sh_rest, sh_degree, depth_bt, depth_zgrad, G, camera, near_z,
+                             blur, grad9, 9, nullptr, gparams, gsh_rest, gdepth, nullptr, 0,
+                             nullptr, nullptr, stream);
 }
 
 int tts_adam_flat(float* params, float* m, float* v, const float* grad, const float* lr1,
@@ -1627,14 +1670,14 @@ int tts_zero(float* buf, int64_t n, hipStream_t stream) {
 
 int tts_background(const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream) {
   if (!w_b_raw || !c_b || !bg) return TTS_EINVAL;
-  k_background<<<1, 64, 0, stream>>>(w_b_raw, c_b, bg);
+  k_background<<<1, 64, 0, stream>>>(BgArgs{w_b_raw, c_b, bg});
   return launch_status();
 }
 
 int tts_background_grad(const float* gwb, int n, const float* w_b_raw, float* gw_b_raw,
                         hipStream_t stream) {
   if (n < 0 || (n > 0 && !gwb) || !w_b_raw || !gw_b_raw) return TTS_EINVAL;
-  k_background_grad<<<1, 256, 0, stream>>>(gwb, n, w_b_raw, gw_b_raw);
+  k_background_grad<<<1, 256, 0, stream>>>(BgGrad{gwb, n, w_b_raw, gw_b_raw});
   return launch_status();
 }
 

@@ -216,6 +216,22 @@ __device__ __forceinline__ float block_sum256(float v, float* tmp) {
   return s;
 }
 
+// The blend's background block out[4] = (softplus(w_b_raw), c_b r, g, b) (spike/render.py:28),
+// written by threads 0-3 of one block of a kernel the render launches anyway (out null: nothing).
+struct BgArgs {
+  const float* raw;
+  const float* c_b;
+  float* out;
+};
+__device__ __forceinline__ void write_background(const BgArgs& a) {
+  if (threadIdx.x == 0) {
+    const float x = a.raw[0];
+    a.out[0] = x > 20.0f ? x : log1pf(expf(x));
+  } else if (threadIdx.x < 4) {
+    a.out[threadIdx.x] = a.c_b[threadIdx.x - 1];
+  }
+}
+
 // Camera block as stored in device memory (16 floats).
 struct Camera {
   float R[9];

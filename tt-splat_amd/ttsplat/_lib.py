@@ -80,6 +80,16 @@ SIGNATURES = {
                                           _vp, _vp, _vp, _c_float, _c_float, _c_int, _c_int,
                                           _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp,
                                           _vp, _vp, _vp, _vp, _vp, _c_size, _vp]),
+    "tts_geom_fwd_bg": (_c_int, [_vp, _vp, _c_int, _vp, _c_int, _vp, _c_float, _c_float, _vp, _vp,
+                                 _vp, _c_float, _c_float, _vp, _vp, _vp, _vp]),
+    "tts_geom_fwd_assign_bins_bg": (_c_int, [_vp, _vp, _c_int, _vp, _c_int, _vp, _c_float,
+                                             _c_float, _vp, _vp, _vp, _c_float, _c_float, _c_int,
+                                             _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp,
+                                             _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_size, _vp,
+                                             _vp, _vp, _vp]),
+    "tts_geom_bwd_render": (_c_int, [_vp, _vp, _c_int, _vp, _c_int, _c_int, _vp, _c_float,
+                                     _c_float, _vp, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _vp,
+                                     _vp, _vp]),
     "tts_geom_bwd_adam_fwd_count": (_c_int, [_vp, _c_int, _vp, _vp, _c_float, _c_float, _vp, _vp,
                                              _vp, _vp, _vp, _vp, _vp, _c_float, _c_float,
                                              _c_float, _vp, _vp, _c_int, _c_int, _c_int, _c_int,

@@ -81,10 +81,12 @@ def _raw_background(model, device):
 
 
 def _raw_background_grads(ctx, at, gwb, w_b_raw, c_b):
-    """Gradients of the inputs at positions `at`, `at + 1`: w_b_raw's from the partial sums of
-    dL/dw_b; c_b is a constant of the reference model, its gradient zero."""
-    gw = kernels.background_grad(gwb, w_b_raw) if ctx.needs_input_grad[at] else None
-    return gw, torch.zeros_like(c_b) if ctx.needs_input_grad[at + 1] else None
+    """Gradients of the inputs at positions `at`, `at + 1`, and geom_bwd's background argument:
+    w_b_raw's from the partial sums of dL/dw_b, written by that launch; c_b is a constant of the
+    reference model, its gradient zero."""
+    gw = torch.empty_like(w_b_raw) if ctx.needs_input_grad[at] else None
+    return (gw, torch.zeros_like(c_b) if ctx.needs_input_grad[at + 1] else None,
+            None if gw is None else (gwb, w_b_raw, gw))
 
 
 @torch.no_grad()
@@ -193,18 +195,23 @@ class BinnedRender(torch.autograd.Function):
     per-slot gradients -> slot->gaussian reduce (through the inverse table when the bins came
     with one, else an atomic scatter) -> geometry bwd.  proj: P's projection from this camera
     when the caller has it already; order: the tiles heaviest first, the splat kernels' dispatch
-    order (26.0 -> 19.0 us forward at G = 100k, 1264x832).  The background is either the block bg
-    [4] or, with bg None, made here from w_b_raw and c_b."""
+    order (26.0 -> 22.9 us forward at G = 100k, 1264x832).  The background is the block bg [4]; with
+    w_b_raw and c_b its gradient goes to them, and bg None is made from them here."""
 
     @staticmethod
     def forward(ctx, P, camera, bg, idx32, v8, inv, H, W, S, k, proj=None, order=None,
                 w_b_raw=None, c_b=None):
         Pc = P.detach().contiguous()
-        if bg is None:
+        if w_b_raw is not None:
             w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
-            bg = kernels.background(w_b_raw, c_b)
+        make = None
+        if bg is None:
+            bg = torch.empty(4, device=Pc.device, dtype=F32)
+            make = (w_b_raw, c_b, bg)
         if proj is None:
-            proj, _ = kernels.geom_fwd(Pc, camera)
+            proj, _ = kernels.geom_fwd(Pc, camera, background=make)
+        elif make is not None:
+            bg = kernels.background(w_b_raw, c_b)
         img, den = kernels.splat_fwd(proj, idx32, v8, bg, H, W, S, k, order=order)
         ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw, c_b)
         ctx.inv, ctx.order = inv, order
@@ -222,17 +229,17 @@ class BinnedRender(torch.autograd.Function):
         gslot = kernels.splat_bwd(proj, idx32, v8, bg, H, W, S, k, img, den,
                                   gimg.float().contiguous(), gslot=gslot, gwb=gwb,
                                   order=ctx.order)
-        if ctx.inv is not None:
-            grad9 = kernels.slot_reduce(gslot, ctx.inv)
-        else:
-            grad9 = kernels.slot_scatter(gslot, idx32, v8, Pc.shape[0])
-        gP = kernels.geom_bwd(Pc, camera, grad9)
-        gbg = gw = gc = None
+        gbg = gw = gc = make = None
         if w_b_raw is not None:
-            gw, gc = _raw_background_grads(ctx, 12, gwb, w_b_raw, c_b)
+            gw, gc, make = _raw_background_grads(ctx, 12, gwb, w_b_raw, c_b)
         else:
             gbg = torch.zeros(4, device=Pc.device, dtype=F32)
             gbg[0] = gwb.sum()
+        if ctx.inv is not None:
+            gP = kernels.geom_bwd(Pc, camera, gslot, inv=ctx.inv, background=make)
+        else:
+            grad9 = kernels.slot_scatter(gslot, idx32, v8, Pc.shape[0])
+            gP = kernels.geom_bwd(Pc, camera, grad9, background=make)
         return gP, None, gbg, None, None, None, None, None, None, None, None, None, gw, gc
 
 
@@ -243,18 +250,21 @@ def render_binned_device(model, cam, tmap, R=1, K=128, cached_bins=None, return_
     P = params_of(model)
     dev = P.device
     camera = cam.device_block(dev)
-    inv = proj = order = None
+    inv = proj = order = bg = None
+    w_b_raw, c_b = _raw_background(model, dev)
     if cached_bins is None:
         Pc = P.detach().contiguous()
+        bg = torch.empty(4, device=dev, dtype=F32)
         order = torch.empty(tmap.T, device=dev, dtype=torch.int32)
         if torch.is_grad_enabled():
             inv = torch.empty(P.shape[0], 9, device=dev, dtype=torch.int32)
         proj, _, idx32, v8, _, _ = kernels.geom_fwd_assign_bins(
-            Pc, camera, tmap.H, tmap.W, tmap.S, K, tmap.span, R, inv=inv, order=order)
+            Pc, camera, tmap.H, tmap.W, tmap.S, K, tmap.span, R, inv=inv, order=order,
+            background=(w_b_raw.detach(), c_b.detach().contiguous(), bg))
         bins = (idx32.long(), v8.bool()) if return_bins else None
     else:
         bins = cached_bins
         idx32, v8 = _checked_bins(bins, P.shape[0])
-    img = BinnedRender.apply(P, camera, None, idx32, v8, inv, tmap.H, tmap.W, tmap.S, float(k),
-                             proj, order, *_raw_background(model, dev))
+    img = BinnedRender.apply(P, camera, bg, idx32, v8, inv, tmap.H, tmap.W, tmap.S, float(k),
+                             proj, order, w_b_raw, c_b)
     return (img, bins) if return_bins else img

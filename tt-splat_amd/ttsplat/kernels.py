@@ -30,15 +30,23 @@ def version():
 
 
 # ------------------------------------------------------------------------------- geometry --
-def background(w_b_raw, c_b):
-    """bg block [softplus(w_b_raw), c_b r, g, b] from two device tensors of 1 and 3 elements."""
-    dev = w_b_raw.device
-    require(w_b_raw, "w_b_raw", F32)
+def _bg_args(background, dev):
+    """(w_b_raw, c_b, bg) checked, as pointers (None: NULLs)."""
+    if background is None:
+        return None, None, None
+    w_b_raw, c_b, bg = background
+    require(w_b_raw, "w_b_raw", F32, None, dev)
     require(c_b, "c_b", F32, None, dev)
+    require(bg, "bg", F32, (4,), dev)
     if w_b_raw.numel() != 1 or c_b.numel() != 3:
         raise ValueError("w_b_raw must hold one element and c_b three")
-    bg = torch.empty(4, device=dev, dtype=F32)
-    call("tts_background", ptr(w_b_raw), ptr(c_b), ptr(bg), stream())
+    return ptr(w_b_raw), ptr(c_b), ptr(bg)
+
+
+def background(w_b_raw, c_b):
+    """bg block [softplus(w_b_raw), c_b r, g, b] from two device tensors of 1 and 3 elements."""
+    bg = torch.empty(4, device=w_b_raw.device, dtype=F32)
+    call("tts_background", *_bg_args((w_b_raw, c_b, bg), w_b_raw.device), stream())
     return bg
 
 
@@ -81,12 +89,13 @@ def _dw_check(depth_bt, dev):
 
 
 def geom_fwd(params, camera, near=NEAR, blur=BLUR, proj=None, keep=None, sh_rest=None,
-             sh_degree=0, depth_bt=None, advance=None, b1=None, b2=None):
+             sh_degree=0, depth_bt=None, advance=None, b1=None, b2=None, background=None):
     """Projection + activations -> proj[G,12], keep[G].  sh_degree > 0: view-dependent colour
     from the rest coefficients sh_rest [15,3,G] (sh_rest_layout of spike's color_rest).
     depth_bt (device (beta, tau)): the depth weight sigmoid(beta (tau - z_cam)) on the opacity.
     advance (a training step's Adam step block): advanced in the same launch, as
-    adam_advance(advance, b1, b2) would."""
+    adam_advance(advance, b1, b2) would.  background: (w_b_raw, c_b, bg) -- the background block
+    bg [4] written in the same launch."""
     G = params.shape[0]
     dev = params.device
     require(params, "params", F32, (G, 14))
@@ -99,10 +108,11 @@ def geom_fwd(params, camera, near=NEAR, blur=BLUR, proj=None, keep=None, sh_rest
     require(keep, "keep", U8, (G,), dev)
     if advance is not None:
         require(advance, "advance", I32, (4,), dev)
-    if sh_degree > 0 or depth_bt is not None or advance is not None:
-        call("tts_geom_fwd_ex", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt), G,
+    if sh_degree > 0 or depth_bt is not None or advance is not None or background is not None:
+        call("tts_geom_fwd_bg", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt), G,
              ptr(camera), near, blur, ptr(proj), ptr(keep), ptr(advance),
-             BETA1 if b1 is None else b1, BETA2 if b2 is None else b2, stream())
+             BETA1 if b1 is None else b1, BETA2 if b2 is None else b2,
+             *_bg_args(background, dev), stream())
     else:
         call("tts_geom_fwd", ptr(params), G, ptr(camera), near, blur, ptr(proj), ptr(keep),
              stream())
@@ -110,22 +120,34 @@ def geom_fwd(params, camera, near=NEAR, blur=BLUR, proj=None, keep=None, sh_rest
 
 
 def geom_bwd(params, camera, grad9, near=NEAR, blur=BLUR, out=None, sh_rest=None, sh_degree=0,
-             gsh_out=None, depth_bt=None, depth_zgrad=False, gdepth=None, sh_dirgrad=False):
+             gsh_out=None, depth_bt=None, depth_zgrad=False, gdepth=None, sh_dirgrad=False,
+             inv=None, background=None):
     """grad9[G,9] -> dL/dparams[G,14].  With sh_degree > 0 also dL/dsh_rest [15,3,G]; with
     depth_bt also dL/d(beta, tau) per gaussian [G,2] (depth_zgrad: plus the gradient through
     z_cam into the means; sh_dirgrad: plus the SH colour's gradient through its view direction
     into the means, as spike's dense autograd has them).  Returns gparams, or a tuple
-    (gparams, gsh, gdepth) when either extension is on (absent parts None)."""
+    (gparams, gsh, gdepth) when either extension is on (absent parts None).
+    grad9 may have rows of 10 (the soft-Z arm's), or, with the inverse table inv [G,9], be the slot
+    gradients [T,K,9] it sums.  background: (gwb, w_b_raw, gw_b_raw) -- background_grad's result
+    written to gw_b_raw in the same launch."""
     G = params.shape[0]
     dev = params.device
     require(params, "params", F32, (G, 14))
     require(camera, "camera", F32, (16,), dev)
-    require(grad9, "grad9", F32, (G, 9), dev)
+    if inv is not None:
+        require(grad9, "gslot", F32, None, dev)
+        require(inv, "inv", I32, (G, 9), dev)
+        if sh_degree > 0 or depth_bt is not None:
+            raise ValueError("slot gradients come without SH and depth weight")
+    else:
+        stride = 10 if grad9.dim() == 2 and grad9.shape[1] == 10 else 9
+        require(grad9, "grad9", F32, (G, stride), dev)
     _sh_check(sh_rest, sh_degree, G, dev)
     _dw_check(depth_bt, dev)
     out = torch.empty(G, 14, device=dev, dtype=F32) if out is None else out
     require(out, "gparams", F32, (G, 14), dev)
-    if sh_degree > 0 or depth_bt is not None:
+    if sh_degree > 0 or depth_bt is not None or background is not None or inv is not None \
+            or stride != 9:
         gsh = None
         if sh_degree > 0:
             gsh = torch.empty(SH_REST, 3, G, device=dev, dtype=F32) if gsh_out is None else gsh_out
@@ -135,10 +157,17 @@ def geom_bwd(params, camera, grad9, near=NEAR, blur=BLUR, out=None, sh_rest=None
             gdw = torch.empty(G, 2, device=dev, dtype=F32) if gdepth is None else gdepth
             require(gdw, "gdepth", F32, (G, 2), dev)
         flags = (1 if depth_zgrad else 0) | (2 if sh_dirgrad and sh_degree > 0 else 0)
-        call("tts_geom_bwd_ex", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt),
-             flags, G, ptr(camera), near, blur, ptr(grad9), ptr(out), ptr(gsh), ptr(gdw),
-             stream())
-        return out, gsh, gdw
+        gwb = raw = graw = None
+        if background is not None:
+            gwb, raw, graw = background
+            require(gwb, "gwb", F32, None, dev)
+            require(raw, "w_b_raw", F32, None, dev)
+            require(graw, "gw_b_raw", F32, raw.shape, dev)
+        call("tts_geom_bwd_render", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt),
+             flags, G, ptr(camera), near, blur, ptr(grad9), 9 if inv is not None else stride,
+             ptr(inv), ptr(out), ptr(gsh), ptr(gdw), ptr(gwb), 0 if gwb is None else gwb.numel(),
+             ptr(raw), ptr(graw), stream())
+        return (out, gsh, gdw) if sh_degree > 0 or depth_bt is not None else out
     call("tts_geom_bwd", ptr(params), G, ptr(camera), near, blur, ptr(grad9), ptr(out), stream())
     return out
 
@@ -192,12 +221,13 @@ def geom_fwd_assign_bins(params, camera, H, W, S=16, K=128, span=2048, R=1, near
                          blur=BLUR, proj=None, keep=None, sh_rest=None, sh_degree=0,
                          depth_bt=None, advance=None, b1=None, b2=None, workspace=None, idx=None,
                          valid=None, count=None, ncand=None, inv=None, order=None,
-                         slot_rec=None, pos_count=None):
+                         slot_rec=None, pos_count=None, background=None):
     """geom_fwd then assign_bins on proj's means and keep, as one call (for G <= 131072 the
     binning's count pass runs inside the geometry launch).  Returns (proj, keep, idx, valid,
     count, ncand); inv and order are written when buffers are passed, and with order the slot
     records slot_rec [T,K,12] (proj[idx] of every kept slot, tiles in dispatch order) and
-    pos_count [T] (their kept counts) when those are passed."""
+    pos_count [T] (their kept counts) when those are passed.  background: (w_b_raw, c_b, bg) as
+    geom_fwd takes it."""
     G = params.shape[0]
     dev = params.device
     require(params, "params", F32, (G, 14))
@@ -231,11 +261,11 @@ def geom_fwd_assign_bins(params, camera, H, W, S=16, K=128, span=2048, R=1, near
         _aligned16(require(slot_rec, "slot_rec", F32, (T, K, 12), dev), "slot_rec")
         require(pos_count, "pos_count", I32, (T,), dev)
     workspace = bin_workspace(G, H, W, S, dev) if workspace is None else workspace
-    call("tts_geom_fwd_assign_bins", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt),
+    call("tts_geom_fwd_assign_bins_bg", ptr(params), ptr(sh_rest), int(sh_degree), ptr(depth_bt),
          G, ptr(camera), near, blur, ptr(proj), ptr(keep), ptr(advance),
          BETA1 if b1 is None else b1, BETA2 if b2 is None else b2, H, W, S, R, K, span,
          ptr(idx), ptr(valid), ptr(count), ptr(ncand), ptr(inv), ptr(order), ptr(slot_rec),
-         ptr(pos_count), ptr(workspace), workspace.numel(), stream())
+         ptr(pos_count), ptr(workspace), workspace.numel(), *_bg_args(background, dev), stream())
     return proj, keep, idx, valid, count, ncand
 
 

@@ -50,11 +50,13 @@ class DenseRender(torch.autograd.Function):
         szc = None if szb is None else szb.detach().float().reshape(1).contiguous()
         rc = None if rest is None else rest.detach().float().contiguous()
         deg = int(sh_degree) if rc is not None else 0
-        proj, _ = kernels.geom_fwd(Pc, camera, near=near, blur=blur, depth_bt=btc, sh_rest=rc,
-                                   sh_degree=deg)
+        make = None
         if bg is None:
             w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
-            bg = kernels.background(w_b_raw, c_b)
+            bg = torch.empty(4, device=Pc.device, dtype=F32)
+            make = (w_b_raw, c_b, bg)
+        proj, _ = kernels.geom_fwd(Pc, camera, near=near, blur=blur, depth_bt=btc, sh_rest=rc,
+                                   sh_degree=deg, background=make)
         bgc = bg.detach().contiguous()
         if blend == "A":
             img, den = kernels.render_dense(proj, H, W, k, bgc)
@@ -76,25 +78,25 @@ class DenseRender(torch.autograd.Function):
         if blend == "A":
             grad9, gwb = kernels.render_dense_bwd(proj, H, W, k, bgc, img, den, gi)
         else:
-            g, gwb = kernels.render_dense_arm_bwd(proj, H, W, k, bgc, blend, img, den, aux, gi,
-                                                  szc)
-            grad9 = g[:, :9].contiguous()
+            grad9, gwb = kernels.render_dense_arm_bwd(proj, H, W, k, bgc, blend, img, den, aux, gi,
+                                                      szc)
             if blend == "SZ":
-                gszb = g[:, 9].sum().reshape(1)
+                gszb = grad9[:, 9].sum().reshape(1)
+        gbg = gw = gc = make = None
+        if w_b_raw is not None:
+            gw, gc, make = _raw_background_grads(ctx, 13, gwb, w_b_raw, c_b)
+        else:
+            gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
         gbt = grest = None
         if btc is None and deg == 0:
-            gP = kernels.geom_bwd(Pc, camera, grad9, near=near, blur=blur)
+            gP = kernels.geom_bwd(Pc, camera, grad9, near=near, blur=blur, background=make)
         else:
             gP, grest, gdw = kernels.geom_bwd(Pc, camera, grad9, near=near, blur=blur,
                                               depth_bt=btc, depth_zgrad=btc is not None,
-                                              sh_rest=rc, sh_degree=deg, sh_dirgrad=True)
+                                              sh_rest=rc, sh_degree=deg, sh_dirgrad=True,
+                                              background=make)
             if gdw is not None:
                 gbt = gdw.sum(0)
-        gbg = gw = gc = None
-        if w_b_raw is not None:
-            gw, gc = _raw_background_grads(ctx, 13, gwb, w_b_raw, c_b)
-        else:
-            gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
         return (gP, None, gbg, gbt, gszb, grest, None, None, None, None, None, None, None, gw,
                 gc)
 
