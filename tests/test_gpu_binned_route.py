@@ -53,3 +53,35 @@ def test_int64_ids_are_the_int32_ones(S, K, G):
         idx, valid = binned.assign_bins(mu, k, binned.TileMap(H, W, S), 1, K)
         assert torch.equal(idx, b[0]) and valid.dtype == torch.bool
         assert torch.equal(valid, b[1].bool())
+
+
+@pytest.mark.parametrize("dense", [False, True])
+def test_background_inputs_between_forward_and_backward(dense):
+    """c_b, and a w_b_raw that needs no gradient, may change in place before the backward; w_b_raw's
+    gradient can be differentiated again (through softplus: the renders themselves cannot)."""
+    from ttsplat.render import render
+    _, P, _ = config_inputs("c1_ref", G=200)
+    cam, tmap = pinhole(32, 48, (0.3, 0.2, 3.0)), binned.TileMap(32, 48)
+
+    def image(model):
+        return render(model, cam, "A") if dense else binned.render_binned_device(model, cam, tmap)
+
+    model = GaussianModel(P.cuda())
+    model.params.requires_grad_(True)
+    img = image(model)
+    model.c_b.mul_(0.5)
+    model.w_b_raw.add_(1.0)
+    img.square().sum().backward()
+    assert bool(torch.isfinite(model.params.grad).all())
+
+    model = GaussianModel(P.cuda())
+    w = model.w_b_raw.requires_grad_(True)
+    c = model.c_b.requires_grad_(True)
+    loss = image(model).square().sum()
+    gw, gc = torch.autograd.grad(loss, [w, c], retain_graph=True)
+    assert gw.shape == w.shape and torch.equal(gc, torch.zeros(3, device="cuda"))
+    (g2,) = torch.autograd.grad(loss, w, create_graph=True)
+    assert torch.allclose(gw, g2, rtol=1e-5)
+    (gg,) = torch.autograd.grad(g2, w)
+    s = torch.sigmoid(w.detach())
+    assert torch.allclose(gg, g2.detach() * (1 - s), rtol=1e-5)

@@ -83,6 +83,15 @@ inline size_t quad_ws_bytes(int G, int P) {
          pad256((size_t)P * 8) + (sh > 1 ? sh * (size_t)G * (kQuadComp + 1) * 4 : 0);
 }
 
+// A long 1-D grid: blocks past 2^21 go to the z dimension (a launch holds under 2^32 threads per
+// dimension).  The kernels take block_id() and leave when it is past their work.
+inline dim3 grid_split(int64_t blocks, int y = 1) {
+  constexpr int64_t kRow = int64_t(1) << 21;
+  return blocks <= kRow ? dim3((unsigned)blocks, y)
+                        : dim3((unsigned)kRow, y, (unsigned)((blocks + kRow - 1) / kRow));
+}
+__device__ __forceinline__ int block_id() { return (int)(blockIdx.x + gridDim.x * blockIdx.z); }
+
 // ---------------------------------------------------------------- support culling
 //
 // A gaussian weighs nothing where Q >= k, so a tile of pixels only needs the gaussians whose
@@ -164,7 +173,8 @@ struct DenseWalk {
       }
       return;
     }
-    const float cx = (float)(X0 + (lane_x() & ~7)) + 4.0f, cy = (float)(Y0 + (lane_y() & ~7)) + 4.0f;
+    const float cx = (float)(X0 + (lane_x() & ~7)) + 4.0f;
+    const float cy = (float)(Y0 + (lane_y() & ~7)) + 4.0f;
     int seen = 0;
     for (int j0 = 0; j0 < n; j0 += 64) {
       const int j = min(j0 + lane, n - 1);
@@ -283,8 +293,9 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
                                                      float4* __restrict__ aux) {
   using Walk = DenseWalk<TS, NT>;
   __shared__ Walk s;
-  const int tx = (W + TS - 1) / TS;
-  const int X0 = (int)(blockIdx.x % tx) * TS, Y0 = (int)(blockIdx.x / tx) * TS;
+  const int tx = (W + TS - 1) / TS, bid = block_id();
+  const int X0 = bid % tx * TS, Y0 = bid / tx * TS;
+  if (Y0 >= H) return;
   const int x = X0 + Walk::lane_x(), y = Y0 + Walk::lane_y();
   const float px = (float)x + 0.5f, py = (float)y + 0.5f;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
@@ -354,12 +365,12 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
   __shared__ float4 s_c[kThetaThreads];  // o*keep*color, o*keep
   __shared__ float2 s_b[kThetaThreads];  // theta 4, 5
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int p0 = blockIdx.x * 64 * PX + lane;
+  const int64_t p0 = (int64_t)block_id() * 64 * PX + lane;
   float f[PX][6], n[PX][4];
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) f[i][k] = p0 + i * 64 < P ? phi[(int64_t)(p0 + i * 64) * 6 + k] : 0.f;
+    for (int k = 0; k < 6; ++k) f[i][k] = p0 + i * 64 < P ? phi[(p0 + i * 64) * 6 + k] : 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) n[i][k] = 0.f;
   }
@@ -500,8 +511,9 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
                                                   float2* __restrict__ ex, int* __restrict__ wild) {
   using Walk = DenseWalk<TS, NT>;
   __shared__ Walk s;
-  const int tx = (W + TS - 1) / TS;
-  const int X0 = (int)(blockIdx.x % tx) * TS, Y0 = (int)(blockIdx.x / tx) * TS;
+  const int tx = (W + TS - 1) / TS, bid = block_id();
+  const int X0 = bid % tx * TS, Y0 = bid / tx * TS;
+  if (Y0 >= H) return;
   const int x = X0 + Walk::lane_x(), y = Y0 + Walk::lane_y();
   const bool in = x < W && y < H;
   const int64_t p = (int64_t)y * W + x;
@@ -551,14 +563,14 @@ __global__ __launch_bounds__(256) void k_render_dense_bwd(
   __shared__ float s_sum[4][NC];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = wave % WPG;
-  const int g = (int)blockIdx.x * (4 / WPG) + wave / WPG;
+  const int64_t g = (int64_t)block_id() * (4 / WPG) + wave / WPG;
   const bool act = g < G;
-  const float4* rec = reinterpret_cast<const float4*>(proj + (int64_t)min(g, G - 1) * 12);
+  const float4* rec = reinterpret_cast<const float4*>(proj + min(g, (int64_t)G - 1) * 12);
   const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
   int any = 0;
   for (int i = lane; i < n_wild; i += 64) any |= wild[i];
   if (__ballot(any != 0)) cull = 0;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && gwb) {
+  if (block_id() == 0 && blockIdx.y == 0 && wave == 0 && gwb) {
     float t = 0.0f;
     for (int i = lane; i < n_pre; i += 64) t += gwb_part[i];
     t = wave_sum(t);
@@ -701,8 +713,8 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense_bwd(
   float4* s_fa = s_px + kThetaThreads;                                // phi 0..3
   float2* s_fb = reinterpret_cast<float2*>(s_fa + kThetaThreads);     // phi 4..5
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int band = blockIdx.y;
-  const int g = blockIdx.x * 64 + lane;
+  const int band = blockIdx.y, gblock = block_id();
+  const int64_t g = (int64_t)gblock * 64 + lane;
   const bool act = g < G;
   float th[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float og = 0.f, kp = 0.f, col[3] = {0.f, 0.f, 0.f};
@@ -758,12 +770,12 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense_bwd(
       v[5] += gu * fb2.y;
     }
   }
-  if (blockIdx.x == 0) {
+  if (gblock == 0) {
     const float t = wave_sum(wpart);
     if (lane == 0) s_wb[wave] = t;
   }
   __syncthreads();
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (gblock == 0 && threadIdx.x == 0) {
     float t = 0.f;
 #pragma unroll
     for (int w = 0; w < kThetaWaves; ++w) t += s_wb[w];
@@ -844,16 +856,16 @@ void launch_render_dense(const float* proj, int G, int H, int W, float ik, const
                          const float* szb, float* image, float* den, float4* aux,
                          hipStream_t stream) {
   const int ts = dense_tile_side(H, W), cull = dense_cull(H, W);
-  const int nb = dense_tiles(H, W, ts);
+  const dim3 grid = grid_split(dense_tiles(H, W, ts));
   if (ts == 32)
-    k_render_dense<ARM, 32, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
-                                                           den, aux);
+    k_render_dense<ARM, 32, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb,
+                                                             image, den, aux);
   else if (ts == 16)
-    k_render_dense<ARM, 16, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
-                                                           den, aux);
+    k_render_dense<ARM, 16, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb,
+                                                             image, den, aux);
   else
-    k_render_dense<ARM, 8, 512><<<nb, 512, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
-                                                        den, aux);
+    k_render_dense<ARM, 8, 512><<<grid, 512, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
+                                                          den, aux);
 }
 
 // The whole quad backward of an arm; grad has kQuadComp columns (SZ: one more).
@@ -876,25 +888,26 @@ int launch_dense_bwd(const float* proj, int G, int H, int W, float ik, const flo
   const int npre = P / 256 + 1 < kPreBlocks ? P / 256 + 1 : kPreBlocks;
   k_dense_pre<ARM><<<npre, 256, 0, stream>>>(image, den, aux, gimage, P, bg, q, ex, gwbp, wild);
   if (ARM == kArmSZ) {
-    const int ts = dense_tile_side(H, W), nb = dense_tiles(H, W, ts);
+    const int ts = dense_tile_side(H, W);
+    const dim3 grid = grid_split(dense_tiles(H, W, ts));
     if (ts == 32)
-      k_softz_pre<32, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                     wild + npre);
+      k_softz_pre<32, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                       wild + npre);
     else if (ts == 16)
-      k_softz_pre<16, 1024><<<nb, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                     wild + npre);
+      k_softz_pre<16, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                       wild + npre);
     else
-      k_softz_pre<8, 512><<<nb, 512, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                  wild + npre);
+      k_softz_pre<8, 512><<<grid, 512, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                    wild + npre);
   }
   const int sh = quad_shares(G), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
   float* dst = sh > 1 ? part : grad;
   const int nw = npre + (ARM == kArmSZ ? 1 : 0);
   if (dense_wide(G, P))
-    k_render_dense_bwd<ARM, 4><<<dim3(G, sh), 256, 0, stream>>>(
+    k_render_dense_bwd<ARM, 4><<<grid_split(G, sh), 256, 0, stream>>>(
         proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
   else
-    k_render_dense_bwd<ARM, 1><<<dim3((G + 3) / 4, sh), 256, 0, stream>>>(
+    k_render_dense_bwd<ARM, 1><<<grid_split(((int64_t)G + 3) / 4, sh), 256, 0, stream>>>(
         proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
   if (sh > 1)
     k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, sh, G, nc, nullptr,
@@ -1007,11 +1020,11 @@ int tts_wsr_dense(const float* theta, const float* o, const float* color, const 
   // 200x200 116 / 95; G 2000, 600x600 263 / 209 (one thread per pixel, a chain over G: 79, 230, 230
   // and 278).
   if (P <= 32768)
-    k_wsr_dense<1><<<grid1d(P, 64), kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P,
-                                                                bg, C, den);
+    k_wsr_dense<1><<<grid_split(grid1d(P, 64)), kThetaThreads, 0, stream>>>(
+        theta, o, color, keep, phi, G, P, bg, C, den);
   else
-    k_wsr_dense<4><<<grid1d(P, 256), kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P,
-                                                                 bg, C, den);
+    k_wsr_dense<4><<<grid_split(grid1d(P, 256)), kThetaThreads, 0, stream>>>(
+        theta, o, color, keep, phi, G, P, bg, C, den);
   return launch_status();
 }
 
@@ -1027,7 +1040,7 @@ int tts_wsr_dense_bwd(const float* theta, const float* o, const float* color,
   int PB;
   const int nb = theta_ws(workspace, workspace_bytes, G, P, &part, &gwbp, &PB);
   if (nb < 0) return nb;
-  dim3 grid(grid1d(G, 64), nb);
+  const dim3 grid = grid_split(grid1d(G, 64), nb);
   k_wsr_dense_bwd<<<grid, kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P, PB, bg, C,
                                                       den, gC, part, gwbp);
   k_dense_reduce<<<grid1d((int64_t)G * kThetaComp, 256), 256, 0, stream>>>(

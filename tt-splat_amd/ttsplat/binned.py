@@ -80,13 +80,19 @@ def _raw_background(model, device):
             c_b if c_b.numel() == 3 else c_b.reshape(3))
 
 
-def _raw_background_grads(ctx, at, gwb, w_b_raw, c_b):
-    """Gradients of the inputs at positions `at`, `at + 1`, and geom_bwd's background argument:
-    w_b_raw's from the partial sums of dL/dw_b, written by that launch; c_b is a constant of the
-    reference model, its gradient zero."""
-    gw = torch.empty_like(w_b_raw) if ctx.needs_input_grad[at] else None
-    return (gw, torch.zeros_like(c_b) if ctx.needs_input_grad[at + 1] else None,
-            None if gw is None else (gwb, w_b_raw, gw))
+def _raw_background_grads(ctx, at, gwb, w_b_raw):
+    """Gradients of the inputs at positions `at` (w_b_raw) and `at + 1` (c_b), and geom_bwd's
+    background argument.  w_b_raw's comes from the partial sums of dL/dw_b and is written by that
+    launch, or made with tensor operations where it is to be differentiated again; c_b is a
+    constant of the reference model, its gradient zero."""
+    gc = torch.zeros(ctx.c_b_shape, device=gwb.device, dtype=F32) if ctx.needs_input_grad[at + 1] \
+        else None
+    if not ctx.needs_input_grad[at]:
+        return None, gc, None
+    if torch.is_grad_enabled():
+        return (gwb.sum() * torch.sigmoid(w_b_raw)).reshape(w_b_raw.shape), gc, None
+    gw = torch.empty_like(w_b_raw)
+    return gw, gc, (gwb, w_b_raw.detach(), gw)
 
 
 @torch.no_grad()
@@ -202,25 +208,26 @@ class BinnedRender(torch.autograd.Function):
     def forward(ctx, P, camera, bg, idx32, v8, inv, H, W, S, k, proj=None, order=None,
                 w_b_raw=None, c_b=None):
         Pc = P.detach().contiguous()
-        if w_b_raw is not None:
-            w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
         make = None
         if bg is None:
             bg = torch.empty(4, device=Pc.device, dtype=F32)
-            make = (w_b_raw, c_b, bg)
+            make = (w_b_raw.detach(), c_b.detach().contiguous(), bg)
         if proj is None:
             proj, _ = kernels.geom_fwd(Pc, camera, background=make)
         elif make is not None:
-            bg = kernels.background(w_b_raw, c_b)
+            bg = kernels.background(*make[:2])
         img, den = kernels.splat_fwd(proj, idx32, v8, bg, H, W, S, k, order=order)
-        ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw, c_b)
+        keep_raw = w_b_raw is not None and ctx.needs_input_grad[12]
+        ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den,
+                              w_b_raw if keep_raw else None)
+        ctx.c_b_shape = None if c_b is None else c_b.shape
         ctx.inv, ctx.order = inv, order
         ctx.meta = (H, W, S, k)
         return img
 
     @staticmethod
     def backward(ctx, gimg):
-        Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw, c_b = ctx.saved_tensors
+        Pc, camera, bg, idx32, v8, proj, img, den, w_b_raw = ctx.saved_tensors
         H, W, S, k = ctx.meta
         gwb = torch.empty(idx32.shape[0], device=Pc.device, dtype=F32)
         gslot = None
@@ -230,8 +237,8 @@ class BinnedRender(torch.autograd.Function):
                                   gimg.float().contiguous(), gslot=gslot, gwb=gwb,
                                   order=ctx.order)
         gbg = gw = gc = make = None
-        if w_b_raw is not None:
-            gw, gc, make = _raw_background_grads(ctx, 12, gwb, w_b_raw, c_b)
+        if ctx.c_b_shape is not None:
+            gw, gc, make = _raw_background_grads(ctx, 12, gwb, w_b_raw)
         else:
             gbg = torch.zeros(4, device=Pc.device, dtype=F32)
             gbg[0] = gwb.sum()

@@ -183,8 +183,8 @@ def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, i
                 valid=None, count=None, ncand=None, inv=None, order=None, idx_dtype=I32):
     """mu2d: [G,2] fp32 (or any [G,>=2] row-contiguous view, e.g. the proj record),
     keep: [G] uint8 or bool.  Returns idx[T,K] int32 (idx_dtype=torch.int64: int64),
-    valid[T,K] uint8, count[T], ncand[T]; the inverse table inv[G,9] and the heaviest-first tile order[T] are written when buffers are
-    passed."""
+    valid[T,K] uint8, count[T], ncand[T]; the inverse table inv[G,9] and the heaviest-first tile
+    order[T] are written when buffers are passed."""
     G = mu2d.shape[0]
     dev = mu2d.device
     if not mu2d.is_cuda or mu2d.dtype != F32 or mu2d.dim() != 2 or mu2d.shape[1] < 2 \
@@ -211,8 +211,8 @@ def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, i
     if order is not None:
         require(order, "order", I32, (T,), dev)
     workspace = bin_workspace(G, H, W, S, dev) if workspace is None else workspace
-    call("tts_assign_bins" if idx_dtype == I32 else "tts_assign_bins_i64", ptr(mu2d), mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span,
-         ptr(idx), ptr(valid), ptr(count), ptr(ncand), ptr(inv), ptr(order), ptr(workspace),
+    call("tts_assign_bins" if idx_dtype == I32 else "tts_assign_bins_i64", ptr(mu2d),
+         mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span, ptr(idx), ptr(valid), ptr(count), ptr(ncand), ptr(inv), ptr(order), ptr(workspace),
          workspace.numel(), stream())
     return idx, valid, count, ncand
 

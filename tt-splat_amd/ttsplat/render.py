@@ -52,9 +52,8 @@ class DenseRender(torch.autograd.Function):
         deg = int(sh_degree) if rc is not None else 0
         make = None
         if bg is None:
-            w_b_raw, c_b = w_b_raw.detach(), c_b.detach().contiguous()
             bg = torch.empty(4, device=Pc.device, dtype=F32)
-            make = (w_b_raw, c_b, bg)
+            make = (w_b_raw.detach(), c_b.detach().contiguous(), bg)
         proj, _ = kernels.geom_fwd(Pc, camera, near=near, blur=blur, depth_bt=btc, sh_rest=rc,
                                    sh_degree=deg, background=make)
         bgc = bg.detach().contiguous()
@@ -64,13 +63,14 @@ class DenseRender(torch.autograd.Function):
         else:
             img, den, aux = kernels.render_dense_arm(proj, H, W, k, bgc, blend, szc)
         ctx.save_for_backward(Pc, camera, bg, proj, img, den, btc, szc, aux, rc,
-                              w_b_raw, c_b)
+                              w_b_raw if make is not None and ctx.needs_input_grad[13] else None)
+        ctx.c_b_shape = None if make is None else c_b.shape
         ctx.meta = (H, W, k, blur, near, blend, deg)
         return img
 
     @staticmethod
     def backward(ctx, gimg):
-        Pc, camera, bg, proj, img, den, btc, szc, aux, rc, w_b_raw, c_b = ctx.saved_tensors
+        Pc, camera, bg, proj, img, den, btc, szc, aux, rc, w_b_raw = ctx.saved_tensors
         H, W, k, blur, near, blend, deg = ctx.meta
         bgc = bg.detach().contiguous()
         gi = gimg.float().contiguous()
@@ -83,8 +83,8 @@ class DenseRender(torch.autograd.Function):
             if blend == "SZ":
                 gszb = grad9[:, 9].sum().reshape(1)
         gbg = gw = gc = make = None
-        if w_b_raw is not None:
-            gw, gc, make = _raw_background_grads(ctx, 13, gwb, w_b_raw, c_b)
+        if ctx.c_b_shape is not None:
+            gw, gc, make = _raw_background_grads(ctx, 13, gwb, w_b_raw)
         else:
             gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
         gbt = grest = None
