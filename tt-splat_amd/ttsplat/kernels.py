@@ -212,8 +212,8 @@ def assign_bins(mu2d, keep, H, W, S=16, K=128, span=2048, R=1, workspace=None, i
         require(order, "order", I32, (T,), dev)
     workspace = bin_workspace(G, H, W, S, dev) if workspace is None else workspace
     call("tts_assign_bins" if idx_dtype == I32 else "tts_assign_bins_i64", ptr(mu2d),
-         mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span, ptr(idx), ptr(valid), ptr(count), ptr(ncand), ptr(inv), ptr(order), ptr(workspace),
-         workspace.numel(), stream())
+         mu2d.stride(0), ptr(keep), 1, G, H, W, S, R, K, span, ptr(idx), ptr(valid), ptr(count),
+         ptr(ncand), ptr(inv), ptr(order), ptr(workspace), workspace.numel(), stream())
     return idx, valid, count, ncand
 
 
