@@ -518,7 +518,10 @@ __global__ __launch_bounds__(1024) void k_loss_value(const float* __restrict__ p
 // block a shorter chain: at 128x128 40 rows (24 blocks) 11.5 us, 24 rows 9.2, 16 rows 8.0, 8 rows
 // 6.5; at 320x480 11.5, 11.7, 10.1, 11.0; at 600x800 18.8, 17.7, 20.1, 23.9; at 832x1264 30.2,
 // 33.9, 37.0, 45.6.  A launch takes about a + b n with n = blocks per CU, rounded up (fitted to 15
-// sizes from 24x24 to 1072x1920, within 8 %); the rows with the least of it are taken.
+// sizes from 24x24 to 1072x1920, within 10 %); the rows with the least of it are taken.  Whole
+// training steps at 40 / 24 / 16 / 8 rows: G 10000, 800x800 73.7 / 72.1 / 72.7 / 77.4 us; G 20000,
+// 320x480 75.0 / 74.6 / 72.6 / 72.8; 608x800 97.5 / 95.0 / 97.7 / 99.7; 640x640 87.1 / 88.9 / 89.6 /
+// 91.0; 960x1600 133.9 / 131.7 / 138.9 / 150.1.
 using Tile40 = FGeo<40, 15, 13>;
 using Tile24 = FGeo<24, 11, 10>;
 using Tile16 = FGeo<16, 9, 8>;
@@ -530,7 +533,7 @@ inline int loss_items(int H, int W, int rows) {
 }
 inline int loss_rows(int H, int W) {
   struct Cost { int rows; double a, b; };   // us
-  constexpr Cost cost[] = {{40, 6.5, 4.7}, {24, 6.0, 3.1}, {16, 5.9, 2.2}, {8, 5.3, 1.4}};
+  constexpr Cost cost[] = {{40, 6.5, 4.7}, {24, 6.0, 3.1}, {16, 5.9, 2.4}, {8, 5.3, 1.4}};
   int best = 40;
   double least = 1e30;
   for (const Cost& c : cost) {
