@@ -390,7 +390,7 @@ int tts_geom_fwd_assign_bins(const float* params, const float* sh_rest, int sh_d
 /* tts_geom_fwd_ex and tts_geom_fwd_assign_bins that also write the background block tts_background
  * makes (bg, from w_b_raw and c_b; NULL: not), and tts_geom_bwd_ex that also makes
  * tts_background_grad's gradient (gw_b_raw; NULL: not) and takes the projected gradients either as
- * rows grad_stride >= 9 floats apart (inv NULL) or as slot gradients [T,K,9] through the inverse
+ * rows grad_stride = 9 or 10 floats apart (inv NULL) or as slot gradients [T,K,9] through the inverse
  * table inv (tts_slot_reduce's sum; no SH, no depth weight): one launch each. */
 int tts_geom_fwd_bg(const float* params, const float* sh_rest, int sh_degree,
                     const float* depth_bt, int G, const float* camera, float near_z, float blur,

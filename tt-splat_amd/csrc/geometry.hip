@@ -22,6 +22,8 @@
 
 #include <atomic>
 
+#include <type_traits>
+
 #include "bin_count.h"
 
 namespace tts {
@@ -758,7 +760,7 @@ __device__ __forceinline__ void gather_slot_grads(const float* __restrict__ gslo
     for (int c = 0; c < 9; ++c) gin[c] += e[j] >= 0 ? v[j][c] : 0.0f;
 }
 
-// dL/dw_b_raw from n partial sums of dL/dw_b (one block's work, summed in 64 bits in a fixed order).
+// dL/dw_b_raw from n partial sums of dL/dw_b (one block's work, a fixed order in 64 bits).
 struct BgGrad {
   const float* gwb;
   int n;
@@ -780,21 +782,21 @@ __device__ __forceinline__ void background_grad(const BgGrad& a) {
   }
 }
 
-// Gradient of one gaussian's nine projected quantities (grad, rows `stride` floats apart; GATHER:
+// Gradient of one gaussian's nine projected quantities (grad, rows STRIDE floats apart; GATHER:
 // summed here from the slot gradients through the inverse table, as k_slot_reduce) to its
-// parameters.  With bgg.graw the last block, past the gaussians', makes the background's gradient:
-// a render's backward then needs no launches of its own for either.
+// parameters.  BG: the last block, past the gaussians', makes the background's gradient.  A
+// render's backward then needs no launches of its own for either.
 // gsh (SH only): dL/drest in the rest layout; rows l >= n_rest are written as zero.
-template <bool SH, bool GATHER = false>
+template <bool SH, bool GATHER = false, int STRIDE = 9, bool BG = false>
 __global__ __launch_bounds__(256) void k_geom_bwd(const float* __restrict__ params, int G,
                                                   const float* __restrict__ rest, int n_rest,
                                                   DepthW dwa, const float* __restrict__ camera,
                                                   float near_z, float blur,
-                                                  const float* __restrict__ grad, int stride,
+                                                  const float* __restrict__ grad,
                                                   const int32_t* __restrict__ inv,
                                                   float* __restrict__ gparams,
                                                   float* __restrict__ gsh, BgGrad bgg) {
-  if (bgg.graw && blockIdx.x == gridDim.x - 1) {
+  if (BG && blockIdx.x == gridDim.x - 1) {
     background_grad(bgg);
     return;
   }
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(256) void k_geom_bwd(const float* __restrict__ para
     gather_slot_grads(grad, inv, g, gin);
   } else {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) gin[i] = grad[(int64_t)g * stride + i];
+    for (int i = 0; i < 9; ++i) gin[i] = grad[(int64_t)g * STRIDE + i];
   }
   geo_backward(p, cam, s, gin, gout, gcol, gdw, (dwa.zgrad & TTS_GRAD_DEPTH_Z) != 0);
   if (SH && (dwa.zgrad & TTS_GRAD_SH_DIR)) sh_dir_grad(p, cam, rv, n_rest, gcol, gout);
@@ -1020,8 +1022,9 @@ __global__ __launch_bounds__(kAdamBlock) void k_geom_bwd_adam(
   }
   __syncthreads();
   if ((int)threadIdx.x < rows)
-    bwd_adam_row<SH, MC, ACC>(threadIdx.x, g, G, s_p, s_m, s_v, s_inv, rest, sh_m, sh_v, n_rest, camera,
-                         near_z, blur, gslot, gparams, lr, lr_sh, step, b1, b2, eps, mc, dwa, gacc, scale);
+    bwd_adam_row<SH, MC, ACC>(threadIdx.x, g, G, s_p, s_m, s_v, s_inv, rest, sh_m, sh_v, n_rest,
+                              camera, near_z, blur, gslot, gparams, lr, lr_sh, step, b1, b2, eps,
+                              mc, dwa, gacc, scale);
   __syncthreads();
   stage_out<14, 15, kAdamBlock>(params, g0, rows, s_p);
   stage_out<14, 15, kAdamBlock>(m, g0, rows, s_m);
@@ -1427,7 +1430,7 @@ int tts_geom_bwd(const float* params, int G, const float* camera, float near_z, 
   if (G == 0) return TTS_OK;
   k_geom_bwd<false><<<grid1d(G, 256), 256, 0, stream>>>(params, G, nullptr, 0,
                                                         DepthW{nullptr, nullptr, 1.0f, 0, 0},
-                                                        camera, near_z, blur, grad9, 9, nullptr,
+                                                        camera, near_z, blur, grad9, nullptr,
                                                         gparams, nullptr, BgGrad{});
   return launch_status();
 }
@@ -1442,7 +1445,7 @@ int tts_geom_bwd_render(const float* params, const float* sh_rest, int sh_degree
   if (const int e = sh_args(sh_degree, sh_rest)) return e;
   if (sh_degree > 0 && !gsh_rest) return TTS_EINVAL;
   if (inv && (sh_degree > 0 || depth_bt)) return TTS_EINVAL;  // the binned render has neither
-  if (!inv && grad_stride < 9) return TTS_EINVAL;
+  if (!inv && grad_stride != 9 && grad_stride != 10) return TTS_EINVAL;
   if (gw_b_raw && (n_gwb < 0 || (n_gwb > 0 && !gwb) || !w_b_raw)) return TTS_EINVAL;
   if (G >= (1 << 30)) return TTS_EG;
   const BgGrad bgg{gwb, n_gwb, w_b_raw, gw_b_raw};
@@ -1452,16 +1455,17 @@ int tts_geom_bwd_render(const float* params, const float* sh_rest, int sh_degree
   }
   const DepthW dwa{depth_bt, gdepth, 1.0f, 0, depth_zgrad & (TTS_GRAD_DEPTH_Z | TTS_GRAD_SH_DIR)};
   const dim3 grid = grid1d(G, 256) + (gw_b_raw ? 1 : 0);
-  if (sh_degree > 0)
-    k_geom_bwd<true><<<grid, 256, 0, stream>>>(params, G, sh_rest, sh_rest_count(sh_degree), dwa,
-                                               camera, near_z, blur, grad, grad_stride, nullptr,
-                                               gparams, gsh_rest, bgg);
-  else if (inv)
-    k_geom_bwd<false, true><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z,
-                                                      blur, grad, 9, inv, gparams, nullptr, bgg);
-  else
-    k_geom_bwd<false><<<grid, 256, 0, stream>>>(params, G, nullptr, 0, dwa, camera, near_z, blur,
-                                                grad, grad_stride, nullptr, gparams, nullptr, bgg);
+  const float* rest = sh_degree > 0 ? sh_rest : nullptr;
+  auto pick = [&](auto bg) {
+    constexpr bool BG = decltype(bg)::value;
+    if (inv) return &k_geom_bwd<false, true, 9, BG>;
+    if (sh_degree > 0)
+      return grad_stride == 9 ? &k_geom_bwd<true, false, 9, BG> : &k_geom_bwd<true, false, 10, BG>;
+    return grad_stride == 9 ? &k_geom_bwd<false, false, 9, BG> : &k_geom_bwd<false, false, 10, BG>;
+  };
+  auto* fn = gw_b_raw ? pick(std::true_type{}) : pick(std::false_type{});
+  fn<<<grid, 256, 0, stream>>>(params, G, rest, sh_rest_count(sh_degree), dwa, camera, near_z, blur,
+                               grad, inv, gparams, gsh_rest, bgg);
   return launch_status();
 }
 
