@@ -1,7 +1,7 @@
-// Binned poly-splat + WSR render, forward and backward.  One 256-thread workgroup per S x S
-// tile (S = 16 or 32).  Math: tools/bh_views.py:65-71 (forward), spike/backward.py:42-58 and
-// tools/resident_traced.py:60-88 (backward + theta backward), tools/m4_train_binned.py:130-143
-// (tile-local theta_u).
+// Binned poly-splat + WSR render, forward and backward.  One workgroup per S x S tile (S = 16 or
+// 32; 256 threads, 512 in the backward of few tiles).  Math: tools/bh_views.py:65-71 (forward),
+// spike/backward.py:42-58 and tools/resident_traced.py:60-88 (backward + theta backward),
+// tools/m4_train_binned.py:130-143 (tile-local theta_u).
 //
 // Forward: the tile's valid slots are compacted into LDS as theta_u (6) and (col_o, o_col) (4);
 // each thread owns S*S/256 pixels and walks the slots:
@@ -93,6 +93,7 @@ __device__ __forceinline__ void build_slot(const float* __restrict__ proj, int g
 }
 
 // Compact the tile's valid slots into LDS in slot order.  Returns the valid count.
+template <int NT = 256>
 __device__ __forceinline__ int load_slots_proj(const float* __restrict__ proj,
                                                const int32_t* __restrict__ idx,
                                                const uint8_t* __restrict__ valid, int t, int K,
@@ -102,7 +103,7 @@ __device__ __forceinline__ int load_slots_proj(const float* __restrict__ proj,
   // valid slot's proj record is requested before the compaction scan, whose barriers then
   // overlap that round trip
   int base = 0;
-  for (int s0 = 0; s0 < K; s0 += 256) {
+  for (int s0 = 0; s0 < K; s0 += NT) {
     const int s = s0 + threadIdx.x;
     const int64_t ts = (int64_t)t * K + min(s, K - 1);
     const uint8_t vb = valid[ts];  // both loads unconditional: in flight together
@@ -116,7 +117,7 @@ __device__ __forceinline__ int load_slots_proj(const float* __restrict__ proj,
       r2 = r[2];
     }
     int total;
-    const int pos = base + block_excl_scan256(v, s_tmp, &total);
+    const int pos = base + block_excl_scan<NT>(v, s_tmp, &total);
     if (v) {
       float4 ta, tb, cl;
       slot_from_rec(r0, r1, r2, ox, oy, inv_k, ta, tb, cl);
@@ -136,12 +137,13 @@ __device__ __forceinline__ int load_slots_proj(const float* __restrict__ proj,
 // The same from slot records (rec = slot_rec [T][K][12] in dispatch order, block b reads its
 // own K records and kept count): the kept slots are the prefix [0, pos_count[b]), so no
 // compaction.  Returns the kept count.
+template <int NT = 256>
 __device__ __forceinline__ int load_slots_rec(const float* __restrict__ rec,
                                               const int32_t* __restrict__ pos_count, int K,
                                               float ox, float oy, float inv_k, SlotLDS sl,
                                               bool* bad) {
   const int nb = min(pos_count[blockIdx.x], K);
-  for (int s = threadIdx.x; s < K; s += 256) {
+  for (int s = threadIdx.x; s < K; s += NT) {
     // read whether kept or not: the loads are in flight beside pos_count
     const float4* r = reinterpret_cast<const float4*>(rec + ((int64_t)blockIdx.x * K + s) * 12);
     const float4 r0 = r[0], r1 = r[1], r2 = r[2];
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(256) void k_splat_fwd(
 // add instead of a half-rate max) r2^2 q/4 = w q and r2 (q/4)(2 C) = relu(u) q.C exactly
 // (scalings by powers of two).  WILD = true: relu_bits on unscaled q (a NaN u only occurs in tiles whose
 // den the forward made NaN, so every gradient there is NaN whatever relu gives).
-template <int S, bool FROM_PROJ, bool WILD>
+template <int S, bool FROM_PROJ, bool WILD, int NT = 256>
 __device__ __forceinline__ void bwd_contract(int n, const SlotLDS& sl, const float4* s_px,
                                              int t, int K, int ox, int oy,
                                              float inv_k, const float* __restrict__ proj,
@@ -277,8 +279,8 @@ __device__ __forceinline__ void bwd_contract(int n, const SlotLDS& sl, const flo
   // threads per slot: split rows while slots are few.  The tps threads of a slot are adjacent
   // lanes of one wave (rows h, h + tps, ...), so their partial sums combine with lane shuffles.
   int tps = 1;
-  while (tps < 16 && tps * 2 * n <= 256) tps <<= 1;
-  const int sg = 256 / tps;
+  while (tps < 16 && tps * 2 * n <= NT) tps <<= 1;
+  const int sg = NT / tps;
   const int h = threadIdx.x % tps, sl_local = threadIdx.x / tps;
   for (int c0s = 0; c0s < n; c0s += sg) {
     const int s = c0s + sl_local;
@@ -383,10 +385,11 @@ __device__ __forceinline__ void bwd_contract(int n, const SlotLDS& sl, const flo
   }
 }
 
+// NT threads: 256, or 512 (bwd_wide; the second half only loads and contracts slots).
 // REC (with FROM_PROJ): proj is slot_rec [T][K][12] in dispatch order and pos_count[b] the
 // kept count of block b's tile (load_slots_rec).
-template <int S, bool FROM_PROJ, typename OT = float, bool REC = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_splat_bwd(
+template <int S, bool FROM_PROJ, typename OT = float, bool REC = false, int NT = 256>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_splat_bwd(
     const float* __restrict__ proj, const int32_t* __restrict__ idx,
     const uint8_t* __restrict__ valid, const OT* __restrict__ theta,
     const OT* __restrict__ col, const OT* __restrict__ oc,
@@ -397,10 +400,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     float* __restrict__ gtheta, float* __restrict__ gcol, float* __restrict__ goc,
     float* __restrict__ gwb) {
   constexpr int P = S * S;
-  constexpr int PPT = P / 256;
+  constexpr int PPT = (P + NT - 1) / NT;
   extern __shared__ __attribute__((aligned(16))) unsigned char s_dyn[];
-  __shared__ int s_tmp[4];
-  __shared__ float s_ftmp[4];
+  __shared__ int s_tmp[NT / 64];
+  __shared__ float s_ftmp[NT / 64];
   const SlotLDS sl = carve_slots(s_dyn, K);
   // pixel rows padded to S + 1 entries: the tps rows read together fall in different banks
   float4* s_px = reinterpret_cast<float4*>(s_dyn + slot_lds_bytes(K) + (16 - slot_lds_bytes(K) % 16) % 16);
@@ -412,7 +415,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   float pg[PPT][3], pc[PPT][3], pd[PPT];
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    const int p = threadIdx.x + 256 * i;
+    // threads past the pixels load the last one
+    const int p = P % NT == 0 ? (int)threadIdx.x + NT * i : min((int)threadIdx.x + NT * i, P - 1);
     const int64_t pix = (int64_t)(oy + p / S) * W + ox + p % S;
     pd[i] = den[pix];
 #pragma unroll
@@ -424,9 +428,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
   int n;
   bool bad = false;  // a wild slot (theta_wild): the contraction keeps relu on unscaled terms
   if constexpr (REC) {
-    n = load_slots_rec(proj, pos_count, K, (float)ox, (float)oy, inv_k, sl, &bad);
+    n = load_slots_rec<NT>(proj, pos_count, K, (float)ox, (float)oy, inv_k, sl, &bad);
   } else if constexpr (FROM_PROJ) {
-    n = load_slots_proj(proj, idx, valid, t, K, (float)ox, (float)oy, inv_k, sl, s_tmp, &bad);
+    n = load_slots_proj<NT>(proj, idx, valid, t, K, (float)ox, (float)oy, inv_k, sl, s_tmp, &bad);
   } else {
     load_slots_theta(theta, col, oc, t, K, sl, &bad);
     n = K;
@@ -442,21 +446,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
     const float inv = __builtin_amdgcn_rcpf(pd[i]);   // hardware reciprocal, 1 ulp
     const float4 q = make_float4(pg[i][0] * inv, pg[i][1] * inv, pg[i][2] * inv,
                                  -(pg[i][0] * pc[i][0] + pg[i][1] * pc[i][1] + pg[i][2] * pc[i][2]) * inv);
-    const int p = threadIdx.x + 256 * i;
+    const int p = threadIdx.x + NT * i;
+    if (P % NT != 0 && p >= P) continue;   // (their share of dL/dw_b too)
     s_px[(p / S) * (S + 1) + p % S] = make_float4(q.x * qs, q.y * qs, q.z * qs, q.w * qs);
     wpart += q.x * bg1 + q.y * bg2 + q.z * bg3 + q.w;
   }
   if (gwb) {  // per-tile partial of dL/dw_b (summed by the caller)
-    const float tot = block_sum256(wpart, s_ftmp);
+    const float tot = block_sum<NT>(wpart, s_ftmp);
     if (threadIdx.x == 0) gwb[t] = tot;
   }
   __syncthreads();
 
   if (wild)
-    bwd_contract<S, FROM_PROJ, true>(n, sl, s_px, t, K, ox, oy, inv_k, proj, gslot, gtheta, gcol,
+    bwd_contract<S, FROM_PROJ, true, NT>(n, sl, s_px, t, K, ox, oy, inv_k, proj, gslot, gtheta, gcol,
                                      goc);
   else
-    bwd_contract<S, FROM_PROJ, false>(n, sl, s_px, t, K, ox, oy, inv_k, proj, gslot, gtheta,
+    bwd_contract<S, FROM_PROJ, false, NT>(n, sl, s_px, t, K, ox, oy, inv_k, proj, gslot, gtheta,
                                       gcol, goc);
 }
 
@@ -941,6 +946,13 @@ int launch_fwd(const float* proj, const int32_t* idx, const uint8_t* valid, cons
   return launch_status();
 }
 
+// Threads of a 16 x 16 tile's backward: up to two tiles per CU a block of 512 halves each slot's
+// rows per thread (the walk is a serial chain there); past that the GPU is full and the slot
+// prologue's extra waves cost.  Whole training steps with 256 / 512 threads (us): 64 tiles 60.9 /
+// 58.3, 256 tiles at K 256 79.7 / 74.8, 247 59.3 / 57.4, 425 67.2 / 65.9, 600 73.3 / 73.6, 2500
+// 71.5 / 76.6 (1024 threads: 58.8, 75.0, 57.9, 67.9, 76.8, 97.6).
+inline bool bwd_wide(int T) { return T <= 512; }
+
 template <bool FROM_PROJ, typename OT = float>
 int launch_bwd(const float* proj, const int32_t* idx, const uint8_t* valid, const OT* theta,
                const OT* col, const OT* oc, const int32_t* order, int H, int W, int S, int K,
@@ -950,7 +962,11 @@ int launch_bwd(const float* proj, const int32_t* idx, const uint8_t* valid, cons
                hipStream_t stream) {
   const int ntx = W / S, T = (H / S) * ntx;
   const float inv_k = (float)(1.0 / (double)k);
-  if (S == 16)
+  if (S == 16 && FROM_PROJ && bwd_wide(T))
+    k_splat_bwd<16, FROM_PROJ, OT, false, 512><<<T, 512, bwd_lds(K, 16), stream>>>(
+        proj, idx, valid, theta, col, oc, order, nullptr, ntx, W, K, inv_k, bg, image, den,
+        gimage, gslot, gtheta, gcol, goc, gwb);
+  else if (S == 16)
     k_splat_bwd<16, FROM_PROJ, OT><<<T, 256, bwd_lds(K, 16), stream>>>(
         proj, idx, valid, theta, col, oc, order, nullptr, ntx, W, K, inv_k, bg, image, den,
         gimage, gslot, gtheta, gcol, goc, gwb);
@@ -1071,7 +1087,9 @@ int tts_splat_bwd_rec(const float* slot_rec, const int32_t* pos_count, const int
   if (!slot_rec || !pos_count || !order || !bg || !image || !den || !gimage || !gslot)
     return TTS_EINVAL;
   const int ntx = W / S, T = (H / S) * ntx;
-  k_splat_bwd<16, true, float, true><<<T, 256, bwd_lds(K, 16), stream>>>(
+  auto* fn = bwd_wide(T) ? &k_splat_bwd<16, true, float, true, 512>
+                         : &k_splat_bwd<16, true, float, true>;
+  fn<<<T, bwd_wide(T) ? 512 : 256, bwd_lds(K, 16), stream>>>(
       slot_rec, nullptr, nullptr, nullptr, nullptr, nullptr, order, pos_count, ntx, W, K,
       (float)(1.0 / (double)k), bg, image, den, gimage, gslot, nullptr, nullptr, nullptr, gwb);
   return launch_status();

@@ -205,15 +205,22 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// Block-wide float sum for blockDim.x == 256; result valid in every thread.
-__device__ __forceinline__ float block_sum256(float v, float* tmp) {
+// Block-wide float sum for blockDim.x == NT, in wave order; result valid in every thread.  `tmp`
+// holds NT/64 floats.
+template <int NT>
+__device__ __forceinline__ float block_sum(float v, float* tmp) {
   v = wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) tmp[wave] = v;
   __syncthreads();
-  float s = tmp[0] + tmp[1] + tmp[2] + tmp[3];
+  float s = tmp[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) s += tmp[w];
   __syncthreads();
   return s;
+}
+__device__ __forceinline__ float block_sum256(float v, float* tmp) {
+  return block_sum<256>(v, tmp);
 }
 
 // The blend's background block out[4] = (softplus(w_b_raw), c_b r, g, b) (spike/render.py:28),
