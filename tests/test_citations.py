@@ -17,7 +17,8 @@ SKIP_PREFIX = ("SURVEY", "VERDICT", "ADVICE", "BASELINE", "BENCH_", "GPUTEST_", 
                "MULTICHIP_", "PROGRESS")
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "spike")),
+                    reason="reference checkout not present")
 def test_reference_citations_point_at_existing_lines():
     files = subprocess.run(["git", "ls-files"], cwd=ROOT, capture_output=True, text=True,
                            check=True).stdout.split()
