@@ -52,6 +52,14 @@ def test_binding_matches_header(lib):
         assert len(args) == d[name], name
 
 
+@pytest.mark.parametrize("G", [1 << 20, (1 << 30) // 40 + 1, 1 << 25, 1 << 30])
+@pytest.mark.parametrize("P", [1, 1 << 20, 1 << 30])
+def test_dense_workspace_holds_one_band_of_partials(lib, G, P):
+    """The band count falls as G grows until one band is left, whose ten floats a gaussian are past
+    the cap on the partials' size from G = 2^30 / 40 on."""
+    assert lib.tts_dense_workspace_bytes(G, P) >= 40 * G
+
+
 def test_host_only_entry_points(lib):
     assert lib.tts_version() >> 16 == 0
     assert b"tile side" in lib.tts_strerror(-2)

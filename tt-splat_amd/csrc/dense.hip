@@ -38,7 +38,7 @@ constexpr int kThetaComp = 10;  // theta 0..5, o, color r, g, b
 constexpr int kDenseTargetBlocks = 2048;
 constexpr size_t kDenseMaxWorkspace = size_t(1) << 30;
 
-// Pixels per band of the theta form's backward (a multiple of 256) for G gaussians over P pixels:
+// Pixels per band of the theta form's backward (a multiple of 256, or P) for G gaussians over P pixels:
 // up to 2048 (64 gaussians, band) blocks of 16 waves, but bands of whole 1024-pixel stagings where
 // those still give each CU two blocks.  Measured, about 512 / 1024 / 2048 blocks (us, band sums
 // included): G 2000, 128x128 26 / 28 / 34; G 6000, 100x100 45 / 43 / 45; 200x200 135 / 131 / 122;
@@ -51,8 +51,9 @@ inline int dense_band_pixels(int G, int P) {
   pb = ((pb + 255) / 256) * 256;
   if (pb < 256) pb = 256;
   if (pb < 1024 && (int64_t)gchunks * ((P + 1023) / 1024) >= 512) pb = 1024;
-  // keep the partials within the workspace cap
-  while ((size_t)((P + pb - 1) / pb) * (size_t)G * kThetaComp * 4 > kDenseMaxWorkspace) pb *= 2;
+  // keep the partials within the workspace cap, down to one band (past the cap from G = 2^30 / 40)
+  while (pb < P && (size_t)((P + pb - 1) / pb) * (size_t)G * kThetaComp * 4 > kDenseMaxWorkspace)
+    pb = pb <= P / 2 ? 2 * pb : P;
   return pb;
 }
 
