@@ -35,11 +35,12 @@ def _bg(w_b, c_b, device):
 
 
 def _keep_u8(keep):
+    """The mask's own copy: its owner may write into it before the backward reads it."""
     if keep is None:
         return None
-    if keep.dtype == torch.bool:        # a bool's bytes are 0 and 1 already
-        return keep.contiguous().view(torch.uint8)
-    return (keep != 0).to(torch.uint8).contiguous()
+    if keep.dtype != torch.bool:
+        keep = keep != 0
+    return keep.to(torch.uint8).contiguous()
 
 
 class WSRPolySplatHot(torch.autograd.Function):
