@@ -178,3 +178,20 @@ def test_backward_matches_the_general_path(G, H, W, size):
     b, _ = kernels.render_dense_bwd(everywhere(p), H, W, 4.0, bg, img, den, gi)
     # H W terms in another order; they cancel in part, so against each column's largest gradient
     assert float(((a - b).abs() / b.abs().amax(0)).max()) <= H * W * 2.0 ** -24
+
+
+def test_backward_softz_product_past_the_float_range():
+    """o_col (Z/den0) (z - z*) has three factors: where it overflows, zero weights give NaN, as
+    visiting every pair does, also for a gaussian whose support misses the image."""
+    H, W = 24, 31
+    proj = records(40, H, W, seed=2)
+    proj[7, 0:2] = -400.0
+    proj[7, 9] = 1e17
+    beta = torch.tensor([1e-17], device="cuda")
+    img, den, aux = kernels.render_dense_arm(proj.cuda(), H, W, 4.0,
+                                             torch.tensor(BG, device="cuda"), "SZ", beta)
+    aux[..., 0], aux[..., 1] = 1e17, 1e-30     # z*, den0: Z/den0 is about 1e13
+    gi = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+    got, _ = kernels.render_dense_arm_bwd(proj.cuda(), H, W, 4.0, torch.tensor(BG, device="cuda"),
+                                          "SZ", img, den, aux, gi, beta)
+    assert bool(torch.isnan(got[7, 0:5]).all())

@@ -102,14 +102,14 @@ __device__ __forceinline__ int block_id() { return (int)(blockIdx.x + gridDim.x 
 // |2b dx dy| <= a dx^2 + c dy^2), so the points lie in the ellipse of the form with a and c
 // reduced by 1e-6; 3e-5 is taken from a*c below, which also covers the rounding of a*c - b^2, and
 // 0.1 % is added to k.  No bound is given, and the gaussian is taken everywhere, when the form is
-// not positive definite by that margin, or when a value is so large (or not a number) that its
-// product with a zero weight would not be zero.
+// not positive definite by that margin, or when a value is so large (or not a number) that a
+// product it enters, times a zero weight, might not be zero.
 __device__ __forceinline__ float2 support_half(float4 r0, float4 r1, float4 r2, float kk) {
   const float a = r0.z, b = r0.w, c = r1.x;
   const float det = a * c * (1.0f - 3e-5f) - b * b;
   const bool ok = fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && a > 0.0f && a < 1e9f &&
                   c > 0.0f && c < 1e9f && det > 1e-30f &&
-                  fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e18f;
+                  fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e12f;
   const float s = kk / det;
   return ok ? make_float2(sqrtf(s * c), sqrtf(s * a)) : make_float2(INFINITY, INFINITY);
 }
@@ -122,8 +122,9 @@ __device__ __forceinline__ float quad_u(float dx, float dy, float a, float b2, f
 // k with the margin above
 __device__ __forceinline__ float support_k(float inv_k) { return 1.001f / inv_k; }
 
-// Largest magnitude that still gives zero when a zero weight multiplies it and its products.
-__device__ __forceinline__ bool tame(float v) { return fabsf(v) < 1e18f; }
+// Magnitudes whose products stay finite, so that a zero weight makes them zero: the longest is soft-Z's
+// o_col (Z/den0) (z - z*), three factors.
+__device__ __forceinline__ bool tame(float v) { return fabsf(v) < 1e12f; }
 
 // Does the box reach the pixel centres within `half` of `centre`?  (false only when it cannot:
 // an infinite extent gives true, a NaN difference too; 0.01 covers the rounding of both sides)
