@@ -111,3 +111,14 @@ def test_geometry_launches_carry_the_background(G):
     got = kernels.geom_bwd(P, camb, gslot, inv=inv)
     # the same sum and formulas, contracted by the compiler per kernel
     assert torch.allclose(got, ref, rtol=1e-4, atol=1e-5 * float(ref.abs().max()))
+
+
+def test_loss_value_of_a_tensor_weight_and_of_tracked_partials():
+    H, W = 40, 50
+    p = torch.rand(kernels.loss_partials_count(H, W)[0], device="cuda", requires_grad=True)
+    lam = torch.tensor([0.0, 0.2, 1.0], device="cuda", requires_grad=True)
+    v = kernels.loss_from_partials(p, H, W, lam)
+    one = [kernels.loss_from_partials(p.detach(), H, W, float(x)) for x in lam.detach()]
+    assert torch.allclose(v.detach(), torch.stack(one), rtol=1e-6)   # the weight in 32 bits
+    gp, gl = torch.autograd.grad(v.sum(), [p, lam])
+    assert bool((gp != 0).any()) and gl.shape == (3,)

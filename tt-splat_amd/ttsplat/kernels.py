@@ -675,10 +675,13 @@ def loss_grad_stats(image, target, stats, lam=0.2, gimage=None, partials=None):
 
 
 def loss_from_partials(partials, H, W, lam=0.2):
-    """Loss value from the partial sums written by loss_grad (a device scalar)."""
+    """Loss value from the partial sums written by loss_grad (a device scalar; shaped like lam where
+    that is a tensor)."""
     n, ns = loss_partials_count(H, W)
-    if not (partials.is_cuda and partials.dtype == F32 and partials.is_contiguous()
-            and partials.numel() == n):    # partials moved or converted by the caller
+    if not (isinstance(lam, (int, float)) and partials.is_cuda and partials.dtype == F32
+            and partials.is_contiguous() and partials.numel() == n and not partials.requires_grad
+            and partials.device.index == torch.cuda.current_device()):
+        # partials moved, converted or differentiated by the caller, a weight on the device
         l1_sum, s_sum = partials[ns:].double().sum(), partials[:ns].double().sum()
         return ((1.0 - lam) * l1_sum / (3.0 * H * W)
                 + lam * (1.0 - s_sum / (3.0 * (H - 10) * (W - 10)))).float()
