@@ -1,0 +1,43 @@
+"""The dense backward's ways through the gaussians of a block: two large boxes walked jointly, one
+large box among small ones, by one block and in shares; against autograd of the formula in 64 bits,
+and twice with the same result."""
+import pytest
+import torch
+
+from test_gpu_dense_cull import grads, oracle_detached_z, records
+
+pytestmark = pytest.mark.gpu
+
+
+# four waves per gaussian (G <= 4096, or 2^17 pixels and more), sixteen and one; cells of 8 x 8 pixels
+# cut at the image's edge; `big` every how many gaussians (1: all); thin ones (no box: condition past
+# the bound) among them
+@pytest.mark.parametrize("G,H,W,big,cond", [
+    (1, 300, 301, 1, 10.0), (3, 9, 700, 1, 10.0), (4, 64, 64, 1, 10.0), (5, 131, 77, 1, 10.0),
+    (9, 1, 1201, 1, 10.0), (40, 203, 199, 1, 30.0), (41, 333, 400, 3, 10.0),
+    (260, 150, 160, 97, 10.0), (257, 150, 103, 1, 10.0), (300, 510, 515, 40, 10.0),
+    (18, 120, 130, 2, 1e5), (4101, 97, 60, 1, 10.0), (4103, 91, 95, 600, 10.0),
+    (4102, 64, 33, 3, 10.0)])
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+def test_backward_follows_autograd(G, H, W, big, cond, arm):
+    print(f"[boxes] {G} {H}x{W} {big} {arm}", flush=True)
+    proj = records(G, H, W, seed=G, cond=10.0, size=2.0)
+    wide = records(G, H, W, seed=G + 1, cond=cond, size=1.5 * max(H, W))
+    proj[::big] = wide[::big]
+    proj[:, 6:10] *= 0.2          # revealage: many opaque layers would leave nothing to see
+    gi = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(3))
+    got, gwb = grads(proj.cuda(), H, W, arm, gi.cuda())
+    again, gwb2 = grads(proj.cuda(), H, W, arm, gi.cuda())
+    assert torch.equal(got, again) and torch.equal(gwb, gwb2)
+    P = proj.double().requires_grad_(True)
+    beta = torch.tensor(3.0, dtype=torch.float64, requires_grad=True)
+    (oracle_detached_z(P, H, W, arm, beta) * gi.double()).sum().backward()
+    ref = torch.cat([P.grad[:, 2:5], P.grad[:, 0:2], P.grad[:, 6:10]], 1)
+    # the contract of the dense gradients: 1e-3 relative L2 (u carries 12 eps cond)
+    for sl in (slice(0, 3), slice(3, 5), slice(5, 8), slice(8, 9)):
+        e = float((got[:, sl].cpu().double() - ref[:, sl]).norm() / ref[:, sl].norm())
+        print(f"  {sl.start}: {e:.2e}")
+        assert e <= 1e-3, (sl, e)
+    if arm == "SZ":
+        d = abs(float(got[:, 9].double().sum()) - float(beta.grad))
+        assert d <= 1e-3 * abs(float(beta.grad)) + 1e-5

@@ -28,6 +28,8 @@
 //        R = exp(sum log(1 - min(W, 1 - 1e-4))) (no w_b); dL/dW gains -dL/dlogR / (1 - a).
 // aux [P,4] carries the per-pixel forward state to the backward (SZ: z*, den0; RV: R, C_avg).
 
+#include <type_traits>
+
 #include "tts_common.h"
 
 namespace tts {
@@ -38,11 +40,11 @@ constexpr int kThetaComp = 10;  // theta 0..5, o, color r, g, b
 constexpr int kDenseTargetBlocks = 2048;
 constexpr size_t kDenseMaxWorkspace = size_t(1) << 30;
 
-// Pixels per band of the theta form's backward (a multiple of 256, or P) for G gaussians over P pixels:
-// up to 2048 (64 gaussians, band) blocks of 16 waves, but bands of whole 1024-pixel stagings where
-// those still give each CU two blocks.  Measured, about 512 / 1024 / 2048 blocks (us, band sums
-// included): G 2000, 128x128 26 / 28 / 34; G 6000, 100x100 45 / 43 / 45; 200x200 135 / 131 / 122;
-// G 2000, 600x600 360 / 350 / 346.
+// Pixels per band of the theta form's backward (a multiple of 256, or P) for G gaussians over P
+// pixels: up to 2048 (64 gaussians, band) blocks of 16 waves, but bands of whole 1024-pixel
+// stagings where those still give each CU two blocks.  Measured, about 512 / 1024 / 2048 blocks
+// (us, band sums included): G 2000, 128x128 26 / 28 / 34; G 6000, 100x100 45 / 43 / 45; 200x200 135
+// / 131 / 122; G 2000, 600x600 360 / 350 / 346.
 inline int dense_band_pixels(int G, int P) {
   const int gchunks = (G + 63) / 64;
   int nb = kDenseTargetBlocks / (gchunks > 0 ? gchunks : 1);
@@ -67,19 +69,25 @@ inline size_t theta_ws_bytes(int G, int P) {
   return 256 + pad256(nb * 4) + nb * (size_t)G * kThetaComp * 4;
 }
 
-// Workspace of the quad form: [align to 256][gwb partials, kPreBlocks floats][wild flags,
-// kPreBlocks + 1 ints, padded to 256][per-pixel gradients, P float4][arm extras, P float2, padded]
-// [row-share partials, shares*G*(kQuadComp + 1), when there is more than one share].
 constexpr int kPreBlocks = 256;
 
-// Row shares of a gaussian's box in the backward: few gaussians over a large image would leave
-// most of the GPU idle (four waves per gaussian and share).  G 1, 20, 100 over 800x800, every pixel
-// in the box: 68, 71 and 217 us.
-inline int quad_shares(int G) { return G >= 256 ? 1 : (G >= 64 ? 4 : 16); }
+// Workspace of the quad form: [align to 256][gwb partials, kPreBlocks floats][wild flags,
+// kPreBlocks + 1 ints, padded to 256][per-pixel gradients, P float4][arm extras, P float2, padded]
+// [the shares' gradients, shares*G*(kQuadComp + 1), when there is more than one share].
+//
+// Shares of a gaussian's box in the backward: few gaussians over a large image would leave most of
+// the GPU idle, and from 256 on the sum of the shares costs more than it gives.  Every box the
+// whole image, shares as here / 16 below 64 gaussians and 4 below 256 (us): G 1, 800x800 44 / 65; G
+// 100 62 / 216; G 255, 400x400 42 / 67.
+inline int quad_shares(int G, int P) {
+  if (G >= 256) return 1;
+  const int by_g = 1024 / G, by_p = P / 1024, n = by_g < by_p ? by_g : by_p;
+  return n < 1 ? 1 : (n > 16 ? 16 : n);
+}
 
 inline size_t quad_ws_bytes(int G, int P) {
   if (G <= 0 || P <= 0) return 0;
-  const size_t sh = (size_t)quad_shares(G);
+  const size_t sh = (size_t)quad_shares(G, P);
   return 256 + kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4) + pad256((size_t)P * 16) +
          pad256((size_t)P * 8) + (sh > 1 ? sh * (size_t)G * (kQuadComp + 1) * 4 : 0);
 }
@@ -104,12 +112,15 @@ __device__ __forceinline__ int block_id() { return (int)(blockIdx.x + gridDim.x 
 // 0.1 % is added to k.  No bound is given, and the gaussian is taken everywhere, when the form is
 // not positive definite by that margin, or when a value is so large (or not a number) that a
 // product it enters, times a zero weight, might not be zero.
+__device__ __forceinline__ bool calm_record(float4 r0, float4 r1, float4 r2) {
+  return fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && fabsf(r0.z) < 1e9f && fabsf(r0.w) < 1e9f &&
+         fabsf(r1.x) < 1e9f &&
+         fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e12f;
+}
 __device__ __forceinline__ float2 support_half(float4 r0, float4 r1, float4 r2, float kk) {
   const float a = r0.z, b = r0.w, c = r1.x;
   const float det = a * c * (1.0f - 3e-5f) - b * b;
-  const bool ok = fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && a > 0.0f && a < 1e9f &&
-                  c > 0.0f && c < 1e9f && det > 1e-30f &&
-                  fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e12f;
+  const bool ok = calm_record(r0, r1, r2) && a > 0.0f && c > 0.0f && det > 1e-30f;
   const float s = kk / det;
   return ok ? make_float2(sqrtf(s * c), sqrtf(s * a)) : make_float2(INFINITY, INFINITY);
 }
@@ -119,11 +130,17 @@ __device__ __forceinline__ float quad_u(float dx, float dy, float a, float b2, f
   const float Q = __builtin_fmaf(__builtin_fmaf(a, dx, b2 * dy), dx, (c * dy) * dy);
   return __builtin_fmaf(-Q, inv_k, 1.0f);
 }
+// The same with the row's b2 dy and (c dy) dy at hand.
+__device__ __forceinline__ float quad_u_row(float dx, float a, float b2dy, float cdy2,
+                                            float inv_k) {
+  const float Q = __builtin_fmaf(__builtin_fmaf(a, dx, b2dy), dx, cdy2);
+  return __builtin_fmaf(-Q, inv_k, 1.0f);
+}
 // k with the margin above
 __device__ __forceinline__ float support_k(float inv_k) { return 1.001f / inv_k; }
 
-// Magnitudes whose products stay finite, so that a zero weight makes them zero: the longest is soft-Z's
-// o_col (Z/den0) (z - z*), three factors.
+// Magnitudes whose products stay finite, so that a zero weight makes them zero: the longest is
+// soft-Z's o_col (Z/den0) (z - z*), three factors.
 __device__ __forceinline__ bool tame(float v) { return fabsf(v) < 1e12f; }
 
 // Does the box reach the pixel centres within `half` of `centre`?  (false only when it cannot:
@@ -546,42 +563,133 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
   }
 }
 
-// Quad backward, pass 2: WPG waves per gaussian (and row share) walk the pixels of its support
-// box, one pixel per lane, and sum its gradients over lanes and waves in a fixed order.
-// ncomp = 9 (a, b, c, mu_x, mu_y, col_o rgb, o_col), 10 for SZ (+ this gaussian's dL/dbeta).
-// Bound by the latency of a wave's few dependent steps (record, box, two to ten rounds of pixel
-// loads, lane sums); on large images by L2 reads of q (16 bytes a pair).  One thread per gaussian
-// over every pixel, bands of pixels staged in LDS, took 43 us at G 2000, 128x128, 472 at G 10000,
-// 300x300 and 3061 at 800x800 (soft-Z 296, 2994, 15818), its band sums included; this takes 19,
-// 25 and 85 (soft-Z 23, 63, 189).  That form is the faster one only where the support boxes fill
-// over half of the image on average (every box the whole image, G 2000, 400x400: 226 against 340).
-template <int ARM, int WPG>
-__global__ __launch_bounds__(256) void k_render_dense_bwd(
+// Quad backward, pass 2: the pixels of the gaussians' support boxes, one pixel per lane, sums over
+// lanes, waves and blocks in a fixed order.  ncomp = 9 (a, b, c, mu_x, mu_y, col_o rgb, o_col), 10
+// for SZ (+ this gaussian's dL/dbeta).
+//
+// A block serves GPB gaussians with WPG waves each.  Where every box is small each gaussian's waves
+// walk its box: bound by the latency of a few dependent steps (record, box, two to ten rounds of
+// pixel loads, lane sums).  Otherwise all the block's waves walk one box after another, or, where
+// two gaussians' boxes fill most of their union, both jointly: the waves deal out its 8 x 8 pixel
+// cells and evaluate the pair on each, a lane staying in its row.  The pixel's 16-byte load, its
+// coordinates and the loop are then paid once for two gaussians and the row's terms once per row:
+// 20 VALU instructions a pixel and gaussian, which bound it (a box by itself: about 40, and 16
+// bytes of L2 reads).  Only for calm records (no value whose product with a zero weight might not
+// be zero). gridDim.y > 1 (few gaussians): each row of blocks takes a share of every box, or of the
+// cells, and writes its own gradients; k_dense_reduce adds them.
+//
+// Whole arm-A backward in us, against one thread per gaussian over every pixel (bands of pixels
+// staged in LDS, band sums): small boxes, G 2000, 128x128 19 (that form 43), G 10000, 300x300 25
+// (472), 800x800 85 (3061); every box the whole image, G 2000, 128x128 28 (41), 400x400 177 (224),
+// G 10000, 300x300 481 (466); a whole-image box among 256 small ones, 800x800 223 (391), among
+// 10000 427 (3000).  Each box by itself always, by its own waves: 43, 333, 867, 791, 808.  Soft-Z,
+// every box the whole image: 118 (295), 992 (1004), G 4000, 400x400 1925 (1862).
+struct Gauss {
+  float mx, my, a, b, c, z, cr, cg, cb, oc;
+};
+// (a uniform index: scalar loads)
+__device__ __forceinline__ Gauss gauss(const float* __restrict__ proj, int64_t g) {
+  const float* r = proj + g * 12;
+  return {r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8], r[9]};
+}
+template <int ARM>
+struct PairSums {
+  float r = 0.f, g = 0.f, b = 0.f, o = 0.f, beta = 0.f;   // dL/d col_o, o_col, softz_beta
+};
+// Adds one pair's colour, density (and soft-Z beta) terms; returns its dL/dw_geo.
+template <int ARM>
+__device__ __forceinline__ float pair_grad(PairSums<ARM>& s, float w, float4 q, float2 e,
+                                           const Gauss& gs, float beta) {
+  const float oc = gs.oc, zg = gs.z;
+  const float gw = q.x * gs.cr + q.y * gs.cg + q.z * gs.cb + q.w * oc;  // dL/dw_geo of arm A
+  if (ARM == kArmSZ) {   // e: z*, Z/den0
+    const float h = sigmoidf_(-beta * (zg - e.x));
+    const float t = e.y * (zg - e.x);  // dL/dW0 through z*
+    s.r += w * h * q.x;
+    s.g += w * h * q.y;
+    s.b += w * h * q.z;
+    s.o += w * (h * q.w + t);
+    s.beta -= w * gw * h * (1.0f - h) * (zg - e.x);
+    return h * gw + oc * t;
+  }
+  s.r += w * q.x;
+  s.g += w * q.y;
+  s.b += w * q.z;
+  if (ARM == kArmRV) {   // e.x: dL/dlogR
+    const float W0 = w * oc;
+    const float t = W0 <= 1.0f - 1e-4f ? -e.x / (1.0f - W0) : 0.0f;  // clamp gate
+    s.o += w * (q.w + t);
+    return gw + oc * t;
+  }
+  s.o += w * q.w;
+  return gw;
+}
+
+template <int ARM>
+__device__ __forceinline__ float2 pixel_extra(const float2* __restrict__ ex, int64_t p) {
+  return ARM == kArmRV ? make_float2(ex[p].x, 0.0f) : ex[p];
+}
+
+// Two gaussians are walked jointly where that visits 4 / 5 of the pixels of their boxes or less (a
+// visit costs a pair half of what it does alone, but twice the sums at the end), from boxes of 8192
+// pixels in all on.
+__device__ __forceinline__ bool joint_pays(int cells, int64_t pix) {
+  return pix > 8192 && (int64_t)cells * 80 <= pix;
+}
+
+// The 8 x 8 cells of the union of the boxes in lanes j and j + 1: from pixel (x0, y0), up to (x1,
+// y1).
+struct Cells {
+  int x0, x1, y0, y1, cols, rows;
+};
+__device__ __forceinline__ Cells pair_cells(int x0, int x1, int y0, int y1, int j) {
+  Cells u;
+  u.x0 = min(__builtin_amdgcn_readlane(x0, j), __builtin_amdgcn_readlane(x0, j + 1)) & ~7;
+  u.x1 = max(__builtin_amdgcn_readlane(x1, j), __builtin_amdgcn_readlane(x1, j + 1));
+  u.y0 = min(__builtin_amdgcn_readlane(y0, j), __builtin_amdgcn_readlane(y0, j + 1));
+  u.y1 = max(__builtin_amdgcn_readlane(y1, j), __builtin_amdgcn_readlane(y1, j + 1));
+  u.cols = (u.x1 - u.x0 + 7) / 8;
+  u.rows = (u.y1 - u.y0 + 7) / 8;
+  return u;
+}
+
+template <int ARM, int GPB, int WPG>
+__global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
     const float* __restrict__ proj, int G, int W, int H, float inv_k, int cull,
     const float* __restrict__ szb, const float4* __restrict__ qbuf, const float2* __restrict__ ex,
     const int* __restrict__ wild, int n_pre, int n_wild, const float* __restrict__ gwb_part,
     float* __restrict__ out, float* __restrict__ gwb) {
   constexpr int NC = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
-  __shared__ float s_sum[4][NC];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = wave % WPG;
-  const int64_t g = (int64_t)block_id() * (4 / WPG) + wave / WPG;
+  constexpr int NW = GPB * WPG, NV = GPB * NC;
+  // not for soft-Z, whose exponential is most of a pair either way (5 % gained jointly, for 48
+  // registers more)
+  constexpr bool kShared = GPB > 1 && ARM != kArmSZ;
+  static_assert(NV <= 64 && (GPB & (GPB - 1)) == 0, "one wave finishes");
+  __shared__ float s_sum[NW][NV];
+  __shared__ float s_tot[NV];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // a scalar to the compiler
+  int share = blockIdx.y, shares = gridDim.y;
+  const int64_t g0 = (int64_t)block_id() * GPB;
+  if (g0 >= G) return;
+  // lane GPB i + j holds gaussian j of the block
+  const int64_t g = g0 + (lane & (GPB - 1));
   const bool act = g < G;
   const float4* rec = reinterpret_cast<const float4*>(proj + min(g, (int64_t)G - 1) * 12);
   const float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+  const Gauss own = gauss(proj, min(g0 + wave / WPG, (int64_t)G - 1));
   int any = 0;
   for (int i = lane; i < n_wild; i += 64) any |= wild[i];
   if (__ballot(any != 0)) cull = 0;
-  if (block_id() == 0 && blockIdx.y == 0 && wave == 0 && gwb) {
+  if (g0 == 0 && share == 0 && wave == 0 && gwb) {
     float t = 0.0f;
     for (int i = lane; i < n_pre; i += 64) t += gwb_part[i];
     t = wave_sum(t);
     if (lane == 0) gwb[0] = t;
   }
-  const float mx = r0.x, my = r0.y, a = r0.z, b = r0.w, c = r1.x, zg = r1.y;
-  const float cr = r1.z, cg = r1.w, cb = r2.x, oc = r2.y;
+  out += ((int64_t)share * G + g0) * NC;
+  const float mx = r0.x, my = r0.y;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
-  const float b2 = 2.0f * b;
   // pixels [x0, x1) x [y0, y1): centres within the box; fminf / fmaxf turn an infinite box (and
   // the NaN of an infinite mean less an infinite extent) into the whole image
   int x0 = 0, x1 = W, y0 = 0, y1 = H;
@@ -592,110 +700,221 @@ __global__ __launch_bounds__(256) void k_render_dense_bwd(
     x1 = (int)fmaxf(fminf(floorf(mx + e.x - 0.49f) + 1.0f, (float)W), (float)x0);
     y1 = (int)fmaxf(fminf(floorf(my + e.y - 0.49f) + 1.0f, (float)H), (float)y0);
   }
-  const int rows = y1 - y0;
-  y1 = y0 + (int)((int64_t)rows * (blockIdx.y + 1) / gridDim.y);
-  y0 = y0 + (int)((int64_t)rows * blockIdx.y / gridDim.y);
-  const int bw = x1 - x0, n = act ? bw * (y1 - y0) : 0;
-  constexpr int S = 64 * WPG;
-  float sxx = 0.f, sxy = 0.f, syy = 0.f, sx = 0.f, sy = 0.f;
-  float gr = 0.f, gg = 0.f, gbl = 0.f, go = 0.f, gbeta = 0.f;
-  int i = sub * 64 + lane;
-  if (i < n) {
-    // this lane's pixel, stepped by S pixels in box order without dividing again
-    int x = i % bw, y = i / bw;
-    const int dxs = S % bw, dys = S / bw;
-    int64_t p = (int64_t)(y0 + y) * W + x0 + x;
-    float4 q = qbuf[p];
-    float2 e = ARM != kArmA ? ex[p] : make_float2(0.f, 0.f);
-    while (true) {
-      const float dx = (float)(x0 + x) + 0.5f - mx, dy = (float)(y0 + y) + 0.5f - my;
-      const float4 qc = q;
-      const float2 ec = e;
-      i += S;
-      if (i < n) {   // the next pixel's loads, in flight during this one
-        x += dxs;
-        y += dys;
-        if (x >= bw) {
-          x -= bw;
-          ++y;
+  const int n_pix = act ? (x1 - x0) * (y1 - y0) : 0;
+  if (n_pix == 0) x0 = x1 = y0 = y1 = 0;
+  // the pairs to be walked jointly; boxes of 32 rounds of their own waves and more are for all
+  // waves
+  int joint = 0;
+  if (kShared && __ballot(n_pix > 4096)) {
+    const bool calm = calm_record(r0, r1, r2) && inv_k < INFINITY;
+#pragma unroll
+    for (int j = 0; j < GPB; j += 2) {
+      const int n0 = __builtin_amdgcn_readlane(n_pix, j);
+      const int n1 = __builtin_amdgcn_readlane(n_pix, j + 1);
+      const Cells u = pair_cells(x0, x1, y0, y1, j);
+      if (n0 > 0 && n1 > 0 && joint_pays(u.cols * u.rows, (int64_t)n0 + n1) &&
+          __builtin_amdgcn_readlane((int)calm, j) && __builtin_amdgcn_readlane((int)calm, j + 1))
+        joint |= 1 << j;
+    }
+  }
+  const bool large = kShared && (joint || __ballot(n_pix > 8192));
+  if (shares > 1 && !__ballot(n_pix > 1024)) {   // not worth sharing
+    if (share > 0) {
+      if (threadIdx.x < NV && g0 + threadIdx.x / NC < G) out[threadIdx.x] = 0.0f;
+      return;
+    }
+    shares = 1;
+  }
+
+  // sums of gaussian j over every parts-th run of 64 pixels of its box, from run `part` on
+  auto walk = [&](const Gauss& h, int j, int part, int parts, float (&v)[10]) {
+    // (lanes are read while every one is active)
+    const int bx = __builtin_amdgcn_readlane(x0, j), by = __builtin_amdgcn_readlane(y0, j);
+    const int bw = __builtin_amdgcn_readlane(x1, j) - bx;
+    const int jn = __builtin_amdgcn_readlane(n_pix, j);
+    PairSums<ARM> ps;
+    float sxx = 0.f, sxy = 0.f, syy = 0.f, sx = 0.f, sy = 0.f;
+    int i = 64 * part + lane;
+    if (i < jn) {
+      // this lane's pixel, stepped by S pixels in box order without dividing again
+      const int S = 64 * parts, dxs = S % bw, dys = S / bw;
+      int x = i % bw, y = i / bw;
+      int64_t p = (int64_t)(by + y) * W + bx + x;
+      float4 q = qbuf[p];
+      float2 e = ARM != kArmA ? pixel_extra<ARM>(ex, p) : make_float2(0.f, 0.f);
+      while (true) {
+        const float dx = (float)(bx + x) + 0.5f - h.mx, dy = (float)(by + y) + 0.5f - h.my;
+        const float4 qc = q;
+        const float2 ec = e;
+        i += S;
+        if (i < jn) {   // the next pixel's loads, in flight during this one
+          x += dxs;
+          y += dys;
+          if (x >= bw) {
+            x -= bw;
+            ++y;
+          }
+          p = (int64_t)(by + y) * W + bx + x;
+          q = qbuf[p];
+          if (ARM != kArmA) e = pixel_extra<ARM>(ex, p);
         }
-        p = (int64_t)(y0 + y) * W + x0 + x;
-        q = qbuf[p];
-        if (ARM != kArmA) e = ex[p];
+        const float r = relu_nan(quad_u(dx, dy, h.a, 2.0f * h.b, h.c, inv_k));
+        const float gu = r * pair_grad<ARM>(ps, r * r, qc, ec, h, beta);
+        const float tx = gu * dx, ty = gu * dy;
+        sxx += tx * dx;
+        sxy += tx * dy;
+        syy += ty * dy;
+        sx += tx;
+        sy += ty;
+        if (i >= jn) break;
       }
-      const float r = relu_nan(quad_u(dx, dy, a, b2, c, inv_k));
-      const float w = r * r;
-      const float gw = qc.x * cr + qc.y * cg + qc.z * cb + qc.w * oc;  // dL/dw_geo of arm A
-      float dw;                                                       // dL/dw_geo of this arm
-      if (ARM == kArmSZ) {   // ec: z*, Z/den0
-        const float h = sigmoidf_(-beta * (zg - ec.x));
-        const float t = ec.y * (zg - ec.x);  // dL/dW0 through z*
-        gr += w * h * qc.x;
-        gg += w * h * qc.y;
-        gbl += w * h * qc.z;
-        go += w * (h * qc.w + t);
-        gbeta -= w * gw * h * (1.0f - h) * (zg - ec.x);
-        dw = h * gw + oc * t;
-      } else if (ARM == kArmRV) {   // ec.x: dL/dlogR
-        const float W0 = w * oc;
-        const float t = W0 <= 1.0f - 1e-4f ? -ec.x / (1.0f - W0) : 0.0f;  // clamp gate
-        gr += w * qc.x;
-        gg += w * qc.y;
-        gbl += w * qc.z;
-        go += w * (qc.w + t);
-        dw = gw + oc * t;
-      } else {
-        gr += w * qc.x;
-        gg += w * qc.y;
-        gbl += w * qc.z;
-        go += w * qc.w;
-        dw = gw;
+    }
+    v[0] = sxx; v[1] = sxy; v[2] = syy; v[3] = sx; v[4] = sy;
+    v[5] = ps.r; v[6] = ps.g; v[7] = ps.b; v[8] = ps.o; v[9] = ps.beta;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) v[k] = wave_sum(v[k]);
+  };
+  // lane k < NC writes component k of gaussian j from its sums v (of all lanes)
+  auto finish = [&](const Gauss& h, int j, const float (&v)[10]) {
+    // dL/dQ = dL/du * (-1/k) = -2 gu / k
+    const float s = -2.0f * inv_k;
+    const float m_x = s * v[3], m_y = s * v[4];
+    float o = s * v[0];                                           // dQ/da = dx^2
+    o = lane == 1 ? 2.0f * (s * v[1]) : o;                        // dQ/db = 2 dx dy
+    o = lane == 2 ? s * v[2] : o;                                 // dQ/dc = dy^2
+    o = lane == 3 ? -2.0f * (h.a * m_x + h.b * m_y) : o;            // dQ/dmu_x = -2 (a dx + b dy)
+    o = lane == 4 ? -2.0f * (h.b * m_x + h.c * m_y) : o;            // dQ/dmu_y = -2 (b dx + c dy)
+#pragma unroll
+    for (int k = 5; k < NC; ++k) o = lane == k ? v[k] : o;
+    if (lane < NC && g0 + j < G) out[j * NC + lane] = o;
+  };
+
+  float v[10];
+  if (!large) {   // each gaussian's waves walk its box
+    const int j = wave / WPG, sub = wave % WPG;
+    walk(own, j, WPG * share + sub, WPG * shares, v);
+    if (WPG > 1) {
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) s_sum[wave][k] = v[k];
       }
-      const float gu = r * dw;  // half of dL/du
-      const float tx = gu * dx, ty = gu * dy;
-      sxx += tx * dx;
-      sxy += tx * dy;
-      syy += ty * dy;
-      sx += tx;
-      sy += ty;
-      if (i >= n) break;
+      __syncthreads();
+      if (sub != 0) return;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        float t = s_sum[wave][k];
+#pragma unroll
+        for (int w = 1; w < WPG; ++w) t += s_sum[wave + w][k];
+        v[k] = t;
+      }
+    }
+    finish(own, j, v);
+    return;
+  }
+
+  // all waves walk one pair, or one box, after another
+  const int part = NW * share + wave, parts = NW * shares;
+  for (int j0 = 0; j0 < GPB; j0 += 2) {
+    if (joint >> j0 & 1) {
+      const Cells u = pair_cells(x0, x1, y0, y1, j0);
+      const Gauss h[2] = {gauss(proj, g0 + j0), gauss(proj, g0 + j0 + 1)};   // (both have pixels)
+      PairSums<ARM> ps[2];
+      float sxx[2] = {}, sxy[2] = {}, syy[2] = {}, sx[2] = {}, sy[2] = {};
+      const int cells = u.cols * u.rows;
+      int i = (int)((int64_t)cells * part / parts);
+      const int i1 = (int)((int64_t)cells * (part + 1) / parts);
+      int band = i / u.cols, col = i - band * u.cols;
+      while (i < i1) {   // cells [i, i + m) of one band of 8 rows
+        const int m = min(i1 - i, u.cols - col);
+        const int y = u.y0 + band * 8 + (lane >> 3);
+        const bool row = y < u.y1;
+        int x = u.x0 + col * 8 + (lane & 7);
+        const float yf = (float)y + 0.5f;
+        float dy[2], bd[2], cd[2], s0[2], s1[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          dy[j] = yf - h[j].my;
+          bd[j] = (2.0f * h[j].b) * dy[j];
+          cd[j] = (h[j].c * dy[j]) * dy[j];
+          s0[j] = s1[j] = 0.0f;
+        }
+        int64_t p = (int64_t)y * W + x;
+        float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+        float2 e = make_float2(0.f, 0.f);
+        if (row && x < u.x1) {
+          q = qbuf[p];
+          if (ARM != kArmA) e = pixel_extra<ARM>(ex, p);
+        }
+        for (int k = 0; k < m; ++k) {
+          const float4 qc = q;
+          const float2 ec = e;
+          const bool in = row && x < u.x1;
+          const float xf = (float)x + 0.5f;
+          x += 8;
+          p += 8;
+          if (k + 1 < m && row && x < u.x1) {   // the next cell's loads, in flight during this one
+            q = qbuf[p];
+            if (ARM != kArmA) e = pixel_extra<ARM>(ex, p);
+          }
+          if (in) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              const float dx = xf - h[j].mx;
+              // calm: no NaN; gu is half of dL/du
+              const float r = fmaxf(quad_u_row(dx, h[j].a, bd[j], cd[j], inv_k), 0.0f);
+              const float gu = r * pair_grad<ARM>(ps[j], r * r, qc, ec, h[j], beta);
+              const float tx = gu * dx;
+              s0[j] += gu;
+              s1[j] += tx;
+              sxx[j] += tx * dx;
+            }
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {   // the row's dy
+          const float t = dy[j] * s0[j];
+          sx[j] += s1[j];
+          sy[j] += t;
+          sxy[j] += dy[j] * s1[j];
+          syy[j] += dy[j] * t;
+        }
+        i += m;
+        col = 0;
+        ++band;
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float sum[10] = {sxx[j], sxy[j], syy[j], sx[j], sy[j],
+                             ps[j].r, ps[j].g, ps[j].b, ps[j].o, 0.f};
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+          const float t = wave_sum(sum[k]);
+          if (lane == 0) s_sum[wave][(j0 + j) * NC + k] = t;
+        }
+      }
+      continue;
+    }
+    for (int j = j0; j < min(j0 + 2, GPB); ++j) {
+      walk(gauss(proj, min(g0 + j, (int64_t)G - 1)), j, part, parts, v);
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) s_sum[wave][j * NC + k] = v[k];
+      }
     }
   }
-  float v[NC] = {sxx, sxy, syy, sx, sy, gr, gg, gbl, go};
-  if (ARM == kArmSZ) v[NC - 1] = gbeta;
+  __syncthreads();
+  if (threadIdx.x < NV) {
+    float t = s_sum[0][threadIdx.x];
 #pragma unroll
-  for (int k = 0; k < NC; ++k) v[k] = wave_sum(v[k]);
-  if (WPG > 1) {
-    if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < NC; ++k) s_sum[wave][k] = v[k];
-    }
-    __syncthreads();
-    const int w0 = wave / WPG * WPG;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      float t = s_sum[w0][k];
-#pragma unroll
-      for (int j = 1; j < WPG; ++j) t += s_sum[w0 + j][k];
-      v[k] = t;
-    }
+    for (int w = 1; w < NW; ++w) t += s_sum[w][threadIdx.x];
+    s_tot[threadIdx.x] = t;
   }
-  if (!act || sub != 0 || lane >= NC) return;
-  // dL/dQ = dL/du * (-1/k) = -2 gu / k
-  const float s = -2.0f * inv_k;
-  const float mxx = s * v[0], mxy = s * v[1], myy = s * v[2], m_x = s * v[3], m_y = s * v[4];
-  float r[NC];
-  r[0] = mxx;                          // dQ/da = dx^2
-  r[1] = 2.0f * mxy;                   // dQ/db = 2 dx dy
-  r[2] = myy;                          // dQ/dc = dy^2
-  r[3] = -2.0f * (a * m_x + b * m_y);  // dQ/dmu_x = -2 (a dx + b dy)
-  r[4] = -2.0f * (b * m_x + c * m_y);  // dQ/dmu_y = -2 (b dx + c dy)
+  __syncthreads();
+  if (wave < GPB) {
 #pragma unroll
-  for (int k = 5; k < NC; ++k) r[k] = v[k];
-  float o = r[0];
-#pragma unroll
-  for (int k = 1; k < NC; ++k) o = lane == k ? r[k] : o;
-  out[((int64_t)blockIdx.y * G + g) * NC + lane] = o;
+    for (int k = 0; k < NC; ++k) v[k] = s_tot[wave * NC + k];
+    finish(gauss(proj, min(g0 + wave, (int64_t)G - 1)), wave, v);
+  }
 }
 
 // theta form, backward: a block owns 64 gaussians (one per lane) and a band of pixels, 1024 of
@@ -808,6 +1027,17 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense_bwd(
   }
 }
 
+template <int N>
+__device__ __forceinline__ void add_bands(const float*& src, int64_t stride, int& left, float& s) {
+  float v[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b) v[b] = src[b * stride];
+#pragma unroll
+  for (int b = 0; b < N; ++b) s += v[b];
+  src += N * stride;
+  left -= N;
+}
+
 // out[g][c] = sum over bands of part[band][g][c], in band order; gwb = sum of gwb_part.
 __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ part, int nb,
                                                       int G, int ncomp,
@@ -818,8 +1048,13 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
   const int64_t n = (int64_t)G * ncomp;
   if (i < n) {
     float s = 0.f;
-#pragma unroll 8
-    for (int b = 0; b < nb; ++b) s += part[(int64_t)b * n + i];
+    const float* src = part + i;
+    int left = nb;   // bands in order, 16 loads in flight, then 8, 4, 2, 1
+    while (left >= 16) add_bands<16>(src, n, left, s);
+    if (left >= 8) add_bands<8>(src, n, left, s);
+    if (left >= 4) add_bands<4>(src, n, left, s);
+    if (left >= 2) add_bands<2>(src, n, left, s);
+    if (left) add_bands<1>(src, n, left, s);
     out[i] = s;
   }
   if (blockIdx.x == 0 && threadIdx.x < 64 && gwb) {   // wave 0: lanes over the bands
@@ -902,15 +1137,22 @@ int launch_dense_bwd(const float* proj, int G, int H, int W, float ik, const flo
       k_softz_pre<8, 512><<<grid, 512, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
                                                     wild + npre);
   }
-  const int sh = quad_shares(G), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
+  const int sh = quad_shares(G, P), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
   float* dst = sh > 1 ? part : grad;
   const int nw = npre + (ARM == kArmSZ ? 1 : 0);
-  if (dense_wide(G, P))
-    k_render_dense_bwd<ARM, 4><<<grid_split(G, sh), 256, 0, stream>>>(
+  auto launch = [&](auto gpb, auto wpg) {
+    constexpr int GPB = decltype(gpb)::value, WPG = decltype(wpg)::value;
+    const dim3 grid = grid_split(((int64_t)G + GPB - 1) / GPB, sh);
+    k_render_dense_bwd<ARM, GPB, WPG><<<grid, 64 * GPB * WPG, 0, stream>>>(
         proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
+  };
+  using std::integral_constant;
+  if (G >= 256 && G < 512 && P >= (1 << 18))
+    launch(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+  else if (!dense_wide(G, P))
+    launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
   else
-    k_render_dense_bwd<ARM, 1><<<grid_split(((int64_t)G + 3) / 4, sh), 256, 0, stream>>>(
-        proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
+    launch(integral_constant<int, ARM == kArmSZ ? 1 : 2>{}, integral_constant<int, 4>{});
   if (sh > 1)
     k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, sh, G, nc, nullptr,
                                                                     grad, nullptr);
