@@ -4,14 +4,14 @@ and twice with the same result."""
 import pytest
 import torch
 
-from test_gpu_dense_cull import grads, oracle_detached_z, records
+from test_gpu_dense_cull import grads, oracle, oracle_detached_z, records, render
 
 pytestmark = pytest.mark.gpu
 
 
-# four waves per gaussian (G <= 4096, or 2^17 pixels and more), sixteen and one; cells of 8 x 8 pixels
-# cut at the image's edge; `big` every how many gaussians (1: all); thin ones (no box: condition past
-# the bound) among them
+# four waves per gaussian (G <= 4096, or 2^17 pixels and more), sixteen and one; cells of 8 x 8
+# pixels cut at the image's edge; `big` every how many gaussians (1: all); thin ones (no box:
+# condition past the bound) among them
 @pytest.mark.parametrize("G,H,W,big,cond", [
     (1, 300, 301, 1, 10.0), (3, 9, 700, 1, 10.0), (4, 64, 64, 1, 10.0), (5, 131, 77, 1, 10.0),
     (9, 1, 1201, 1, 10.0), (40, 203, 199, 1, 30.0), (41, 333, 400, 3, 10.0),
@@ -41,3 +41,20 @@ def test_backward_follows_autograd(G, H, W, big, cond, arm):
     if arm == "SZ":
         d = abs(float(got[:, 9].double().sum()) - float(beta.grad))
         assert d <= 1e-3 * abs(float(beta.grad)) + 1e-5
+
+
+# every pair visited (up to 2, 8, 16 and 32 gaussians by arm and size); tiles of 16 with 256, 512
+# and 1024 threads, of 32 and of 8; lists of whole-image boxes with a small or thin one in between
+@pytest.mark.parametrize("G,H,W", [(2, 31, 9), (8, 40, 33), (16, 257, 3), (17, 60, 70),
+                                   (32, 263, 259), (33, 263, 259), (129, 257, 264), (130, 401, 330),
+                                   (300, 262, 258), (257, 529, 512), (70, 513, 520),
+                                   (1100, 70, 90)])
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+def test_forward_of_large_boxes_follows_the_formula(G, H, W, arm):
+    print(f"[boxes-fwd] {G} {H}x{W} {arm}", flush=True)
+    proj = records(G, H, W, seed=G, cond=10.0, size=1.5 * max(H, W))
+    proj[::37] = records(G, H, W, seed=G + 1, cond=1e5, size=30.0)[::37]
+    proj[:, 6:10] *= 0.1
+    # u carries 12 eps (a dx^2 + c dy^2) / k
+    ref = oracle(proj, H, W, arm)
+    assert float((render(proj.cuda(), H, W, arm).cpu() - ref).abs().max()) <= 1e-4

@@ -112,17 +112,20 @@ __device__ __forceinline__ int block_id() { return (int)(blockIdx.x + gridDim.x 
 // 0.1 % is added to k.  No bound is given, and the gaussian is taken everywhere, when the form is
 // not positive definite by that margin, or when a value is so large (or not a number) that a
 // product it enters, times a zero weight, might not be zero.
+__device__ __forceinline__ float2 support_half(float4 r0, float4 r1, float4 r2, float kk) {
+  const float a = r0.z, b = r0.w, c = r1.x;
+  const float det = a * c * (1.0f - 3e-5f) - b * b;
+  const bool ok = fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && a > 0.0f && a < 1e9f &&
+                  c > 0.0f && c < 1e9f && det > 1e-30f &&
+                  fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e12f;
+  const float s = kk / det;
+  return ok ? make_float2(sqrtf(s * c), sqrtf(s * a)) : make_float2(INFINITY, INFINITY);
+}
+// The limits on the values alone: a calm record may be evaluated anywhere.
 __device__ __forceinline__ bool calm_record(float4 r0, float4 r1, float4 r2) {
   return fabsf(r0.x) < 1e12f && fabsf(r0.y) < 1e12f && fabsf(r0.z) < 1e9f && fabsf(r0.w) < 1e9f &&
          fabsf(r1.x) < 1e9f &&
          fabsf(r1.y) + fabsf(r1.z) + fabsf(r1.w) + fabsf(r2.x) + fabsf(r2.y) < 1e12f;
-}
-__device__ __forceinline__ float2 support_half(float4 r0, float4 r1, float4 r2, float kk) {
-  const float a = r0.z, b = r0.w, c = r1.x;
-  const float det = a * c * (1.0f - 3e-5f) - b * b;
-  const bool ok = calm_record(r0, r1, r2) && a > 0.0f && c > 0.0f && det > 1e-30f;
-  const float s = kk / det;
-  return ok ? make_float2(sqrtf(s * c), sqrtf(s * a)) : make_float2(INFINITY, INFINITY);
 }
 // u = 1 - Q/k with its roundings spelled out: the same value wherever it is inlined.
 __device__ __forceinline__ float quad_u(float dx, float dy, float a, float b2, float c,
@@ -178,7 +181,10 @@ struct DenseWalk {
   }
   __device__ __forceinline__ static int split() { return (threadIdx.x >> 6) % SPL; }
 
-  template <class F>
+  // STRAIGHT: 64 entries that all reach the patch, and are bounded (so calm: u is a number), are
+  // walked without picking the hits.  Arm A, every box the whole image: G 2000, 400x400 157 -> 132
+  // us, 800x800 552 -> 473; not for the other arms, whose pairs cost several times as much.
+  template <bool STRAIGHT, class F>
   __device__ __forceinline__ void evaluate(int n, int X0, int Y0, const F& f) {
     const int lane = threadIdx.x & 63, sp = split();
     if (TS == 8) {
@@ -187,8 +193,8 @@ struct DenseWalk {
         const int j1 = two ? j + SPL : j;
         const float4 A0 = a[j], B0 = b[j], A1 = a[j1], B1 = b[j1];
         const float2 O0 = o[j], O1 = o[j1];
-        f(A0, B0, O0);
-        if (two) f(A1, B1, O1);
+        f(A0, B0, O0, std::false_type{});
+        if (two) f(A1, B1, O1, std::false_type{});
       }
       return;
     }
@@ -201,6 +207,11 @@ struct DenseWalk {
       const float2 e = h[j];
       const bool hit = j0 + lane < n && reaches(cx, 3.5f, A.x, e.x) && reaches(cy, 3.5f, A.y, e.y);
       uint64_t m = __ballot(hit);
+      if (STRAIGHT && m == ~0ull && __ballot(!(e.x < INFINITY)) == 0) {
+#pragma unroll 2
+        for (int i = j0 + sp; i < j0 + 64; i += SPL) f(a[i], b[i], o[i], std::true_type{});
+        continue;
+      }
       if (SPL > 1) {
         const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
@@ -216,15 +227,16 @@ struct DenseWalk {
         m &= m - 1;
         const float4 A0 = a[i0], B0 = b[i0], A1 = a[i1], B1 = b[i1];
         const float2 O0 = o[i0], O1 = o[i1];
-        f(A0, B0, O0);
-        if (two) f(A1, B1, O1);
+        f(A0, B0, O0, std::false_type{});
+        if (two) f(A1, B1, O1, std::false_type{});
       }
     }
   }
 
-  // f(A, B, O) for every gaussian that may weigh on this lane's pixel (and some that do not).
+  // f(A, B, O, calm) for every gaussian that may weigh on this lane's pixel (and some that do not);
+  // calm: a type that says whether 1 - Q/k is known to be a number.
   // cull = 0 takes every gaussian.  Ends with a barrier.
-  template <class F>
+  template <bool STRAIGHT = false, class F>
   __device__ __forceinline__ void walk(const float* __restrict__ proj, int G, float inv_k, int cull,
                                        int X0, int Y0, const F& f) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -266,7 +278,7 @@ struct DenseWalk {
       buf ^= 1;
       if (n > CAP - NT || G - g0 <= NT) {
         __syncthreads();
-        evaluate(n, X0, Y0, f);
+        evaluate<STRAIGHT>(n, X0, Y0, f);
         n = 0;
         __syncthreads();
       }
@@ -298,6 +310,50 @@ struct DenseWalk {
 
 // ---------------------------------------------------------------- forward
 
+struct Gauss {
+  float mx, my, a, b, c, z, cr, cg, cb, oc;
+};
+// (a uniform index: scalar loads)
+__device__ __forceinline__ Gauss gauss(const float* __restrict__ proj, int64_t g) {
+  const float* r = proj + g * 12;
+  return {r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8], r[9]};
+}
+
+// One pair's terms of a pixel's sums: colour, density, and revealage's logarithm.
+template <int ARM, int N>
+__device__ __forceinline__ void add_pair(float (&v)[N], float w, float cr, float cg, float cb,
+                                         float oc, float z, float zstar, float beta) {
+  if (ARM == kArmSZ) w *= sigmoidf_(-beta * (z - zstar));
+  if (ARM == kArmRV) v[N - 1] += log1pf(-fminf(w * oc, 1.0f - 1e-4f));
+  v[0] += w * cr;
+  v[1] += w * cg;
+  v[2] += w * cb;
+  v[3] += w * oc;
+}
+// The pixel of those sums, and what its backward needs.
+template <int ARM, int N>
+__device__ __forceinline__ void blend_pixel(int64_t p, const float (&v)[N], float zstar, float den0,
+                                            const float* __restrict__ bg, float* __restrict__ image,
+                                            float* __restrict__ den_out, float4* __restrict__ aux) {
+  if (ARM == kArmRV) {
+    const float d = v[3] + 1e-6f, R = expf(v[N - 1]);
+    const float a0 = v[0] / d, a1 = v[1] / d, a2 = v[2] / d;
+    image[p * 3 + 0] = a0 * (1.0f - R) + bg[1] * R;
+    image[p * 3 + 1] = a1 * (1.0f - R) + bg[2] * R;
+    image[p * 3 + 2] = a2 * (1.0f - R) + bg[3] * R;
+    if (den_out) den_out[p] = d;
+    aux[p] = make_float4(R, a0, a1, a2);
+  } else {
+    const float wb = bg[0];
+    const float d = v[3] + wb;
+    image[p * 3 + 0] = (v[0] + wb * bg[1]) / d;
+    image[p * 3 + 1] = (v[1] + wb * bg[2]) / d;
+    image[p * 3 + 2] = (v[2] + wb * bg[3]) / d;
+    if (den_out) den_out[p] = d;
+    if (ARM == kArmSZ) aux[p] = make_float4(zstar, den0, 0.0f, 0.0f);
+  }
+}
+
 // Bound by the tile tests (48 bytes of L2 per gaussian and tile) and by the pairs inside the
 // support.  Visiting every pair instead, one thread per pixel, took 91 us at G 2000, 128x128 (64
 // blocks, a serial chain of 2000), 1840-2040 us at G 10000, 800x800, and 441 us for SZ at G 3001,
@@ -319,15 +375,17 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
   const float px = (float)x + 0.5f, py = (float)y + 0.5f;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
   float zstar = 0.0f, den0 = 0.0f;
-  auto weight = [&](const float4& A, const float4& B) {
-    const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
+  auto weight = [&](const float4& A, const float4& B, auto calm) {
+    const float u = quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k);
+    const float r = decltype(calm)::value ? fmaxf(u, 0.0f) : relu_nan(u);
     return r * r;
   };
   if (ARM == kArmSZ) {   // z* first
     if (!tame(beta)) cull = 0;
     float v[2] = {0.f, 0.f};
-    s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
-      const float w = weight(A, B);
+    s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O,
+                                             auto calm) {
+      const float w = weight(A, B, calm);
       v[0] += w * O.x;
       v[1] += w * O.x * O.y;
     });
@@ -337,35 +395,63 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
     if (__syncthreads_or(!tame(zstar))) cull = 0;
   }
   float v[ARM == kArmRV ? 5 : 4] = {};
-  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
-    float w = weight(A, B);
-    if (ARM == kArmSZ) w *= sigmoidf_(-beta * (O.y - zstar));
-    if (ARM == kArmRV) v[4] += log1pf(-fminf(w * O.x, 1.0f - 1e-4f));
-    v[0] += w * B.y;
-    v[1] += w * B.z;
-    v[2] += w * B.w;
-    v[3] += w * O.x;
+  s.template walk<ARM == kArmA>(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B,
+                                                                  const float2& O, auto calm) {
+    add_pair<ARM>(v, weight(A, B, calm), B.y, B.z, B.w, O.x, O.y, zstar, beta);
   });
   s.join(v);
   if (Walk::split() != 0 || x >= W || y >= H) return;
-  const int64_t p = (int64_t)y * W + x;
-  if (ARM == kArmRV) {
-    const float d = v[3] + 1e-6f, R = expf(v[ARM == kArmRV ? 4 : 0]);
-    const float a0 = v[0] / d, a1 = v[1] / d, a2 = v[2] / d;
-    image[p * 3 + 0] = a0 * (1.0f - R) + bg[1] * R;
-    image[p * 3 + 1] = a1 * (1.0f - R) + bg[2] * R;
-    image[p * 3 + 2] = a2 * (1.0f - R) + bg[3] * R;
-    if (den_out) den_out[p] = d;
-    aux[p] = make_float4(R, a0, a1, a2);
-  } else {
-    const float wb = bg[0];
-    const float d = v[3] + wb;
-    image[p * 3 + 0] = (v[0] + wb * bg[1]) / d;
-    image[p * 3 + 1] = (v[1] + wb * bg[2]) / d;
-    image[p * 3 + 2] = (v[2] + wb * bg[3]) / d;
-    if (den_out) den_out[p] = d;
-    if (ARM == kArmSZ) aux[p] = make_float4(zstar, den0, 0.0f, 0.0f);
+  blend_pixel<ARM>((int64_t)y * W + x, v, zstar, den0, bg, image, den_out, aux);
+}
+
+// The same for up to kFew gaussians: one thread per pixel, every pair visited, no list to build.
+constexpr int kFew = 32;
+template <int ARM>
+__global__ __launch_bounds__(256) void k_render_dense_few(const float* __restrict__ proj, int G,
+                                                          int W, int P, float inv_k,
+                                                          const float* __restrict__ bg,
+                                                          const float* __restrict__ szb,
+                                                          float* __restrict__ image,
+                                                          float* __restrict__ den_out,
+                                                          float4* __restrict__ aux) {
+  __shared__ float4 s_a[kFew], s_b[kFew];
+  __shared__ float2 s_o[kFew];
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  const float px = (float)(p % W) + 0.5f, py = (float)(p / W) + 0.5f;
+  if ((int)threadIdx.x < G) {
+    const float4* r = reinterpret_cast<const float4*>(proj + (int64_t)threadIdx.x * 12);
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+    s_a[threadIdx.x] = make_float4(r0.x, r0.y, r0.z, 2.0f * r0.w);
+    s_b[threadIdx.x] = make_float4(r1.x, r1.z, r1.w, r2.x);
+    s_o[threadIdx.x] = make_float2(r2.y, r1.y);
   }
+  __syncthreads();
+  const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
+  float zstar = 0.0f, den0 = 0.0f;
+  auto weight = [&](const float4& A, const float4& B) {
+    const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
+    return r * r;
+  };
+  if (ARM == kArmSZ) {   // z* first
+    float n = 0.0f, d = 0.0f;
+#pragma unroll 4
+    for (int g = 0; g < G; ++g) {
+      const float w = weight(s_a[g], s_b[g]);
+      const float2 O = s_o[g];
+      d += w * O.x;
+      n += w * O.x * O.y;
+    }
+    den0 = d + 1e-6f;
+    zstar = n / den0;
+  }
+  float v[ARM == kArmRV ? 5 : 4] = {};
+#pragma unroll 4
+  for (int g = 0; g < G; ++g) {
+    const float4 A = s_a[g], B = s_b[g];
+    const float2 O = s_o[g];
+    add_pair<ARM>(v, weight(A, B), B.y, B.z, B.w, O.x, O.y, zstar, beta);
+  }
+  if (p < P) blend_pixel<ARM>(p, v, zstar, den0, bg, image, den_out, aux);
 }
 
 // theta form, forward: 16 waves share a block's 64 * PX pixels (PX per lane), the gaussians are
@@ -550,7 +636,8 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
                    !tame(beta);
   if (__syncthreads_or(bad)) cull = 0;
   float Z[1] = {0.0f};
-  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
+  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O,
+                                           auto) {
     const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
     const float h = sigmoidf_(-beta * (O.y - zs));
     Z[0] += r * r * (q.x * B.y + q.y * B.z + q.z * B.w + q.w * O.x) * h * (1.0f - h);
@@ -584,14 +671,6 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
 // G 10000, 300x300 481 (466); a whole-image box among 256 small ones, 800x800 223 (391), among
 // 10000 427 (3000).  Each box by itself always, by its own waves: 43, 333, 867, 791, 808.  Soft-Z,
 // every box the whole image: 118 (295), 992 (1004), G 4000, 400x400 1925 (1862).
-struct Gauss {
-  float mx, my, a, b, c, z, cr, cg, cb, oc;
-};
-// (a uniform index: scalar loads)
-__device__ __forceinline__ Gauss gauss(const float* __restrict__ proj, int64_t g) {
-  const float* r = proj + g * 12;
-  return {r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8], r[9]};
-}
 template <int ARM>
 struct PairSums {
   float r = 0.f, g = 0.f, b = 0.f, o = 0.f, beta = 0.f;   // dL/d col_o, o_col, softz_beta
@@ -1073,36 +1152,69 @@ inline bool dense_wide(int G, int P) { return G <= 4096 || P >= (1 << 17); }
 
 inline int dense_tiles(int H, int W, int ts) { return ((H + ts - 1) / ts) * ((W + ts - 1) / ts); }
 
-// The support boxes allow 0.01 for the rounding of pixel coordinates (2^-8 at 2^16).
-inline int dense_cull(int H, int W) { return H <= (1 << 16) && W <= (1 << 16); }
+// The support boxes allow 0.01 for the rounding of pixel coordinates (2^-8 at 2^16), and a 1/k in
+// range.
+inline int dense_cull(int H, int W, float ik) {
+  return H <= (1 << 16) && W <= (1 << 16) && ik < INFINITY;
+}
 
-// Tile side of the forward: every block tests all gaussians against its tile, so large tiles
-// test less, and small ones make more blocks.  Measured, arm A, sides 8 / 16 / 32 (us; SZ and RV
-// order the same way):
-//   G 10000, 800x800 (625 tiles of 32): 262 / 91 / 41;  G 500, 500x600 (304): 16 / 13 / 13
-//   G 2000, 400x400 (169 of 32, 625 of 16): 20 / 13 / 13 (RV 29 / 22 / 32)
-//   G 10000, 300x300 (361 of 16): 53 / 25 / 38;  100x60 (28 of 16): 28 / 43 / 113
-//   G 3001, 131x173 (99 of 16): 12 / 12 / 18 (SZ 20 / 22 / 47)
-inline int dense_tile_side(int H, int W) {
-  if (dense_tiles(H, W, 32) >= 300) return 32;
-  return dense_tiles(H, W, 16) >= 256 ? 16 : 8;
+// Tiles and threads of the forward's walk (and of the soft-Z pass): every block tests all gaussians
+// against its tile, so large tiles test less and small ones make more blocks; where every box is
+// the whole image the pairs bound it, and blocks that fill the GPU evenly count.  Measured, arm A,
+// small boxes / whole-image boxes (us; soft-Z orders the same way):
+//                        few       16/256      16/512      16/1024     32/1024     8/512
+//   G 16, 128x128        3.0/3.0   3.3/4.8     3.6/4.2     4.4/4.8     4.0/5.6     3.4/3.5
+//   G 32, 400x400        4.6/4.6   3.8/6.9     4.9/7.3     7.4/10      4.2/7.7     8.8/10
+//   G 64, 800x800        16/16     6.7/19      9.7/21      18/32       7.7/22      25/38
+//   G 256, 800x800       51/52     7.0/57      10/59       19/70       8.0/65      26/74
+//   G 256, 400x400       19/19     4.0/23      5.1/22      7.7/24      4.4/26      8.9/22
+//   G 600, 512x512                 6.3/60      7.4/59      9.6/61      4.7/58      17/63
+//   G 2000, 128x128                15/136      8.9/68      7.6/57      12/180      6.3/27
+//   G 2000, 256x256                9.6/136     6.9/70      6.2/58      7.4/177     11/54
+//   G 2000, 400x400                10/159      9.3/135     11/142      6.3/179     20/119
+//   G 2000, 800x800                20/419      21/415      27/444      11/475      62/443
+// (one thread per pixel, every pair visited: 3.0, 4.8, 16, 58, 20, -, 88, -, 125, -)
+template <class F>
+void dense_tiling(int G, int H, int W, const F& f) {
+  using std::integral_constant;
+  auto go = [&](auto ts, auto nt) {
+    f(grid_split(dense_tiles(H, W, decltype(ts)::value)), ts, nt);
+  };
+  if (dense_tiles(H, W, 16) < 256)
+    go(integral_constant<int, 8>{}, integral_constant<int, 512>{});
+  else if (G <= (dense_tiles(H, W, 32) >= 256 ? 256 : 128))
+    go(integral_constant<int, 16>{}, integral_constant<int, 256>{});
+  else if (dense_tiles(H, W, 32) >= 256)
+    go(integral_constant<int, 32>{}, integral_constant<int, 1024>{});
+  else if (dense_tiles(H, W, 16) >= 512 && G <= 8192)
+    go(integral_constant<int, 16>{}, integral_constant<int, 512>{});
+  else
+    go(integral_constant<int, 16>{}, integral_constant<int, 1024>{});
+}
+
+// So few gaussians that the forward visits every pair (the table above; the other arms' pairs cost
+// more).
+inline bool dense_few(int arm, int G, int H, int W) {
+  static_assert(kFew >= 32, "staged at once");
+  if (arm != kArmA) return G <= (arm == kArmSZ ? 8 : 2);
+  return G <= 16 || (G <= 32 && dense_tiles(H, W, 16) >= 256 && dense_tiles(H, W, 32) <= 256);
 }
 
 template <int ARM>
 void launch_render_dense(const float* proj, int G, int H, int W, float ik, const float* bg,
                          const float* szb, float* image, float* den, float4* aux,
                          hipStream_t stream) {
-  const int ts = dense_tile_side(H, W), cull = dense_cull(H, W);
-  const dim3 grid = grid_split(dense_tiles(H, W, ts));
-  if (ts == 32)
-    k_render_dense<ARM, 32, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb,
-                                                             image, den, aux);
-  else if (ts == 16)
-    k_render_dense<ARM, 16, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb,
-                                                             image, den, aux);
-  else
-    k_render_dense<ARM, 8, 512><<<grid, 512, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
-                                                          den, aux);
+  if (dense_few(ARM, G, H, W)) {
+    k_render_dense_few<ARM><<<grid1d(H * W, 256), 256, 0, stream>>>(proj, G, W, H * W, ik, bg, szb,
+                                                                   image, den, aux);
+    return;
+  }
+  const int cull = dense_cull(H, W, ik);
+  dense_tiling(G, H, W, [&](dim3 grid, auto ts, auto nt) {
+    constexpr int TS = decltype(ts)::value, NT = decltype(nt)::value;
+    k_render_dense<ARM, TS, NT><<<grid, NT, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image, den,
+                                                         aux);
+  });
 }
 
 // The whole quad backward of an arm; grad has kQuadComp columns (SZ: one more).
@@ -1121,22 +1233,15 @@ int launch_dense_bwd(const float* proj, int G, int H, int W, float ik, const flo
   base += pad256((size_t)P * 16);
   float2* ex = reinterpret_cast<float2*>(base);
   float* part = reinterpret_cast<float*>(base + pad256((size_t)P * 8));
-  const int cull = dense_cull(H, W);
+  const int cull = dense_cull(H, W, ik);
   const int npre = P / 256 + 1 < kPreBlocks ? P / 256 + 1 : kPreBlocks;
   k_dense_pre<ARM><<<npre, 256, 0, stream>>>(image, den, aux, gimage, P, bg, q, ex, gwbp, wild);
-  if (ARM == kArmSZ) {
-    const int ts = dense_tile_side(H, W);
-    const dim3 grid = grid_split(dense_tiles(H, W, ts));
-    if (ts == 32)
-      k_softz_pre<32, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                       wild + npre);
-    else if (ts == 16)
-      k_softz_pre<16, 1024><<<grid, 1024, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                       wild + npre);
-    else
-      k_softz_pre<8, 512><<<grid, 512, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                    wild + npre);
-  }
+  if constexpr (ARM == kArmSZ)
+    dense_tiling(G, H, W, [&](dim3 grid, auto ts, auto nt) {
+      constexpr int TS = decltype(ts)::value, NT = decltype(nt)::value;
+      k_softz_pre<TS, NT><<<grid, NT, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
+                                                   wild + npre);
+    });
   const int sh = quad_shares(G, P), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
   float* dst = sh > 1 ? part : grad;
   const int nw = npre + (ARM == kArmSZ ? 1 : 0);
