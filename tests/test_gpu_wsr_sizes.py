@@ -11,7 +11,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("G,P,keep", [(1, 1, None), (1, 65, "bool"), (15, 64, "float"),
                                       (63, 1023, "u8"), (64, 1025, None), (65, 129, "bool"),
                                       (1023, 63, "bool"), (1025, 300, None), (2100, 257, "u8"),
-                                      (5, 32769, "bool"), (130, 33000, None), (3000, 2049, None)])
+                                      (5, 32769, "bool"), (130, 33000, None), (3000, 2049, None),
+                                      (32, 32767, "u8"), (33, 255, "bool"), (100, 32771, "bool"),
+                                      (101, 32833, None), (300, 33023, "u8"), (301, 32769, None),
+                                      (257, 1, "bool")])
 def test_wsr_follows_the_formula(G, P, keep):
     print(f"[wsr] {G} {P} {keep}", flush=True)
     g = torch.Generator().manual_seed(G * 7 + P)

@@ -454,23 +454,24 @@ __global__ __launch_bounds__(256) void k_render_dense_few(const float* __restric
   if (p < P) blend_pixel<ARM>(p, v, zstar, den0, bg, image, den_out, aux);
 }
 
-// theta form, forward: 16 waves share a block's 64 * PX pixels (PX per lane), the gaussians are
-// dealt to the waves in runs and the waves' sums joined in wave order.  Every pair counts (the
-// basis is arbitrary, so there is no support box): bound by the 10 CU cycles of LDS a gaussian's
-// 40 bytes take per wave and, with PX pixels sharing them, by the VALU (13 instructions a pair).
+// theta form, forward: SPL waves of a block share 64 * PX pixels (PX per lane), the gaussians are dealt
+// to them in runs and their sums joined in wave order.  Every pair counts (the basis is arbitrary, so
+// there is no support box): bound by the 10 CU cycles of LDS a gaussian's 40 bytes take per wave and,
+// with PX pixels sharing them, by the VALU (13 instructions a pair); the joins cost where there are
+// few gaussians, a wave's own pixels (SPL = 1) where there are few pixels.
 constexpr int kThetaThreads = 1024;
 constexpr int kThetaWaves = kThetaThreads / 64;
 
-template <int PX>
-__global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
+template <int PX, int SPL, int NT>
+__global__ __launch_bounds__(NT) void k_wsr_dense(
     const float* __restrict__ theta, const float* __restrict__ o, const float* __restrict__ color,
     const uint8_t* __restrict__ keep, const float* __restrict__ phi, int G, int P,
     const float* __restrict__ bg, float* __restrict__ C, float* __restrict__ den_out) {
-  __shared__ float4 s_a[kThetaThreads];  // theta 0..3
-  __shared__ float4 s_c[kThetaThreads];  // o*keep*color, o*keep
-  __shared__ float2 s_b[kThetaThreads];  // theta 4, 5
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t p0 = (int64_t)block_id() * 64 * PX + lane;
+  __shared__ float4 s_a[NT];  // theta 0..3
+  __shared__ float4 s_c[NT];  // o*keep*color, o*keep
+  __shared__ float2 s_b[NT];  // theta 4, 5
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = wave % SPL;
+  const int64_t p0 = ((int64_t)block_id() * (NT / 64 / SPL) + wave / SPL) * 64 * PX + lane;
   float f[PX][6], n[PX][4];
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
@@ -479,8 +480,8 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
 #pragma unroll
     for (int k = 0; k < 4; ++k) n[i][k] = 0.f;
   }
-  for (int g0 = 0; g0 < G; g0 += kThetaThreads) {
-    const int cnt = min(kThetaThreads, G - g0);
+  for (int g0 = 0; g0 < G; g0 += NT) {
+    const int cnt = min(NT, G - g0);
     __syncthreads();
     if ((int)threadIdx.x < cnt) {
       const int g = g0 + threadIdx.x;
@@ -492,9 +493,9 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
                                      ok * color[(int64_t)g * 3 + 2], ok);
     }
     __syncthreads();
-    const int j1 = (int)((wave + 1) * cnt) / kThetaWaves;
+    const int j1 = (sub + 1) * cnt / SPL;
 #pragma unroll 4
-    for (int j = (int)(wave * cnt) / kThetaWaves; j < j1; ++j) {
+    for (int j = sub * cnt / SPL; j < j1; ++j) {
       const float4 A = s_a[j], Cc = s_c[j];
       const float2 B = s_b[j];
 #pragma unroll
@@ -510,28 +511,32 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense(
       }
     }
   }
-  // joined per PX: [wave][4][64] floats fill s_a
+  static_assert(SPL == 1 || PX <= SPL, "a finishing wave each");
+  // a pixel's sums, joined over the waves that share it: [wave][4][64] floats fill s_a
   float* s = reinterpret_cast<float*>(s_a);
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
-    __syncthreads();
+    if (SPL > 1) {
+      __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s[(wave * 4 + k) * 64 + lane] = n[i][k];
-    __syncthreads();
-    if (wave != i) continue;   // wave i finishes the block's i-th run of pixels
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int k = 0; k < 4; ++k) s[(wave * 4 + k) * 64 + lane] = n[i][k];
+      __syncthreads();
+      if (sub != i) continue;   // wave i of the sharing ones finishes their i-th run of pixels
 #pragma unroll
-    for (int w = 0; w < kThetaWaves; ++w) {
+      for (int k = 0; k < 4; ++k) n[i][k] = 0.f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] += s[(w * 4 + k) * 64 + lane];
+      for (int w = 0; w < SPL; ++w) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) n[i][k] += s[((wave - i + w) * 4 + k) * 64 + lane];
+      }
     }
     const int64_t p = p0 + i * 64;
     if (p < P) {
       const float wb = bg[0];
-      const float d = v[3] + wb;
-      C[p * 3 + 0] = (v[0] + wb * bg[1]) / d;
-      C[p * 3 + 1] = (v[1] + wb * bg[2]) / d;
-      C[p * 3 + 2] = (v[2] + wb * bg[3]) / d;
+      const float d = n[i][3] + wb;
+      C[p * 3 + 0] = (n[i][0] + wb * bg[1]) / d;
+      C[p * 3 + 1] = (n[i][1] + wb * bg[2]) / d;
+      C[p * 3 + 2] = (n[i][2] + wb * bg[3]) / d;
       if (den_out) den_out[p] = d;
     }
   }
@@ -1364,15 +1369,30 @@ int tts_wsr_dense(const float* theta, const float* o, const float* color, const 
   if ((G > 0 && (!theta || !o || !color)) || !phi || !bg || !C || P <= 0 || G < 0)
     return TTS_EINVAL;
   if (G > (1 << 30) || P > (1 << 30)) return TTS_EINVAL;
-  // Pixels per lane: four read the gaussians' LDS records a quarter as often, one makes four times
-  // the blocks.  Measured, one / four (us): G 2000, 128x128 19 / 37; G 6000, 100x100 45 / 94,
-  // 200x200 116 / 95; G 2000, 600x600 263 / 209 (one thread per pixel, a chain over G: 79, 230, 230
-  // and 278).
-  if (P <= 32768)
-    k_wsr_dense<1><<<grid_split(grid1d(P, 64)), kThetaThreads, 0, stream>>>(
+  // Pixels per lane / sharing waves / threads, measured (us):
+  //                      1/1/256  4/4/256  1/16/1024  4/16/1024
+  //   G 1, P 16384         2.5      4.0       3.7        7.4
+  //   G 1, P 640000        5.9       13        46         56
+  //   G 64, P 50000        5.0      5.8       7.6        8.5
+  //   G 150, P 640000       33       30        62         78
+  //   G 300, P 160000       23       20        25         32
+  //   G 2000, P 16384       80       62        19         37
+  //   G 2000, P 50000       81       62        54         39
+  //   G 2000, P 640000     381      292       461        363
+  //   G 6000, P 100000     253      206       240        193
+  const bool few = G <= 32 || (G <= 100 && P > 32768);
+  const bool four = P > 32768 && (G <= 300 || (G <= 4096 && P >= (1 << 16)) || P >= (1 << 18));
+  if (few)
+    k_wsr_dense<1, 1, 256><<<grid_split(grid1d(P, 256)), 256, 0, stream>>>(
+        theta, o, color, keep, phi, G, P, bg, C, den);
+  else if (four)
+    k_wsr_dense<4, 4, 256><<<grid_split(grid1d(P, 256)), 256, 0, stream>>>(
+        theta, o, color, keep, phi, G, P, bg, C, den);
+  else if (P <= 32768)
+    k_wsr_dense<1, 16, 1024><<<grid_split(grid1d(P, 64)), 1024, 0, stream>>>(
         theta, o, color, keep, phi, G, P, bg, C, den);
   else
-    k_wsr_dense<4><<<grid_split(grid1d(P, 256)), kThetaThreads, 0, stream>>>(
+    k_wsr_dense<4, 16, 1024><<<grid_split(grid1d(P, 256)), 1024, 0, stream>>>(
         theta, o, color, keep, phi, G, P, bg, C, den);
   return launch_status();
 }
