@@ -57,3 +57,19 @@ def test_wsr_is_deterministic_and_gradients_sum_over_bands():
     a = kernels.wsr_dense_bwd(th, o, col, None, phi, bg, C, den, gC)
     b = kernels.wsr_dense_bwd(th, o, col, None, phi, bg, C, den, gC)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_wsr_bands_of_many_gaussians():
+    """Bands past one round of blocks (G 20000: 313 blocks a band, 8 bands of uneven length)."""
+    g = torch.Generator().manual_seed(5)
+    G, P = 20000, 9001
+    leaves = [t.cuda() for t in (torch.randn(G, 6, generator=g) * 0.2, torch.rand(G, generator=g),
+                                 torch.rand(G, 3, generator=g), torch.tensor(0.3))]
+    phi, cb = torch.randn(P, 6, generator=g).cuda(), torch.tensor([0.9, 0.5, 0.2]).cuda()
+    R = torch.randn(P, 3, generator=g).cuda()
+    dev = [t.requires_grad_(True) for t in leaves]
+    got = torch.autograd.grad((backward.wsr_polysplat(*dev, phi, cb) * R).sum(), dev)
+    ref = [t.detach().double().requires_grad_(True) for t in leaves]
+    C = backward_formula(ref, phi.double(), cb.double(), None)
+    for a, b in zip(got, torch.autograd.grad((C * R.double()).sum(), ref)):
+        assert float((a.double() - b).norm()) <= 1e-3 * float(b.norm()) + 1e-5
