@@ -4,6 +4,8 @@ and twice with the same result."""
 import pytest
 import torch
 
+from ttsplat import kernels
+
 from test_gpu_dense_cull import grads, oracle, oracle_detached_z, records, render
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +60,38 @@ def test_forward_of_large_boxes_follows_the_formula(G, H, W, arm):
     # u carries 12 eps (a dx^2 + c dy^2) / k
     ref = oracle(proj, H, W, arm)
     assert float((render(proj.cuda(), H, W, arm).cpu() - ref).abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+def test_wide_images_give_up_the_boxes(arm):
+    """A side over 65536: every pair is visited, in both passes."""
+    H, W, G = 1, 65537, 40
+    proj = records(G, H, W, seed=1, cond=10.0, size=3.0)
+    proj[0, 0], proj[1, 0] = 65530.0, 2.0
+    gi = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(3))
+    P = proj.double().requires_grad_(True)
+    beta = torch.tensor(3.0, dtype=torch.float64)
+    ref = oracle_detached_z(P, H, W, arm, beta)
+    (ref * gi.double()).sum().backward()
+    assert float((render(proj.cuda(), H, W, arm).cpu() - ref.detach()).abs().max()) <= 1e-4
+    got = grads(proj.cuda(), H, W, arm, gi.cuda())[0].cpu().double()[:, :9]
+    want = torch.cat([P.grad[:, 2:5], P.grad[:, 0:2], P.grad[:, 6:10]], 1)
+    for sl in (slice(0, 3), slice(3, 5), slice(5, 8), slice(8, 9)):
+        assert float((got[:, sl] - want[:, sl]).norm()) <= 1e-3 * float(want[:, sl].norm())
+
+
+def test_backward_of_more_blocks_than_a_grid_row():
+    """Over 2^21 blocks: the last gaussians' gradients (2^23 and more of them, four to a block) are
+    those of the same gaussians alone."""
+    H, W, n = 6, 5, 12
+    tail = records(n, H, W, seed=2).cuda()
+    proj = torch.zeros((1 << 23) + n, 12, device="cuda")
+    proj[:, 0], proj[:, 2], proj[:, 4] = -100.0, 1.0, 1.0
+    proj[-n:] = tail
+    bg = torch.tensor([0.05, 0.9, 1.0, 0.8], device="cuda")
+    img, den = kernels.render_dense(tail, H, W, 4.0, bg)
+    gi = torch.randn(H, W, 3, generator=torch.Generator().manual_seed(1)).cuda()
+    got, gwb = kernels.render_dense_bwd(proj, H, W, 4.0, bg, img, den, gi)
+    few, gwb2 = kernels.render_dense_bwd(torch.cat([tail] * 400), H, W, 4.0, bg, img, den, gi)
+    assert torch.equal(got[-n:], few[-n:]) and torch.equal(gwb, gwb2)
+    assert not bool(got[:-n].any())

@@ -481,6 +481,7 @@ __global__ __launch_bounds__(NT) void k_wsr_dense(
   __shared__ float2 s_b[NT];  // theta 4, 5
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = wave % SPL;
   const int64_t p0 = ((int64_t)block_id() * (NT / 64 / SPL) + wave / SPL) * 64 * PX + lane;
+  if ((int64_t)block_id() * (NT / SPL) * PX >= P) return;
   float f[PX][6], n[PX][4];
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
@@ -1028,6 +1029,7 @@ __global__ __launch_bounds__(kThetaThreads) void k_wsr_dense_bwd(
   float2* s_fb = reinterpret_cast<float2*>(s_fa + kThetaThreads);     // phi 4..5
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int band = blockIdx.y, gblock = block_id();
+  if ((int64_t)gblock * 64 >= G) return;
   const int64_t g = (int64_t)gblock * 64 + lane;
   const bool act = g < G;
   float th[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
