@@ -553,7 +553,9 @@ int tts_background_grad(const float* gwb, int n, const float* w_b_raw, float* gw
 #define TTS_ARM_SZ 1  /* soft-Z visibility prepass (:50-68) */
 #define TTS_ARM_RV 2  /* revealage compositing (:71-83) */
 
-/* Workspace for the dense backward entry points (G gaussians, P pixels). */
+/* Workspace for the dense backward entry points (G gaussians, P pixels): 24 bytes a pixel up to 2^25
+ * pixels (805 MB; larger images are taken in runs of that many), or 40 bytes a gaussian and band of
+ * tts_wsr_dense_bwd (up to 1 GiB, and one band past that), whichever is more. */
 size_t tts_dense_workspace_bytes(int G, int P);
 
 /* Dense arm-A render from proj[G,12]: Q = a dx^2 + 2b dx dy + c dy^2 at pixel centres

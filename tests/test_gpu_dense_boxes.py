@@ -4,7 +4,7 @@ and twice with the same result."""
 import pytest
 import torch
 
-from ttsplat import kernels
+from ttsplat import _lib, kernels
 
 from test_gpu_dense_cull import grads, oracle, oracle_detached_z, records, render
 
@@ -95,3 +95,39 @@ def test_backward_of_more_blocks_than_a_grid_row():
     few, gwb2 = kernels.render_dense_bwd(torch.cat([tail] * 400), H, W, 4.0, bg, img, den, gi)
     assert torch.equal(got[-n:], few[-n:]) and torch.equal(gwb, gwb2)
     assert not bool(got[:-n].any())
+
+
+@pytest.mark.parametrize("arm", ["A", "SZ", "RV"])
+@pytest.mark.parametrize("G", [40, 300])
+def test_backward_of_images_past_one_run(G, arm):
+    """2^25 pixels are one run of the backward: an image of rows past it against the same gaussians
+    on a crop around the cut, and the workspace."""
+    W, H, cut = 8192, 4096 + 40, 4096
+    crop = records(G, 80, 120, seed=4, size=4.0)
+    crop[:, 1] = (crop[:, 1] * 64).round() / 64        # the same place 4056 rows further down
+    crop[:, 0] = crop[:, 0].clamp(10, 110)
+    full = crop.clone()
+    full[:, 1] += cut - 40
+    g = torch.Generator().manual_seed(3)
+    gi = torch.zeros(H, W, 3, device="cuda")
+    gc = torch.randn(80, 120, 3, generator=g).cuda()
+    gi[cut - 40:, :120] = gc
+    assert _lib.load().tts_dense_workspace_bytes(G, H * W) < 1 << 30
+    a, wa = grads(full.cuda(), H, W, arm, gi)
+    b, wb = grads(crop.cuda(), 80, 120, arm, gc)
+    # the same terms in another order
+    for sl in (slice(0, 3), slice(3, 5), slice(5, 8), slice(8, 9)):
+        assert float((a[:, sl] - b[:, sl]).norm()) <= 1e-3 * float(b[:, sl].norm())
+    assert abs(float(wa) - float(wb)) <= 1e-3 * abs(float(wb)) + 1e-4
+
+
+def test_backward_of_rows_past_one_run():
+    """One row of more than 2^25 pixels: the second run has no gradient to add."""
+    W = (1 << 25) + 70
+    proj = records(9, 1, 200, seed=4, size=4.0).cuda()
+    gi = torch.zeros(1, W, 3, device="cuda")
+    gi[0, :200] = torch.randn(200, 3, generator=torch.Generator().manual_seed(3)).cuda()
+    a, wa = grads(proj, 1, W, "A", gi)
+    b, wb = grads(proj, 1, 200, "A", gi[:, :200].contiguous())
+    assert float((a - b).norm()) <= 1e-4 * float(b.norm())
+    assert abs(float(wa) - float(wb)) <= 1e-4 * abs(float(wb)) + 1e-4

@@ -80,9 +80,14 @@ inline size_t theta_ws_bytes(int G, int P) {
 
 constexpr int kPreBlocks = 256;
 
-// Workspace of the quad form: [align to 256][gwb partials, kPreBlocks floats][wild flags,
-// kPreBlocks + 1 ints, padded to 256][per-pixel gradients, P float4][arm extras, P float2, padded]
-// [the shares' gradients, shares*G*(kQuadComp + 1), when there is more than one share].
+// The quad form's backward takes the image in runs of up to kRunPixels pixels (whole rows, or part
+// of one), so that its 24 bytes a pixel stay under 1 GiB.
+constexpr int kRunPixels = 1 << 25;
+
+// Workspace of the quad form, n = min(P, kRunPixels): [align to 256][gwb partials, kPreBlocks
+// floats] [wild flags, kPreBlocks + 1 ints, padded to 256][per-pixel gradients, n float4][arm
+// extras, n float2, padded][the shares' gradients, shares*G*(kQuadComp + 1), when there is more
+// than one].
 //
 // Shares of a gaussian's box in the backward: few gaussians over a large image would leave most of
 // the GPU idle, and from 256 on the sum of the shares costs more than it gives.  Every box the
@@ -96,9 +101,9 @@ inline int quad_shares(int G, int P) {
 
 inline size_t quad_ws_bytes(int G, int P) {
   if (G <= 0 || P <= 0) return 0;
-  const size_t sh = (size_t)quad_shares(G, P);
-  return 256 + kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4) + pad256((size_t)P * 16) +
-         pad256((size_t)P * 8) + (sh > 1 ? sh * (size_t)G * (kQuadComp + 1) * 4 : 0);
+  const size_t sh = (size_t)quad_shares(G, P), n = P < kRunPixels ? P : kRunPixels;
+  return 256 + kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4) + pad256(n * 16) + pad256(n * 8) +
+         (sh > 1 ? sh * (size_t)G * (kQuadComp + 1) * 4 : 0);
 }
 
 // A long 1-D grid: blocks past 2^21 go to the z dimension (a launch holds under 2^32 threads per
@@ -621,10 +626,11 @@ __global__ __launch_bounds__(256) void k_dense_pre(const float* __restrict__ ima
 }
 
 // Soft-Z backward, between the passes: Z/den0 of every pixel, Z = dL/dz* =
-// beta sum_g w_geo (gnum . col_o + gden o_col) h (1 - h); ex = (z*, Z/den0).  The forward's walk.
+// beta sum_g w_geo (gnum . col_o + gden o_col) h (1 - h); ex = (z*, Z/den0).  The forward's walk,
+// over the W x H pixels from (xo, yo) on.
 template <int TS, int NT>
 __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj, int G, int W,
-                                                  int H, float inv_k, int cull,
+                                                  int H, int xo, int yo, float inv_k, int cull,
                                                   const float* __restrict__ szb,
                                                   const float4* __restrict__ aux,
                                                   const float4* __restrict__ qbuf,
@@ -637,7 +643,7 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
   const int x = X0 + Walk::lane_x(), y = Y0 + Walk::lane_y();
   const bool in = x < W && y < H;
   const int64_t p = (int64_t)y * W + x;
-  const float px = (float)x + 0.5f, py = (float)y + 0.5f;
+  const float px = (float)x + ((float)xo + 0.5f), py = (float)y + ((float)yo + 0.5f);
   const float beta = szb[0];
   float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
   float zs = 0.f, d0 = 1.f;
@@ -651,8 +657,8 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
                    !tame(beta);
   if (__syncthreads_or(bad)) cull = 0;
   float Z[1] = {0.0f};
-  s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O,
-                                           auto) {
+  s.walk(proj, G, inv_k, cull, X0 + xo, Y0 + yo, [&](const float4& A, const float4& B,
+                                                     const float2& O, auto) {
     const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
     const float h = sigmoidf_(-beta * (O.y - zs));
     Z[0] += r * r * (q.x * B.y + q.y * B.z + q.z * B.w + q.w * O.x) * h * (1.0f - h);
@@ -749,8 +755,9 @@ __device__ __forceinline__ Cells pair_cells(int x0, int x1, int y0, int y1, int 
 
 template <int ARM, int GPB, int WPG>
 __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
-    const float* __restrict__ proj, int G, int W, int H, float inv_k, int cull,
-    const float* __restrict__ szb, const float4* __restrict__ qbuf, const float2* __restrict__ ex,
+    const float* __restrict__ proj, int G, int W, int H, float xc, float yc, int acc, float inv_k,
+    int cull, const float* __restrict__ szb, const float4* __restrict__ qbuf,
+    const float2* __restrict__ ex,
     const int* __restrict__ wild, int n_pre, int n_wild, const float* __restrict__ gwb_part,
     float* __restrict__ out, float* __restrict__ gwb) {
   constexpr int NC = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
@@ -779,7 +786,7 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
     float t = 0.0f;
     for (int i = lane; i < n_pre; i += 64) t += gwb_part[i];
     t = wave_sum(t);
-    if (lane == 0) gwb[0] = t;
+    if (lane == 0) gwb[0] = acc & 1 ? gwb[0] + t : t;
   }
   out += ((int64_t)share * G + g0) * NC;
   const float mx = r0.x, my = r0.y;
@@ -789,10 +796,10 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
   int x0 = 0, x1 = W, y0 = 0, y1 = H;
   if (cull) {
     const float2 e = support_half(r0, r1, r2, support_k(inv_k));
-    x0 = (int)fminf(fmaxf(ceilf(mx - e.x - 0.51f), 0.0f), (float)W);
-    y0 = (int)fminf(fmaxf(ceilf(my - e.y - 0.51f), 0.0f), (float)H);
-    x1 = (int)fmaxf(fminf(floorf(mx + e.x - 0.49f) + 1.0f, (float)W), (float)x0);
-    y1 = (int)fmaxf(fminf(floorf(my + e.y - 0.49f) + 1.0f, (float)H), (float)y0);
+    x0 = (int)fminf(fmaxf(ceilf(mx - e.x - (xc + 0.01f)), 0.0f), (float)W);
+    y0 = (int)fminf(fmaxf(ceilf(my - e.y - (yc + 0.01f)), 0.0f), (float)H);
+    x1 = (int)fmaxf(fminf(floorf(mx + e.x - (xc - 0.01f)) + 1.0f, (float)W), (float)x0);
+    y1 = (int)fmaxf(fminf(floorf(my + e.y - (yc - 0.01f)) + 1.0f, (float)H), (float)y0);
   }
   const int n_pix = act ? (x1 - x0) * (y1 - y0) : 0;
   if (n_pix == 0) x0 = x1 = y0 = y1 = 0;
@@ -837,7 +844,7 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
       float4 q = qbuf[p];
       float2 e = ARM != kArmA ? pixel_extra<ARM>(ex, p) : make_float2(0.f, 0.f);
       while (true) {
-        const float dx = (float)(bx + x) + 0.5f - h.mx, dy = (float)(by + y) + 0.5f - h.my;
+        const float dx = (float)(bx + x) + xc - h.mx, dy = (float)(by + y) + yc - h.my;
         const float4 qc = q;
         const float2 ec = e;
         i += S;
@@ -880,7 +887,7 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
     o = lane == 4 ? -2.0f * (h.b * m_x + h.c * m_y) : o;            // dQ/dmu_y = -2 (b dx + c dy)
 #pragma unroll
     for (int k = 5; k < NC; ++k) o = lane == k ? v[k] : o;
-    if (lane < NC && g0 + j < G) out[j * NC + lane] = o;
+    if (lane < NC && g0 + j < G) out[j * NC + lane] = acc & 2 ? out[j * NC + lane] + o : o;
   };
 
   float v[10];
@@ -923,7 +930,7 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
         const int y = u.y0 + band * 8 + (lane >> 3);
         const bool row = y < u.y1;
         int x = u.x0 + col * 8 + (lane & 7);
-        const float yf = (float)y + 0.5f;
+        const float yf = (float)y + yc;
         float dy[2], bd[2], cd[2], s0[2], s1[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -943,7 +950,7 @@ __global__ __launch_bounds__(64 * GPB * WPG) void k_render_dense_bwd(
           const float4 qc = q;
           const float2 ec = e;
           const bool in = row && x < u.x1;
-          const float xf = (float)x + 0.5f;
+          const float xf = (float)x + xc;
           x += 8;
           p += 8;
           if (k + 1 < m && row && x < u.x1) {   // the next cell's loads, in flight during this one
@@ -1133,12 +1140,13 @@ __device__ __forceinline__ void add_bands(const float*& src, int64_t stride, int
   left -= N;
 }
 
-// out[g][c] = sum over bands of part[band][g][c], in band order; gwb = sum of gwb_part.
+// out[g][c] = sum over bands of part[band][g][c], in band order (acc: added to out); gwb = sum of
+// gwb_part.
 __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ part, int nb,
                                                       int G, int ncomp,
                                                       const float* __restrict__ gwb_part,
                                                       float* __restrict__ out,
-                                                      float* __restrict__ gwb) {
+                                                      float* __restrict__ gwb, int acc) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t n = (int64_t)G * ncomp;
   if (i < n) {
@@ -1150,7 +1158,7 @@ __global__ __launch_bounds__(256) void k_dense_reduce(const float* __restrict__ 
     if (left >= 4) add_bands<4>(src, n, left, s);
     if (left >= 2) add_bands<2>(src, n, left, s);
     if (left) add_bands<1>(src, n, left, s);
-    out[i] = s;
+    out[i] = acc ? out[i] + s : s;
   }
   if (blockIdx.x == 0 && threadIdx.x < 64 && gwb) {   // wave 0: lanes over the bands
     float s = 0.f;
@@ -1228,8 +1236,8 @@ void launch_render_dense(const float* proj, int G, int H, int W, float ik, const
   const int cull = dense_cull(H, W, ik);
   dense_tiling(G, H, W, [&](dim3 grid, auto ts, auto nt) {
     constexpr int TS = decltype(ts)::value, NT = decltype(nt)::value;
-    k_render_dense<ARM, TS, NT><<<grid, NT, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image, den,
-                                                         aux);
+    k_render_dense<ARM, TS, NT><<<grid, NT, 0, stream>>>(proj, G, W, H, ik, cull, bg, szb, image,
+                                                         den, aux);
   });
 }
 
@@ -1241,42 +1249,55 @@ int launch_dense_bwd(const float* proj, int G, int H, int W, float ik, const flo
                      hipStream_t stream) {
   const int P = H * W;
   if (!ws || ws_bytes < quad_ws_bytes(G, P)) return TTS_EWORKSPACE;
+  const int cap = P < kRunPixels ? P : kRunPixels;
   char* base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(ws) + 255) & ~uintptr_t(255));
   float* gwbp = reinterpret_cast<float*>(base);
   int* wild = reinterpret_cast<int*>(base + kPreBlocks * 4);
   base += kPreBlocks * 4 + pad256((kPreBlocks + 1) * 4);
   float4* q = reinterpret_cast<float4*>(base);
-  base += pad256((size_t)P * 16);
+  base += pad256((size_t)cap * 16);
   float2* ex = reinterpret_cast<float2*>(base);
-  float* part = reinterpret_cast<float*>(base + pad256((size_t)P * 8));
+  float* part = reinterpret_cast<float*>(base + pad256((size_t)cap * 8));
   const int cull = dense_cull(H, W, ik);
-  const int npre = P / 256 + 1 < kPreBlocks ? P / 256 + 1 : kPreBlocks;
-  k_dense_pre<ARM><<<npre, 256, 0, stream>>>(image, den, aux, gimage, P, bg, q, ex, gwbp, wild);
-  if constexpr (ARM == kArmSZ)
-    dense_tiling(G, H, W, [&](dim3 grid, auto ts, auto nt) {
-      constexpr int TS = decltype(ts)::value, NT = decltype(nt)::value;
-      k_softz_pre<TS, NT><<<grid, NT, 0, stream>>>(proj, G, W, H, ik, cull, szb, aux, q, ex,
-                                                   wild + npre);
-    });
   const int sh = quad_shares(G, P), nc = ARM == kArmSZ ? kQuadComp + 1 : kQuadComp;
   float* dst = sh > 1 ? part : grad;
-  const int nw = npre + (ARM == kArmSZ ? 1 : 0);
-  auto launch = [&](auto gpb, auto wpg) {
-    constexpr int GPB = decltype(gpb)::value, WPG = decltype(wpg)::value;
-    const dim3 grid = grid_split(((int64_t)G + GPB - 1) / GPB, sh);
-    k_render_dense_bwd<ARM, GPB, WPG><<<grid, 64 * GPB * WPG, 0, stream>>>(
-        proj, G, W, H, ik, cull, szb, q, ex, wild, npre, nw, gwbp, dst, gwb);
-  };
-  using std::integral_constant;
-  if (G >= 256 && G < 512 && P >= (1 << 18))
-    launch(integral_constant<int, 1>{}, integral_constant<int, 16>{});
-  else if (!dense_wide(G, P))
-    launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
-  else
-    launch(integral_constant<int, ARM == kArmSZ ? 1 : 2>{}, integral_constant<int, 4>{});
-  if (sh > 1)
-    k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, sh, G, nc, nullptr,
-                                                                    grad, nullptr);
+  // runs of whole rows, or of part of a row
+  const int rw = W < cap ? W : cap, rh = W < cap ? cap / W : 1;
+  for (int yo = 0; yo < H; yo += rh) {
+    for (int xo = 0; xo < W; xo += rw) {
+      const int w = W - xo < rw ? W - xo : rw, h = H - yo < rh ? H - yo : rh, n = w * h;
+      const int64_t at = (int64_t)yo * W + xo;
+      const float4* ax = ARM == kArmA ? nullptr : aux + at;
+      const int npre = n / 256 + 1 < kPreBlocks ? n / 256 + 1 : kPreBlocks;
+      k_dense_pre<ARM><<<npre, 256, 0, stream>>>(image + at * 3, den + at, ax, gimage + at * 3, n,
+                                                 bg, q, ex, gwbp, wild);
+      if constexpr (ARM == kArmSZ)
+        dense_tiling(G, h, w, [&](dim3 grid, auto ts, auto nt) {
+          constexpr int TS = decltype(ts)::value, NT = decltype(nt)::value;
+          k_softz_pre<TS, NT><<<grid, NT, 0, stream>>>(proj, G, w, h, xo, yo, ik, cull, szb, ax, q,
+                                                       ex, wild + npre);
+        });
+      const int nw = npre + (ARM == kArmSZ ? 1 : 0);
+      const int more = at > 0, acc = more + (more && sh == 1 ? 2 : 0);
+      auto launch = [&](auto gpb, auto wpg) {
+        constexpr int GPB = decltype(gpb)::value, WPG = decltype(wpg)::value;
+        const dim3 grid = grid_split(((int64_t)G + GPB - 1) / GPB, sh);
+        k_render_dense_bwd<ARM, GPB, WPG><<<grid, 64 * GPB * WPG, 0, stream>>>(
+            proj, G, w, h, (float)xo + 0.5f, (float)yo + 0.5f, acc, ik, cull, szb, q, ex, wild,
+            npre, nw, gwbp, dst, gwb);
+      };
+      using std::integral_constant;
+      if (G >= 256 && G < 512 && P >= (1 << 18))
+        launch(integral_constant<int, 1>{}, integral_constant<int, 16>{});
+      else if (!dense_wide(G, P))
+        launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+      else
+        launch(integral_constant<int, ARM == kArmSZ ? 1 : 2>{}, integral_constant<int, 4>{});
+      if (sh > 1)
+        k_dense_reduce<<<grid1d((int64_t)G * nc, 256), 256, 0, stream>>>(part, sh, G, nc, nullptr,
+                                                                        grad, nullptr, more);
+    }
+  }
   return launch_status();
 }
 
@@ -1424,7 +1445,7 @@ int tts_wsr_dense_bwd(const float* theta, const float* o, const float* color,
   k_wsr_dense_bwd<<<grid, kThetaThreads, 0, stream>>>(theta, o, color, keep, phi, G, P, PB, bg, C,
                                                       den, gC, part, gwbp);
   k_dense_reduce<<<grid1d((int64_t)G * kThetaComp, 256), 256, 0, stream>>>(
-      part, nb, G, kThetaComp, gwbp, gtheta10, gwb);
+      part, nb, G, kThetaComp, gwbp, gtheta10, gwb, 0);
   return launch_status();
 }
 
