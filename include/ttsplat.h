@@ -541,7 +541,8 @@ int tts_relocate(float* params, float* m, float* v, float* sh_rest, float* sh_m,
 int tts_zero(float* buf, int64_t n, hipStream_t stream);
 
 /* Background block bg[4] = (softplus(w_b_raw), c_b r, g, b) (spike/render.py:28), and
- * gw_b_raw[0] = softplus'(w_b_raw) * sum gwb[0..n) (spike's autograd through it). */
+ * gw_b_raw[0] = softplus'(w_b_raw) * sum gwb[0..n) (spike's autograd through it): launches of their
+ * own, for callers that do not take them with tts_geom_fwd_bg and tts_geom_bwd_render. */
 int tts_background(const float* w_b_raw, const float* c_b, float* bg, hipStream_t stream);
 int tts_background_grad(const float* gwb, int n, const float* w_b_raw, float* gw_b_raw,
                         hipStream_t stream);

@@ -1460,17 +1460,17 @@ int tts_geom_fwd_assign_bins_bg(const float* params, const float* sh_rest, int s
   // the count pass inside the geometry launch: blocks of 512 (small) or 4096 (large) gaussians
   const bool small = ws.cblock == CountSmall::kBlock;
   const bool fused = G > 0 && (small ? geom_fwd_count_lds(ws.NB, ws.Tpad)
-                                        : geom_fwd_count_large_lds(ws.NB, ws.Tpad)) <= kMaxLdsBytes;
+                                     : geom_fwd_count_large_lds(ws.NB, ws.Tpad)) <= kMaxLdsBytes;
   const float Sf = static_cast<float>(S);
   int e;
   if (fused && small)
     e = launch_geom_fwd_count(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur, proj,
-                                 keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB, ws.Tpad,
-                                 ws.mat, ws.cell_slot, stream);
+                              keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB, ws.Tpad,
+                              ws.mat, ws.cell_slot, stream);
   else if (fused)
     e = launch_geom_fwd_count_large(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur,
-                                       proj, keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB,
-                                       ws.Tpad, ws.mat, ws.cell_slot, stream);
+                                    proj, keep, step_adv, beta1, beta2, ntx, nty, Sf, span, ws.NB,
+                                    ws.Tpad, ws.mat, ws.cell_slot, stream);
   else
     e = tts_geom_fwd_ex(params, sh_rest, sh_degree, depth_bt, G, camera, near_z, blur, proj, keep,
                         step_adv, beta1, beta2, stream);

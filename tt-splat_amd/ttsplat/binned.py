@@ -65,13 +65,6 @@ def _checked_bins(bins, G):
     return idx32, v8
 
 
-def background(model, device):
-    """bg block [w_b, c_b r, g, b] with w_b = softplus(w_b_raw) (spike/render.py:28)."""
-    w_b = F.softplus(torch.as_tensor(model.w_b_raw, dtype=F32, device=device).reshape(1))
-    c_b = torch.as_tensor(model.c_b, dtype=F32, device=device).reshape(3)
-    return torch.cat([w_b, c_b]).contiguous()
-
-
 def _raw_background(model, device):
     """The model's (w_b_raw, c_b) as fp32 tensors on `device` (differentiable conversions)."""
     w_b_raw = torch.as_tensor(model.w_b_raw, dtype=F32, device=device)
@@ -199,28 +192,22 @@ class BinnedRender(torch.autograd.Function):
     """Whole binned render as one differentiable op of the [G,14] parameter block:
     geometry -> (given bins) -> fused splat; backward: fused splat bwd with theta bwd into
     per-slot gradients -> slot->gaussian reduce (through the inverse table when the bins came
-    with one, else an atomic scatter) -> geometry bwd.  proj: P's projection from this camera
-    when the caller has it already; order: the tiles heaviest first, the splat kernels' dispatch
-    order (26.0 -> 22.9 us forward at G = 100k, 1264x832).  The background is the block bg [4]; with
-    w_b_raw and c_b its gradient goes to them, and bg None is made from them here."""
+    with one, else an atomic scatter) -> geometry bwd.  proj and bg: P's projection from this camera
+    and the background block of w_b_raw and c_b, where the binning has made them (None: made here);
+    order: the tiles heaviest first, the splat kernels' dispatch order (26.0 -> 22.9 us forward at
+    G = 100k, 1264x832)."""
 
     @staticmethod
-    def forward(ctx, P, camera, bg, idx32, v8, inv, H, W, S, k, proj=None, order=None,
-                w_b_raw=None, c_b=None):
+    def forward(ctx, P, camera, w_b_raw, c_b, proj, bg, idx32, v8, inv, order, H, W, S, k):
         Pc = P.detach().contiguous()
-        make = None
-        if bg is None:
-            bg = torch.empty(4, device=Pc.device, dtype=F32)
-            make = (w_b_raw.detach(), c_b.detach().contiguous(), bg)
         if proj is None:
-            proj, _ = kernels.geom_fwd(Pc, camera, background=make)
-        elif make is not None:
-            bg = kernels.background(*make[:2])
+            bg = torch.empty(4, device=Pc.device, dtype=F32)
+            proj, _ = kernels.geom_fwd(Pc, camera,
+                                       background=(w_b_raw.detach(), c_b.detach().contiguous(), bg))
         img, den = kernels.splat_fwd(proj, idx32, v8, bg, H, W, S, k, order=order)
-        keep_raw = w_b_raw is not None and ctx.needs_input_grad[12]
         ctx.save_for_backward(Pc, camera, bg, idx32, v8, proj, img, den,
-                              w_b_raw if keep_raw else None)
-        ctx.c_b_shape = None if c_b is None else c_b.shape
+                              w_b_raw if ctx.needs_input_grad[2] else None)
+        ctx.c_b_shape = c_b.shape
         ctx.inv, ctx.order = inv, order
         ctx.meta = (H, W, S, k)
         return img
@@ -236,18 +223,13 @@ class BinnedRender(torch.autograd.Function):
         gslot = kernels.splat_bwd(proj, idx32, v8, bg, H, W, S, k, img, den,
                                   gimg.float().contiguous(), gslot=gslot, gwb=gwb,
                                   order=ctx.order)
-        gbg = gw = gc = make = None
-        if ctx.c_b_shape is not None:
-            gw, gc, make = _raw_background_grads(ctx, 12, gwb, w_b_raw)
-        else:
-            gbg = torch.zeros(4, device=Pc.device, dtype=F32)
-            gbg[0] = gwb.sum()
+        gw, gc, make = _raw_background_grads(ctx, 2, gwb, w_b_raw)
         if ctx.inv is not None:
             gP = kernels.geom_bwd(Pc, camera, gslot, inv=ctx.inv, background=make)
         else:
             grad9 = kernels.slot_scatter(gslot, idx32, v8, Pc.shape[0])
             gP = kernels.geom_bwd(Pc, camera, grad9, background=make)
-        return gP, None, gbg, None, None, None, None, None, None, None, None, None, gw, gc
+        return (gP, None, gw, gc) + (None,) * 10
 
 
 def render_binned_device(model, cam, tmap, R=1, K=128, cached_bins=None, return_bins=False,
@@ -272,6 +254,6 @@ def render_binned_device(model, cam, tmap, R=1, K=128, cached_bins=None, return_
     else:
         bins = cached_bins
         idx32, v8 = _checked_bins(bins, P.shape[0])
-    img = BinnedRender.apply(P, camera, bg, idx32, v8, inv, tmap.H, tmap.W, tmap.S, float(k),
-                             proj, order, w_b_raw, c_b)
+    img = BinnedRender.apply(P, camera, w_b_raw, c_b, proj, bg, idx32, v8, inv, order, tmap.H,
+                             tmap.W, tmap.S, float(k))
     return (img, bins) if return_bins else img

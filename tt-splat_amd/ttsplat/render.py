@@ -2,8 +2,8 @@
 
 `render(model, cam, arm, k, blur_eps, near, sh_degree)` keeps the reference signature.  The
 whole render is one differentiable op of the [G,14] parameter block (and w_b_raw):
-geometry forward (tts_geom_fwd) -> every gaussian against every pixel (tts_render_dense);
-backward: tts_render_dense_bwd -> tts_geom_bwd.  O(H*W*G) work, no O(H*W*G) memory.
+geometry forward (tts_geom_fwd_bg) -> every gaussian against every pixel it may weigh on
+(tts_render_dense); backward: tts_render_dense_bwd -> tts_geom_bwd_render.  No O(H*W*G) memory.
 
 With sh_degree > 0 and a model carrying color_rest [G,15,3] (spike/model.py:45) the colour is
 the view-dependent SH colour in the direction means3d - camera centre (spike/render.py:23-25),
@@ -39,32 +39,27 @@ def _check_arm(arm, sh_degree=0):
 class DenseRender(torch.autograd.Function):
     """bt: (depth_beta, depth_tau) [2] for arm B, or None; szb: softz_beta [1] for arm SZ, or
     None; rest: the SH rest coefficients in the library layout [15,3,G] (sh_degree > 0), or
-    None; blend: "A", "SZ" or "RV" (arm B blends as A).  The background is either the block bg [4]
-    or, with bg None, made here from w_b_raw and c_b."""
+    None; blend: "A", "SZ" or "RV" (arm B blends as A)."""
 
     @staticmethod
-    def forward(ctx, P, camera, bg, bt, szb, rest, sh_degree, blend, H, W, k, blur, near,
-                w_b_raw=None, c_b=None):
+    def forward(ctx, P, camera, w_b_raw, c_b, bt, szb, rest, sh_degree, blend, H, W, k, blur, near):
         Pc = P.detach().contiguous()
         btc = None if bt is None else bt.detach().float().contiguous()
         szc = None if szb is None else szb.detach().float().reshape(1).contiguous()
         rc = None if rest is None else rest.detach().float().contiguous()
         deg = int(sh_degree) if rc is not None else 0
-        make = None
-        if bg is None:
-            bg = torch.empty(4, device=Pc.device, dtype=F32)
-            make = (w_b_raw.detach(), c_b.detach().contiguous(), bg)
+        bg = torch.empty(4, device=Pc.device, dtype=F32)
+        make = (w_b_raw.detach(), c_b.detach().contiguous(), bg)
         proj, _ = kernels.geom_fwd(Pc, camera, near=near, blur=blur, depth_bt=btc, sh_rest=rc,
                                    sh_degree=deg, background=make)
-        bgc = bg.detach().contiguous()
         if blend == "A":
-            img, den = kernels.render_dense(proj, H, W, k, bgc)
+            img, den = kernels.render_dense(proj, H, W, k, bg)
             aux = None
         else:
-            img, den, aux = kernels.render_dense_arm(proj, H, W, k, bgc, blend, szc)
+            img, den, aux = kernels.render_dense_arm(proj, H, W, k, bg, blend, szc)
         ctx.save_for_backward(Pc, camera, bg, proj, img, den, btc, szc, aux, rc,
-                              w_b_raw if make is not None and ctx.needs_input_grad[13] else None)
-        ctx.c_b_shape = None if make is None else c_b.shape
+                              w_b_raw if ctx.needs_input_grad[2] else None)
+        ctx.c_b_shape = c_b.shape
         ctx.meta = (H, W, k, blur, near, blend, deg)
         return img
 
@@ -72,21 +67,16 @@ class DenseRender(torch.autograd.Function):
     def backward(ctx, gimg):
         Pc, camera, bg, proj, img, den, btc, szc, aux, rc, w_b_raw = ctx.saved_tensors
         H, W, k, blur, near, blend, deg = ctx.meta
-        bgc = bg.detach().contiguous()
         gi = gimg.float().contiguous()
         gszb = None
         if blend == "A":
-            grad9, gwb = kernels.render_dense_bwd(proj, H, W, k, bgc, img, den, gi)
+            grad9, gwb = kernels.render_dense_bwd(proj, H, W, k, bg, img, den, gi)
         else:
-            grad9, gwb = kernels.render_dense_arm_bwd(proj, H, W, k, bgc, blend, img, den, aux, gi,
+            grad9, gwb = kernels.render_dense_arm_bwd(proj, H, W, k, bg, blend, img, den, aux, gi,
                                                       szc)
             if blend == "SZ":
                 gszb = grad9[:, 9].sum().reshape(1)
-        gbg = gw = gc = make = None
-        if ctx.c_b_shape is not None:
-            gw, gc, make = _raw_background_grads(ctx, 13, gwb, w_b_raw)
-        else:
-            gbg = torch.cat([gwb, torch.zeros(3, device=gwb.device, dtype=F32)])
+        gw, gc, make = _raw_background_grads(ctx, 2, gwb, w_b_raw)
         gbt = grest = None
         if btc is None and deg == 0:
             gP = kernels.geom_bwd(Pc, camera, grad9, near=near, blur=blur, background=make)
@@ -97,8 +87,7 @@ class DenseRender(torch.autograd.Function):
                                               background=make)
             if gdw is not None:
                 gbt = gdw.sum(0)
-        return (gP, None, gbg, gbt, gszb, grest, None, None, None, None, None, None, None, gw,
-                gc)
+        return (gP, None, gw, gc, gbt, gszb, grest) + (None,) * 7
 
 
 def render(model, cam, arm, k=4.0, blur_eps=0.3, near=0.2, sh_degree=0):
@@ -117,6 +106,6 @@ def render(model, cam, arm, k=4.0, blur_eps=0.3, near=0.2, sh_degree=0):
     color_rest = getattr(model, "color_rest", None)
     if int(sh_degree) > 0 and color_rest is not None:        # spike/render.py:23-25
         rest = kernels.sh_rest_layout(color_rest.to(dev, F32))
-    return DenseRender.apply(P, cam.device_block(dev), None, bt, szb, rest, int(sh_degree), blend,
-                             cam.H, cam.W, float(k), float(blur_eps), float(near),
-                             *_raw_background(model, dev))
+    return DenseRender.apply(P, cam.device_block(dev), *_raw_background(model, dev), bt, szb, rest,
+                             int(sh_degree), blend, cam.H, cam.W, float(k), float(blur_eps),
+                             float(near))
