@@ -195,11 +195,12 @@ struct DenseWalk {
   }
   __device__ __forceinline__ static int split() { return (threadIdx.x >> 6) % SPL; }
 
-  // STRAIGHT: 64 entries that all reach the patch, and are bounded (so calm: u is a number), are
-  // walked without picking the hits.  Arm A, every box the whole image: G 2000, 400x400 157 -> 132
-  // us, 800x800 552 -> 473; not for the other arms, whose pairs cost several times as much.
+  // STRAIGHT: a list of all gaussians tested for it (so that nearly all reach every patch) is
+  // walked without testing the patches.  Arm A, every box the whole image: G 2000, 400x400 157 ->
+  // 125 us, 800x800 536 -> 466 (and 28.9 -> 29.2 at G 10000, 800x800 with small boxes); not for the
+  // other arms, whose pairs cost several times as much.
   template <bool STRAIGHT, class F>
-  __device__ __forceinline__ void evaluate(int n, int X0, int Y0, const F& f) {
+  __device__ __forceinline__ void evaluate(int n, int tested, int X0, int Y0, const F& f) {
     const int lane = threadIdx.x & 63, sp = split();
     if (TS == 8) {
       for (int j = sp; j < n; j += 2 * SPL) {
@@ -207,9 +208,14 @@ struct DenseWalk {
         const int j1 = two ? j + SPL : j;
         const float4 A0 = a[j], B0 = b[j], A1 = a[j1], B1 = b[j1];
         const float2 O0 = o[j], O1 = o[j1];
-        f(A0, B0, O0, std::false_type{});
-        if (two) f(A1, B1, O1, std::false_type{});
+        f(A0, B0, O0);
+        if (two) f(A1, B1, O1);
       }
+      return;
+    }
+    if (STRAIGHT && n == tested) {
+#pragma unroll 2
+      for (int i = sp; i < n; i += SPL) f(a[i], b[i], o[i]);
       return;
     }
     const float cx = (float)(X0 + (lane_x() & ~7)) + 4.0f;
@@ -221,11 +227,6 @@ struct DenseWalk {
       const float2 e = h[j];
       const bool hit = j0 + lane < n && reaches(cx, 3.5f, A.x, e.x) && reaches(cy, 3.5f, A.y, e.y);
       uint64_t m = __ballot(hit);
-      if (STRAIGHT && m == ~0ull && __ballot(!(e.x < INFINITY)) == 0) {
-#pragma unroll 2
-        for (int i = j0 + sp; i < j0 + 64; i += SPL) f(a[i], b[i], o[i], std::true_type{});
-        continue;
-      }
       if (SPL > 1) {
         const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
@@ -241,14 +242,13 @@ struct DenseWalk {
         m &= m - 1;
         const float4 A0 = a[i0], B0 = b[i0], A1 = a[i1], B1 = b[i1];
         const float2 O0 = o[i0], O1 = o[i1];
-        f(A0, B0, O0, std::false_type{});
-        if (two) f(A1, B1, O1, std::false_type{});
+        f(A0, B0, O0);
+        if (two) f(A1, B1, O1);
       }
     }
   }
 
-  // f(A, B, O, calm) for every gaussian that may weigh on this lane's pixel (and some that do not);
-  // calm: a type that says whether 1 - Q/k is known to be a number.
+  // f(A, B, O) for every gaussian that may weigh on this lane's pixel (and some that do not).
   // cull = 0 takes every gaussian.  Ends with a barrier.
   template <bool STRAIGHT = false, class F>
   __device__ __forceinline__ void walk(const float* __restrict__ proj, int G, float inv_k, int cull,
@@ -258,7 +258,7 @@ struct DenseWalk {
     const float half = 0.5f * (TS - 1);
     const float cx = (float)X0 + 0.5f * TS, cy = (float)Y0 + 0.5f * TS;
     const float4* rec = reinterpret_cast<const float4*>(proj);
-    int n = 0, buf = 0;
+    int n = 0, buf = 0, from = 0;   // from: the first gaussian that the list is of
     float4 n0, n1, n2;
     if (G > 0) {
       const int64_t g = min((int)threadIdx.x, G - 1);
@@ -292,8 +292,9 @@ struct DenseWalk {
       buf ^= 1;
       if (n > CAP - NT || G - g0 <= NT) {
         __syncthreads();
-        evaluate<STRAIGHT>(n, X0, Y0, f);
+        evaluate<STRAIGHT>(n, min(G, g0 + NT) - from, X0, Y0, f);
         n = 0;
+        from = g0 + NT;
         __syncthreads();
       }
     }
@@ -389,17 +390,15 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
   const float px = (float)x + 0.5f, py = (float)y + 0.5f;
   const float beta = ARM == kArmSZ ? szb[0] : 0.0f;
   float zstar = 0.0f, den0 = 0.0f;
-  auto weight = [&](const float4& A, const float4& B, auto calm) {
-    const float u = quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k);
-    const float r = decltype(calm)::value ? fmaxf(u, 0.0f) : relu_nan(u);
+  auto weight = [&](const float4& A, const float4& B) {
+    const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
     return r * r;
   };
   if (ARM == kArmSZ) {   // z* first
     if (!tame(beta)) cull = 0;
     float v[2] = {0.f, 0.f};
-    s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O,
-                                             auto calm) {
-      const float w = weight(A, B, calm);
+    s.walk(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B, const float2& O) {
+      const float w = weight(A, B);
       v[0] += w * O.x;
       v[1] += w * O.x * O.y;
     });
@@ -410,8 +409,8 @@ __global__ __launch_bounds__(NT) void k_render_dense(const float* __restrict__ p
   }
   float v[ARM == kArmRV ? 5 : 4] = {};
   s.template walk<ARM == kArmA>(proj, G, inv_k, cull, X0, Y0, [&](const float4& A, const float4& B,
-                                                                  const float2& O, auto calm) {
-    add_pair<ARM>(v, weight(A, B, calm), B.y, B.z, B.w, O.x, O.y, zstar, beta);
+                                                                  const float2& O) {
+    add_pair<ARM>(v, weight(A, B), B.y, B.z, B.w, O.x, O.y, zstar, beta);
   });
   s.join(v);
   if (Walk::split() != 0 || x >= W || y >= H) return;
@@ -658,7 +657,7 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
   if (__syncthreads_or(bad)) cull = 0;
   float Z[1] = {0.0f};
   s.walk(proj, G, inv_k, cull, X0 + xo, Y0 + yo, [&](const float4& A, const float4& B,
-                                                     const float2& O, auto) {
+                                                     const float2& O) {
     const float r = relu_nan(quad_u(px - A.x, py - A.y, A.z, A.w, B.x, inv_k));
     const float h = sigmoidf_(-beta * (O.y - zs));
     Z[0] += r * r * (q.x * B.y + q.y * B.z + q.z * B.w + q.w * O.x) * h * (1.0f - h);
