@@ -1186,17 +1186,17 @@ inline int dense_cull(int H, int W, float ik) {
 // the whole image the pairs bound it, and blocks that fill the GPU evenly count.  Measured, arm A,
 // small boxes / whole-image boxes (us; soft-Z orders the same way):
 //                        few       16/256      16/512      16/1024     32/1024     8/512
-//   G 16, 128x128        3.0/3.0   3.3/4.8     3.6/4.2     4.4/4.8     4.0/5.6     3.4/3.5
-//   G 32, 400x400        4.6/4.6   3.8/6.9     4.9/7.3     7.4/10      4.2/7.7     8.8/10
-//   G 64, 800x800        16/16     6.7/19      9.7/21      18/32       7.7/22      25/38
-//   G 256, 800x800       51/52     7.0/57      10/59       19/70       8.0/65      26/74
-//   G 256, 400x400       19/19     4.0/23      5.1/22      7.7/24      4.4/26      8.9/22
-//   G 600, 512x512                 6.3/60      7.4/59      9.6/61      4.7/58      17/63
-//   G 2000, 128x128                15/136      8.9/68      7.6/57      12/180      6.3/27
-//   G 2000, 256x256                9.6/136     6.9/70      6.2/58      7.4/177     11/54
-//   G 2000, 400x400                10/159      9.3/135     11/142      6.3/179     20/119
-//   G 2000, 800x800                20/419      21/415      27/444      11/475      62/443
-// (one thread per pixel, every pair visited: 3.0, 4.8, 16, 58, 20, -, 88, -, 125, -)
+//   G 16, 128x128        3.0/3.0   3.3/4.0     3.6/3.8     4.4/4.5     4.1/5.1     3.3/3.5
+//   G 32, 400x400        4.6/4.7   3.8/5.9     4.9/6.7     7.6/9.4     4.3/6.8     8.6/10
+//   G 64, 800x800        16/17     6.8/19      9.9/21      18/31       7.9/22      25/37
+//   G 256, 400x400       20/20     4.1/23      5.2/21      8.0/22      4.5/26      9.0/22
+//   G 256, 800x800       50/53     7.0/56      10/55       19/64       8.1/63      25/72
+//   G 600, 512x512                 6.3/58      7.4/54      9.8/53      4.8/55      17/62
+//   G 2000, 128x128                15/123      8.8/60      7.3/48      12/170      6.1/26
+//   G 2000, 256x256                9.9/124     7.0/62      6.3/50      7.3/168     10/58
+//   G 2000, 400x400                10/149      9.3/123     11/122      6.3/169     20/118
+//   G 2000, 800x800                19/403      21/387      27/389      11/458      59/436
+// (one thread per pixel, every pair visited: 3.1, 4.8, 16, 20, 58, -, 88, 90, 125, 390)
 template <class F>
 void dense_tiling(int G, int H, int W, const F& f) {
   using std::integral_constant;
