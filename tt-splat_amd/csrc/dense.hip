@@ -197,7 +197,7 @@ struct DenseWalk {
 
   // STRAIGHT: a list of all gaussians tested for it (so that nearly all reach every patch) is
   // walked without testing the patches.  Arm A, every box the whole image: G 2000, 400x400 157 ->
-  // 125 us, 800x800 536 -> 466 (and 28.9 -> 29.2 at G 10000, 800x800 with small boxes); not for the
+  // 125 us, 800x800 536 -> 466 (and 30.6 -> 31.0 at G 10000, 800x800 with small boxes); not for the
   // other arms, whose pairs cost several times as much.
   template <bool STRAIGHT, class F>
   __device__ __forceinline__ void evaluate(int n, int tested, int X0, int Y0, const F& f) {
@@ -216,7 +216,7 @@ struct DenseWalk {
     if (STRAIGHT && n == tested) {
 #pragma unroll 2
       for (int i = sp; i < n; i += SPL) f(a[i], b[i], o[i]);
-      return;
+      n = 0;
     }
     const float cx = (float)(X0 + (lane_x() & ~7)) + 4.0f;
     const float cy = (float)(Y0 + (lane_y() & ~7)) + 4.0f;
