@@ -686,11 +686,12 @@ __global__ __launch_bounds__(NT) void k_softz_pre(const float* __restrict__ proj
 // cells, and writes its own gradients; k_dense_reduce adds them.
 //
 // Whole arm-A backward in us, against one thread per gaussian over every pixel (bands of pixels
-// staged in LDS, band sums): small boxes, G 2000, 128x128 19 (that form 43), G 10000, 300x300 25
-// (472), 800x800 85 (3061); every box the whole image, G 2000, 128x128 28 (41), 400x400 177 (224),
-// G 10000, 300x300 481 (466); a whole-image box among 256 small ones, 800x800 223 (391), among
-// 10000 427 (3000).  Each box by itself always, by its own waves: 43, 333, 867, 791, 808.  Soft-Z,
-// every box the whole image: 118 (295), 992 (1004), G 4000, 400x400 1925 (1862).
+// staged in LDS, band sums): small boxes, G 2000, 128x128 9.6 (that form 40), G 10000, 300x300 15
+// (435), 800x800 34 (3000); every box the whole image, G 2000, 128x128 29 (41), 400x400 178 (226),
+// 800x800 802 (711), G 10000, 300x300 487 (468); a whole-image box among 256 small ones, 800x800
+// 222 (388), among 10000 445 (3014).  Each box by itself always, by its own waves: 43, 331, 1487,
+// 863, 797, 807.  Soft-Z, every box the whole image: 116 (294), 1009 (1003), G 4000, 400x400 1947
+// (1867).
 template <int ARM>
 struct PairSums {
   float r = 0.f, g = 0.f, b = 0.f, o = 0.f, beta = 0.f;   // dL/d col_o, o_col, softz_beta
